@@ -132,6 +132,8 @@ k_apply_qp(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc, Tables
     x = gmem((const T *)ad.x) + (int64_t)rhs * N;
     y = gmem((T *)ad.y) + (int64_t)rhs * N;
     part = gmem((T *)ad.part) + (int64_t)rhs * 4 * part_stride(ad);
+    // residual mode when set (wave-uniform): y = resid - A x
+    const gptr<const T> rbv = ad.resid ? gmem((const T *)ad.resid) + (int64_t)rhs * N : nullptr;
 
     // ---- element DOFs of x into R0 (PEC DOFs read as zero) ----
     if (eact)
@@ -479,7 +481,7 @@ k_apply_qp(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc, Tables
       if (ess)
       {
         if (owner)
-          y[gid] = x[gid];
+          y[gid] = rbv ? rbv[gid] - x[gid] : x[gid];
         continue;
       }
       // sum of the element vectors of the (up to 4) tile elements sharing the
@@ -525,7 +527,7 @@ k_apply_qp(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc, Tables
         part[slot * part_stride(ad) + pid] = v;
       }
       else
-        y[gid] = v;
+        y[gid] = rbv ? rbv[gid] - v : v;
     }
     if (BATCH && rhs + 1 < r_end)
       __syncthreads(); // the next rhs overwrites the element arrays
