@@ -282,8 +282,10 @@ k_apply_qp(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc, Tables
 
     // ======================= quadrature point =======================
     {
-      const T u0 = U[0], u1 = U[1], u2 = U[2];
-      const T c0 = Cu[0], c1 = Cu[1], c2 = Cu[2];
+      // term weights of a descriptor-table launch (1 unless one term is asked for)
+      const T msc = BATCH ? (T)ad.mscale : T(1), csc = BATCH ? (T)ad.cscale : T(1);
+      const T u0 = msc * U[0], u1 = msc * U[1], u2 = msc * U[2];
+      const T c0 = csc * Cu[0], c1 = csc * Cu[1], c2 = csc * Cu[2];
       U[0] = qf[0] * u0 + qf[1] * u1 + qf[2] * u2;
       U[1] = qf[1] * u0 + qf[3] * u1 + qf[4] * u2;
       U[2] = qf[2] * u0 + qf[4] * u1 + qf[5] * u2;
