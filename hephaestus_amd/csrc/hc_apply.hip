@@ -86,9 +86,7 @@ wave_lds_sync()
 // instances of the device table descs[]; a work item loops over a group of rb
 // right-hand sides with the tile's quadrature data held in registers (read
 // from HBM once per group).
-// EF = 1: element factors (box meshes, ApplyDesc::ef) instead of the
-// quadrature-point factors.
-template <int P, typename T, int TX, int TY, int TZ, int MODE, int SP, int BATCH, int EF, int VT = 1>
+template <int P, typename T, int TX, int TY, int TZ, int MODE, int SP, int BATCH>
 __global__ void __launch_bounds__((Tile<P, TX, TY, TZ, SP>::NT))
 k_apply_tile(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc, Tables<T> tb_arg)
 {
@@ -104,24 +102,16 @@ k_apply_tile(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc, Tabl
   constexpr basis::Tab<T> tb_c = basis::tab<P, T>();
   // FP64: gfx950 has no 64-bit instruction literals, so each use of a double
   // constant costs two scalar moves into a register pair (rematerialised
-  // whenever scalar registers run short).  With VREG the order-P tables are
-  // moved into vector registers once per wave and every contraction reads
-  // them there: 88 more VGPRs at order 3, which fit where a SIMD holds two
-  // waves of these kernels (one qz group, the LDS of two workgroups per CU)
-  // and no quadrature-point factors are held (element factors); every batch
-  // form of such a tile does the same, so their results agree.  Measured at
-  // 48^3 order 3: 177 -> 156 us on the (4, 2, 2) tile; with two qz groups, or
-  // with the quadrature-point factors, the extra registers cost occupancy
-  // and the kernels slow down.  FP32 constants are literals of the VOP2
-  // encoding.
-  // With the quadrature-point factors the order-3 tiles hold 170 VGPRs
-  // already: only the closed-basis tables (64 VGPRs) are moved there.
-  constexpr bool VREG = VT != 0 && sizeof(T) == 8 && SP == 1 && (EF || (P == 3 && MODE == 1 && BATCH != 1));
+  // whenever scalar registers run short).  With VREG the closed-basis tables
+  // are moved into vector registers once per wave (64 VGPRs at order 3, beside
+  // the 170 that hold the quadrature-point factors), where a SIMD holds two
+  // waves of these kernels (one qz group, the LDS of two workgroups per CU);
+  // elsewhere the extra registers cost occupancy and the kernels slow down.
+  // FP32 constants are literals of the VOP2 encoding.
+  constexpr bool VREG = sizeof(T) == 8 && SP == 1 && P == 3 && MODE == 1 && BATCH != 1;
   basis::Tab<T> tb = tb_c;
   if constexpr (VREG)
   {
-    if constexpr (EF)
-      pin_vgpr(tb.Bo, std::make_index_sequence<Q * O>{});
     pin_vgpr(tb.Bc, std::make_index_sequence<Q * D>{});
     pin_vgpr(tb.Gc, std::make_index_sequence<Q * D>{});
   }
@@ -201,11 +191,9 @@ k_apply_tile(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc, Tabl
   const int ilx = tid % TX, idy = (tid / TX) % D, idz = (tid / (TX * D)) % D;
   const int ily = (tid / (TX * D * D)) % TY, ilz = tid / (TX * D * D * TY);
 
-  // ---- loads of one tile: the pencil's 12 Q quadrature factors (or its
-  // element's two factors), the item's x rows of the three components (PEC
-  // DOFs read as zero) ----
-  T qf[EF ? 1 : QH][EF ? 1 : 12];
-  T fe[2]; // element factors dt nu_e, sigma_e
+  // ---- loads of one tile: the pencil's 12 Q quadrature factors, the
+  // item's x rows of the three components (PEC DOFs read as zero) ----
+  T qf[QH][12];
   T xr0[O], xr1[D], xr2[D];
   auto load_qf = [&](const int * e0_, const int * ne_) {
     const bool pin = pact && pl0 < ne_[0] && pl1 < ne_[1] && pl2 < ne_[2];
@@ -213,13 +201,6 @@ k_apply_tile(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc, Tabl
     // their U, Cu are zero or never reach an output (the x^T rows sum valid
     // elements only; quadrature points past Q meet zero table entries).
     const int64_t e = pin ? ((int64_t)(e0_[2] + pl2) * g.n[1] + (e0_[1] + pl1)) * g.n[0] + (e0_[0] + pl0) : 0;
-    if constexpr (EF)
-    {
-      const gptr<const T> ce = gmem((const T *)ad.ef.qc) + 2 * e;
-      fe[0] = ce[0];
-      fe[1] = ce[1];
-      return;
-    }
     const gptr<const T> qe = qd + e * (12 * Q * QQ) + (pin ? pqy * Q + pqx : 0);
 #pragma unroll
     for (int j = 0; j < QH; j++)
@@ -294,8 +275,6 @@ k_apply_tile(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc, Tabl
     }
     load_qf(e0, ne);
   }
-  else if (EF)
-    load_qf(e0, ne);
 
   for (int rhs = r_begin; rhs < r_end; rhs++)
   {
@@ -511,47 +490,10 @@ k_apply_tile(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc, Tabl
     __syncthreads();
 
   // ======================= quadrature points =======================
-  if (MODE == 0 && !EF)
+  if (MODE == 0)
     load_qf(e0, ne);
   // term weights (batched kernel only; the single-instance kernel applies A)
   const T msc = TABLE ? (T)ad.mscale : T(1), csc = TABLE ? (T)ad.cscale : T(1);
-  if constexpr (EF)
-  {
-    // factor of component a at (qx, qy, qz): sigma_e w mk[a] (mass) and
-    // dt nu_e w ck[a] (curl), w = w_qx w_qy w_qz
-    auto qw_sel = [&](int q) {
-      T v = tb_c.qw[0];
-      if constexpr (Q > 1)
-        v = q == 1 ? tb_c.qw[1] : v;
-      if constexpr (Q > 2)
-        v = q == 2 ? tb_c.qw[2] : v;
-      if constexpr (Q > 3)
-        v = q == 3 ? tb_c.qw[3] : v;
-      static_assert(Q <= 4, "weights of at most four points");
-      return v;
-    };
-    const T wxy = qw_sel(pqx) * qw_sel(pqy);
-    const T sgm = TABLE ? fe[1] * msc : fe[1], cnu = TABLE ? fe[0] * csc : fe[0];
-    const T mk0 = (T)ad.ef.mk[0], mk1 = (T)ad.ef.mk[1], mk2 = (T)ad.ef.mk[2];
-    const T ck0 = (T)ad.ef.ck[0], ck1 = (T)ad.ef.ck[1], ck2 = (T)ad.ef.ck[2];
-    with_ph([&](auto phc) {
-      constexpr int PH = decltype(phc)::value;
-#pragma unroll
-      for (int j = 0; j < QH; j++)
-      {
-        const int qz = PH * QH + j; // past Q: zero weight, and U, Cu are zero there
-        const T w = wxy * tb_c.qw[qz];
-        const T sm = w * sgm, sc = w * cnu;
-        U[0][j] = (sm * mk0) * U[0][j];
-        U[1][j] = (sm * mk1) * U[1][j];
-        U[2][j] = (sm * mk2) * U[2][j];
-        Cu[0][j] = (sc * ck0) * Cu[0][j];
-        Cu[1][j] = (sc * ck1) * Cu[1][j];
-        Cu[2][j] = (sc * ck2) * Cu[2][j];
-      }
-    });
-  }
-  else
   {
 #pragma unroll
   for (int j = 0; j < QH; j++)
@@ -954,7 +896,6 @@ launch_one(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, 
     return hipSuccess;
   // BATCH variant: 0 single instance, 1 table with rhs groups, 2 table with one rhs per item
   const int bv = !descs ? 0 : ((grouped & 1) ? 1 : 2);
-  const bool ef = descs ? (grouped & LAUNCH_EF) != 0 : d0.ef.qc != nullptr;
   auto go = [&](auto kern, const auto & t) {
     hipLaunchKernelGGL(kern, dim3(nwork), dim3(C::NT), 0, st, d0, descs, ndesc, t);
   };
@@ -962,21 +903,21 @@ launch_one(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, 
   {
     const Tables<double> & t = *(const Tables<double> *)tb;
     if (bv == 0)
-      ef ? go(k_apply_tile<P, double, TX, TY, TZ, MODE, SP, 0, 1>, t) : go(k_apply_tile<P, double, TX, TY, TZ, MODE, SP, 0, 0>, t);
+      go(k_apply_tile<P, double, TX, TY, TZ, MODE, SP, 0>, t);
     else if (bv == 1)
-      ef ? go(k_apply_tile<P, double, TX, TY, TZ, MODE, SP, 1, 1>, t) : go(k_apply_tile<P, double, TX, TY, TZ, MODE, SP, 1, 0>, t);
+      go(k_apply_tile<P, double, TX, TY, TZ, MODE, SP, 1>, t);
     else
-      ef ? go(k_apply_tile<P, double, TX, TY, TZ, MODE, SP, 2, 1>, t) : go(k_apply_tile<P, double, TX, TY, TZ, MODE, SP, 2, 0>, t);
+      go(k_apply_tile<P, double, TX, TY, TZ, MODE, SP, 2>, t);
   }
   else
   {
     const Tables<float> & t = *(const Tables<float> *)tb;
     if (bv == 0)
-      ef ? go(k_apply_tile<P, float, TX, TY, TZ, MODE, SP, 0, 1>, t) : go(k_apply_tile<P, float, TX, TY, TZ, MODE, SP, 0, 0>, t);
+      go(k_apply_tile<P, float, TX, TY, TZ, MODE, SP, 0>, t);
     else if (bv == 1)
-      ef ? go(k_apply_tile<P, float, TX, TY, TZ, MODE, SP, 1, 1>, t) : go(k_apply_tile<P, float, TX, TY, TZ, MODE, SP, 1, 0>, t);
+      go(k_apply_tile<P, float, TX, TY, TZ, MODE, SP, 1>, t);
     else
-      ef ? go(k_apply_tile<P, float, TX, TY, TZ, MODE, SP, 2, 1>, t) : go(k_apply_tile<P, float, TX, TY, TZ, MODE, SP, 2, 0>, t);
+      go(k_apply_tile<P, float, TX, TY, TZ, MODE, SP, 2>, t);
   }
   return hipGetLastError();
 }
@@ -989,9 +930,7 @@ launch_one(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, 
 
 static const TileCandidate g_cands[] = {
     // first entry of each order = default before tuning (order 3: one qz group,
-    // whose FP64 kernels hold the order tables in vector registers -- the
-    // fastest element-factor tile on box meshes, within a few per cent of the
-    // best with quadrature-point factors)
+    // within a few per cent of the best)
     HC_CAND(1, 4, 4, 4, 1, 2), HC_CAND(1, 4, 4, 4, 1, 1), HC_CAND(1, 8, 4, 2, 1, 1), HC_CAND(1, 8, 4, 2, 0, 2),
     HC_CAND(1, 8, 8, 1, 0, 1), HC_CAND(1, 16, 2, 2, 1, 1), HC_QP(1, 4, 4, 4), HC_QP(1, 8, 4, 2),
     HC_CAND(2, 4, 2, 2, 1, 1), HC_CAND(2, 4, 2, 2, 1, 2), HC_CAND(2, 4, 2, 2, 0, 2), HC_CAND(2, 4, 4, 2, 1, 1),
@@ -1061,6 +1000,12 @@ apply_op(const Geom & g, const PlaneSegs & segs, const Tables<T> & tb, const T *
   d.ntiles = g.nt[0] * g.nt[1] * g.nt[2];
   d.pw0 = 0;
   hipError_t e;
+  if (ef.qc)
+  {
+    // box mesh: one launch, results independent of rb (one rhs per work item)
+    set_box_tile(d, box_tile(g, nrhs));
+    return apply_box<T>(d, nullptr, 1, d.ntiles * nrhs, g.p, d.bt.ns, st);
+  }
   if (rb > 1 && nrhs > 1)
   {
     if (!desc_dev)
@@ -1068,8 +1013,7 @@ apply_op(const Geom & g, const PlaneSegs & segs, const Tables<T> & tb, const T *
     d.rb = rb < nrhs ? rb : nrhs;
     if ((e = hipMemcpyAsync(desc_dev, &d, sizeof(d), hipMemcpyHostToDevice, st)) != hipSuccess)
       return e;
-    e = cand->launch(d, desc_dev, 1, d.ntiles * ((nrhs + d.rb - 1) / d.rb), 1 | (ef.qc ? LAUNCH_EF : 0), &tb,
-                     sizeof(T) == 8 ? 64 : 32, st);
+    e = cand->launch(d, desc_dev, 1, d.ntiles * ((nrhs + d.rb - 1) / d.rb), 1, &tb, sizeof(T) == 8 ? 64 : 32, st);
   }
   else
     e = cand->launch(d, nullptr, 1, d.ntiles * nrhs, 0, &tb, sizeof(T) == 8 ? 64 : 32, st);
@@ -1098,11 +1042,16 @@ apply_scaled(const Geom & g, const PlaneSegs & segs, const Tables<T> & tb, const
   d.ntiles = g.nt[0] * g.nt[1] * g.nt[2];
   d.mscale = mscale;
   d.cscale = cscale;
+  if (ef.qc)
+  {
+    set_box_tile(d, box_tile(g, 1));
+    return apply_box<T>(d, nullptr, 1, d.ntiles, g.p, d.bt.ns, st);
+  }
   // term weights are honoured by the batched kernel (descriptor in device memory)
   hipError_t e = hipMemcpyAsync(desc_dev, &d, sizeof(d), hipMemcpyHostToDevice, st);
   if (e != hipSuccess)
     return e;
-  e = cand->launch(d, desc_dev, 1, d.ntiles, ef.qc ? LAUNCH_EF : 0, &tb, sizeof(T) == 8 ? 64 : 32, st);
+  e = cand->launch(d, desc_dev, 1, d.ntiles, 0, &tb, sizeof(T) == 8 ? 64 : 32, st);
   if (e != hipSuccess)
     return e;
   return assemble_planes<T>(d, nullptr, 1, d.prows, st);
@@ -1138,9 +1087,11 @@ template hipError_t apply_op<float>(const Geom &, const PlaneSegs &, const Table
 template <typename T>
 hipError_t
 apply_multi(const TileCandidate * cand, const Tables<T> & tb, const ApplyDesc * descs_dev, int ndesc, int nwork,
-            int npwork, int grouped, hipStream_t st)
+            int npwork, int grouped, int box_ns, hipStream_t st)
 {
   ApplyDesc dummy{};
+  if (box_ns)
+    return apply_box<T>(dummy, descs_dev, ndesc, nwork, cand->p, box_ns, st);
   hipError_t e = cand->launch(dummy, descs_dev, ndesc, nwork, grouped, &tb, sizeof(T) == 8 ? 64 : 32, st);
   if (e != hipSuccess)
     return e;
@@ -1148,8 +1099,8 @@ apply_multi(const TileCandidate * cand, const Tables<T> & tb, const ApplyDesc * 
 }
 
 template hipError_t apply_multi<double>(const TileCandidate *, const Tables<double> &, const ApplyDesc *, int, int, int,
-                                        int, hipStream_t);
+                                        int, int, hipStream_t);
 template hipError_t apply_multi<float>(const TileCandidate *, const Tables<float> &, const ApplyDesc *, int, int, int, int,
-                                       hipStream_t);
+                                       int, hipStream_t);
 
 } // namespace hc

@@ -1,0 +1,720 @@
+// Apply of dt*nu K + sigma M on axis-aligned box meshes from two factors per
+// element (ApplyDesc::ef), on the FP64 matrix units (gfx950).
+//
+// The operator is that of hc_apply.hip (EquationSystem::Mult,
+// src/equation_systems/equation_system.cpp:200-204, on the system of
+// FormLinearSystem, equation_system.cpp:132-190).  On a box element with
+// J = diag(h) its integrals separate, and the p + 1 point rule integrates
+// them exactly, so they are written with the exact 1-D matrices:
+//   Mc  closed mass matrix (p + 1 Gauss-Lobatto points),
+//   W   open mass matrix: diagonal, the Gauss-Legendre weights, because the
+//       Lagrange basis on the p Gauss points is orthogonal,
+//   Dg  the derivative of a closed 1-D function at the open points, which is
+//       exact because it has degree p - 1.
+// The curl of an ND field is then three differences (Dg along one axis), its
+// mass matrix one contraction and two weights, and its transpose the same
+// differences again:
+//   c_x = D_y u_z - D_z u_y,  c_y = D_z u_x - D_x u_z,  c_z = D_x u_y - D_y u_x
+//   f_a = dt nu ck_a Mc_a W W c_a,   ck_a = h_a^2 / |det J|
+//   y_x = sigma mk_0 W Mc_y Mc_z u_x + D_z^T f_y - D_y^T f_z   (and cyclic)
+// with no quadrature-point values: at order 3 about 220 multiply-adds of 4-wide
+// contractions per 16 lanes and element layer against 600 for interpolation to
+// the quadrature points and back.
+//
+// One 16-lane block of a wave holds the 4 x 4 (x, y) points of an element
+// (orders 2 and 3; 2 x 2 elements at order 1, block-diagonal matrices), the z
+// points are in registers.  A contraction along x or y of one plane is one
+// v_mfma_f64_4x4x4_4b (four independent 4 x 4 products, one per 16-lane
+// block); along z it is register arithmetic with compile-time tables.  Lane
+// layouts (fast lane index f = lane % 4, slow s = lane / 16, block
+// (lane / 4) % 4): "N" f = x, s = y; "T" f = y, s = x.  The instruction takes
+// A[f][s], B[s][f] and returns D[s][f], so a value used as B is contracted
+// along its slow axis and keeps its layout, used as A it is contracted along
+// its slow axis and comes back transposed; no lane exchange is needed except
+// for u_z and f_z (a product with the identity).
+//
+// A workgroup owns a column of tiles: ns elements (cx by cy) marched along z.
+// The top plane of a layer is carried to the next one in registers; the face
+// values of x and y neighbours meet in LDS (one barrier per layer, two
+// buffers).  Elements on the lower x, y and z faces of a tile are computed by
+// both tiles, so every output DOF is summed by one workgroup in a fixed order:
+// one launch, no partial sums in memory, and the same bits for every tile
+// shape.
+//
+// Measured at 48^3 order 3 (9.08 M DOFs): 195 us per FP64 apply with the
+// LDS-staged tile kernel and its face assembly, 63 us here (FP32 vectors: 115
+// and 60 us).  Memory traffic is 164 MB (147 MB algorithmic, 30 us at the copy
+// rate); the bound is the FP64 pipe -- one 4 x 4 x 4 product takes 7 ns per SIMD
+// and a vector FMA 2.3 ns, and they do not overlap -- at about 65 % use, the
+// rest being latency with the four waves per SIMD that 128 registers allow.
+// Of the work 1.31 x 1.1 is duplicated elements of tile and chunk faces.
+#include "hc_basis.hpp"
+#include "hc_kernels.hpp"
+
+#include <algorithm>
+
+namespace hc
+{
+
+namespace
+{
+
+template <int P>
+struct BoxTab
+{
+  double M[P + 1][P + 1] = {}; // closed mass matrix
+  double D[P][P + 1] = {};     // derivative of the closed basis at the open points
+  double w[P] = {};            // open weights
+};
+
+template <int P>
+constexpr BoxTab<P>
+box_tab()
+{
+  BoxTab<P> t{};
+  const basis::Tab<double> b = basis::make_tab(P);
+  double on[PMAX] = {}, ow[PMAX] = {}, cn[PMAX + 1] = {};
+  basis::gauss_legendre01(P, on, ow);
+  basis::gauss_lobatto01(P + 1, cn);
+  for (int i = 0; i < P; i++)
+  {
+    double v[PMAX + 1] = {}, d[PMAX + 1] = {};
+    basis::lagrange(P + 1, cn, on[i], v, d);
+    t.w[i] = ow[i];
+    for (int m = 0; m <= P; m++)
+      t.D[i][m] = d[m];
+  }
+  // entries that are equal by symmetry get one value (one scalar register pair)
+  for (int a = 0; a <= P; a++)
+    for (int c = 0; c <= P; c++)
+    {
+      const int m = a < c ? a : c, n = a < c ? c : a;       // M[a][c] = M[c][a]
+      const bool flip = m + n > P; // = M[P-c][P-a]
+      const int i = flip ? P - n : m, j = flip ? P - m : n;
+      for (int q = 0; q <= P; q++)
+        t.M[a][c] += b.qw[q] * b.Bc[q * (P + 1) + i] * b.Bc[q * (P + 1) + j];
+    }
+  for (int i = 0; i < P; i++)
+  {
+    t.w[i] = ow[i <= P - 1 - i ? i : P - 1 - i];
+    for (int m = 0; m <= P; m++)
+      if (2 * i > P - 1 || (2 * i == P - 1 && 2 * m > P))
+        t.D[i][m] = -t.D[P - 1 - i][P - m];
+  }
+  return t;
+}
+
+// a b + c; NEG: bit 0 negates a (operand modifier of the FP64 form)
+template <int NEG = 0>
+__device__ inline double
+mm(double a, double b, double c)
+{
+  return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, NEG);
+}
+
+} // namespace
+
+// Global memory through a buffer resource at a wave-uniform base, with a 32-bit
+// byte offset per lane: no vector arithmetic per access, and the hardware's
+// range check takes the place of lane masks -- a lane whose offset is OOB loads
+// zero and stores nothing.  Offsets are relative to the first row of a tile in
+// the lowest plane of a layer (box_fits: p + 1 planes stay below 2^32 bytes; a
+// mesh beyond that keeps the quadrature-point factors).
+constexpr uint32_t OOB = 0xFFFFFFFFu;
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+template <typename T>
+__device__ inline __amdgpu_buffer_rsrc_t
+rsrc(const T * p)
+{
+  return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, (int)(OOB - 1), 0x00027000);
+}
+template <typename T>
+__device__ inline T
+ldb(const T * base, uint32_t off, uint32_t sof = 0)
+{
+  if constexpr (sizeof(T) == 8)
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(rsrc(base), (int)off, (int)sof, 0));
+  else
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(rsrc(base), (int)off, (int)sof, 0));
+}
+template <typename T>
+__device__ inline void
+stb(T * base, uint32_t off, T v, uint32_t sof = 0)
+{
+  if constexpr (sizeof(T) == 8)
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), rsrc(base), (int)off, (int)sof, 0);
+  else
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rsrc(base), (int)off, (int)sof, 0);
+}
+
+template <int P, typename T, int NS, bool TABLE, bool RES>
+__global__ void __launch_bounds__(16 * NS, 4)
+k_apply_box(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc)
+{
+#pragma clang fp contract(off)
+  constexpr BoxTab<P> tb = box_tab<P>();
+  constexpr int EJ = (P == 1) ? 2 : 1; // elements per axis in a 16-lane block
+  constexpr int FS = 4 * EJ;           // face values per block, plane and array
+  constexpr uint32_t SZ = sizeof(T);
+
+  const int wi = xcd_remap(blockIdx.x, gridDim.x);
+  int di = 0;
+  if constexpr (TABLE)
+    di = __builtin_amdgcn_readfirstlane(find_instance(wi, ndesc, [&](int i) { return descs[i].w0; }));
+  const ApplyDesc & ad = TABLE ? descs[di] : d0;
+  const int rb = TABLE ? ad.rb : 1;
+  const int ngrp = (ad.nrhs + rb - 1) / rb;
+  const int wl = wi - ad.w0;
+  const int r_begin = (wl % ngrp) * rb;
+  const int r_end = TABLE ? min(ad.nrhs, r_begin + rb) : r_begin + 1;
+  int tile = wl / ngrp;
+  const Geom & g = ad.g;
+  const int bcx = ad.bt.cx, bcy = ad.bt.cy;
+  const int tx = tile % ad.bt.ntx;
+  tile /= ad.bt.ntx;
+  const int ty = tile % ad.bt.nty, tz = tile / ad.bt.nty;
+
+  // face values; entry NS * FS is the zero that lanes without a neighbour add
+  constexpr int FZ = NS * FS;
+  __shared__ double sX[2][P][FZ + 1], sY[2][P][FZ + 1], sZR[2][P][FZ + 1], sZC[2][P][FZ + 1];
+  if (threadIdx.x < 2 * P)
+  {
+    const int b = threadIdx.x / P, k = threadIdx.x % P;
+    sX[b][k][FZ] = sY[b][k][FZ] = sZR[b][k][FZ] = sZC[b][k][FZ] = 0.0;
+  }
+
+  const int lane = threadIdx.x & 63;
+  const int lf = lane & 3, ls = lane >> 4;
+  const int slot = (threadIdx.x >> 6) * 4 + ((lane >> 2) & 3);
+  const int sx = slot % bcx, sy = slot / bcx;
+  const int nx = g.n[0], ny = g.n[1], nz = g.n[2];
+  const int xs = tx * (bcx * EJ - 1), ys = ty * (bcy * EJ - 1); // first computed element
+  const int z0 = tz * ad.bt.zc, z1 = min(nz, z0 + ad.bt.zc);
+  const int zs = z0 - (z0 > 0 ? 1 : 0);
+  const bool sact = sy < bcy;
+  const int pec = g.pec;
+
+  // element and local point of this lane on each axis: index f / s of the lane
+  const int ef = (P == 1) ? (lf >> 1) : 0, pf = (P == 1) ? (lf & 1) : lf;
+  const int es = (P == 1) ? (ls >> 1) : 0, ps = (P == 1) ? (ls & 1) : ls;
+  // N layout: x from f, y from s.  T layout: x from s, y from f.
+  const int exN = xs + sx * EJ + ef, eyN = ys + sy * EJ + es;
+  const int exT = xs + sx * EJ + es, eyT = ys + sy * EJ + ef;
+  const bool vN = sact && exN < nx && eyN < ny, vT = sact && exT < nx && eyT < ny;
+  auto face = [&](int axis, int gi, int n) {
+    return (gi == 0 && ((pec >> (2 * axis)) & 1)) || (gi == n * P && ((pec >> (2 * axis + 1)) & 1));
+  };
+  const bool essx = face(1, eyN * P + ps, ny), essy = face(0, exN * P + pf, nx), essz = essx || essy;
+  const bool essyT = face(0, exT * P + ps, nx);
+  // lanes that read a DOF of the component, and those that write it
+  const bool ldx = vN && pf < P && ps <= P, ldy = vT && pf < P && ps <= P, ldz = vN && pf <= P && ps <= P;
+  const bool outN = vN && (exN > xs || tx == 0) && (eyN > ys || ty == 0);
+  const bool topx = pf == P && exN == nx - 1, topy = ps == P && eyN == ny - 1;
+  const bool ownx = outN && pf < P && (ps < P || topy);
+  const bool owny = outN && ps < P && (pf < P || topx);
+  const bool ownz = outN && (pf < P || topx) && (ps < P || topy);
+  // some lane of the wave holds a PEC DOF of an x or y face; their values are
+  // kept in LDS from load to store (own lane, component y transposed): planes
+  // 1 .. p-1 of x and y and p planes of z of the layer, and the lowest plane of
+  // x and y of the layer (by parity of z: the one above is known a layer early)
+  const bool wave_ess = __any((vN && essz) || (vT && essyT)) != 0;
+  __shared__ double sE[3 * P + 2][16 * NS];
+  constexpr int EX = 0, EY = P - 1, EZ = 2 * P - 2, EX0 = 3 * P - 2, EY0 = 3 * P;
+  const int eN = threadIdx.x, eT = (threadIdx.x & ~51) | (lf << 4) | ls;
+  // byte offsets inside a plane of each component, from the tile's first row
+  const uint32_t cx0 = (uint32_t)g.cd[0][0], cy0 = (uint32_t)g.cd[1][0], cz0 = (uint32_t)g.cd[2][0];
+  const uint32_t lxN = (sx * EJ + ef) * P + pf, lyN = (sy * EJ + es) * P + ps;
+  const uint32_t oxN = (lyN * cx0 + lxN) * SZ, oyN = (lyN * cy0 + lxN) * SZ, ozN = (lyN * cz0 + lxN) * SZ;
+  const uint32_t oyT = (((sy * EJ + ef) * P + pf) * cy0 + (sx * EJ + es) * P + ps) * SZ;
+  const uint32_t ilx = ldx ? oxN : OOB, ily = ldy ? oyT : OOB, ilz = ldz ? ozN : OOB; // loads
+  // entries of a plane of each component
+  const int64_t plx = g.cd[0][0] * g.cd[0][1], ply = g.cd[1][0] * g.cd[1][1], plz = g.cd[2][0] * g.cd[2][1];
+  const uint32_t spx = (uint32_t)plx * SZ, spy = (uint32_t)ply * SZ, spz = (uint32_t)plz * SZ; // plane bytes
+  const int64_t orgx = g.off[0] + (int64_t)ys * P * cx0 + xs * P;
+  const int64_t orgy = g.off[1] + (int64_t)ys * P * cy0 + xs * P;
+  const int64_t orgz = g.off[2] + (int64_t)ys * P * cz0 + xs * P;
+
+  // face exchange: where this lane writes its upper faces and where it finds
+  // the values of the element to the left (x - 1), below (y - 1) and diagonal
+  const int wR = (slot * EJ + es) * 4 + lf; // row s = P, by x
+  const int wC = (slot * EJ + ef) * 4 + ls; // column f = P, by y
+  const bool hasL = pf == 0 && exN > xs, hasB = ps == 0 && eyN > ys;
+  const int slL = (P == 1 && ef == 1) ? slot : slot - 1, slB = (P == 1 && es == 1) ? slot : slot - bcx;
+  const int eL = (P == 1) ? 1 - ef : 0, eB = (P == 1) ? 1 - es : 0;
+  const int rL = hasL ? (slL * EJ + eL) * 4 + ls : FZ;
+  const int rB = hasB ? (slB * EJ + eB) * 4 + lf : FZ;
+  // diagonal: row P of the element below the left one, at its x point P
+  const int slD = (P == 1 && es == 1) ? slL : slL - bcx;
+  const int rD = (hasL && hasB) ? (slD * EJ + eB) * 4 + ((P == 1) ? 2 * eL + 1 : P) : FZ;
+
+  // matrix operands: lane (f, s) holds entry [f][s] as A and [s][f] as B
+  const bool dia = (P > 1) || (ef == es); // block-diagonal at order 1
+  double opM = 0, opD = 0, opDt = 0, wf = 0, wsl = 0;
+#pragma unroll
+  for (int i = 0; i <= P; i++)
+#pragma unroll
+    for (int j = 0; j <= P; j++)
+    {
+      if (pf == i && ps == j && dia)
+        opM = tb.M[i][j];
+      if (i < P && pf == i && ps == j && dia)
+        opD = tb.D[i][j]; // [open f][closed s]
+      if (i < P && ps == i && pf == j && dia)
+        opDt = tb.D[i][j]; // [open s][closed f]
+    }
+  const double opI = (lf == ls) ? 1.0 : 0.0;
+#pragma unroll
+  for (int i = 0; i < P; i++)
+  {
+    if (pf == i)
+      wf = tb.w[i];
+    if (ps == i)
+      wsl = tb.w[i];
+  }
+  // lane weights of the element factors (mass x, y, z; curl x, y, z): the
+  // weights of x and y are equal per axis up to the axis constants
+  const double msc = ad.mscale, csc = ad.cscale;
+  const double mk0 = ad.ef.mk[0] * msc, mk1 = ad.ef.mk[1] * msc, mk2 = ad.ef.mk[2] * msc;
+  const double ck0 = ad.ef.ck[0] * csc, ck1 = ad.ef.ck[1] * csc, ck2 = -(ad.ef.ck[2] * csc);
+  const double wfs = wf * wsl;
+
+  const T * qc = (const T *)ad.ef.qc + 2 * ((int64_t)ys * nx + xs);
+  const uint32_t oeN = vN ? ((uint32_t)(sy * EJ + es) * nx + sx * EJ + ef) * 2 * SZ : OOB;
+  const uint32_t oeT = vT ? ((uint32_t)(sy * EJ + ef) * nx + sx * EJ + es) * 2 * SZ : OOB;
+  const int64_t epl = 2 * (int64_t)nx * ny;
+
+  for (int rhs = r_begin; rhs < r_end; rhs++)
+  {
+    if (ad.done && gmem(ad.done)[(int64_t)rhs * ad.done_stride] != ad.gate)
+      continue;
+    const int64_t rof = (int64_t)rhs * g.off[3];
+    const T * xv = (const T *)ad.x + rof;
+    // offsets (entries) of the current layer's lowest plane of each component
+    int64_t bx = orgx + (int64_t)zs * P * plx, by = orgy + (int64_t)zs * P * ply, bz = orgz + (int64_t)zs * P * plz;
+
+    double ux[P + 1], uy[P + 1]; // this layer (uy in T layout)
+    T nux[P], nuy[P], nuz[P];    // next layer, as loaded
+    T nq[P == 1 ? 4 : 2];
+    auto load_layer = [&](int64_t ax, int64_t ay, int64_t az, int z) {
+#pragma unroll
+      for (int k = 0; k < P; k++)
+      {
+        nux[k] = ldb(xv + ax, ilx, (k + 1) * spx);
+        nuy[k] = ldb(xv + ay, ily, (k + 1) * spy);
+        nuz[k] = ldb(xv + az, ilz, k * spz);
+      }
+      const T * q = qc + z * epl;
+      nq[0] = ldb(q, oeN);
+      nq[1] = ldb(q + 1, oeN);
+      if constexpr (P == 1)
+      {
+        nq[2] = ldb(q, oeT);
+        nq[3] = ldb(q + 1, oeT);
+      }
+    };
+    {
+      const bool zf = zs == 0 && (pec & 16);
+      const T vx = ldb(xv + bx, ilx), vy = ldb(xv + by, ily);
+      load_layer(bx, by, bz, zs);
+      ux[0] = (zf || essx) ? 0.0 : (double)vx;
+      uy[0] = (zf || essyT) ? 0.0 : (double)vy;
+      sE[EX0 + (zs & 1)][eN] = (double)vx;
+      sE[EY0 + (zs & 1)][eT] = (double)vy;
+      // stores that store nothing: in the loop the loads of the next layer are
+      // followed by 3 p stores, and the wait for them may count on that only
+      // if every way into the loop has them
+#pragma unroll
+      for (int k = 0; k < 3 * P; k++)
+        stb((T *)ad.y + rof, OOB, T(0), k);
+    }
+    double carx = 0.0, cary = 0.0;
+    int buf = 0;
+    for (int z = zs; z < z1; z++)
+    {
+      double uz[P];
+      const bool ztop = z == nz - 1 && (pec & 32); // PEC top plane: u_x, u_y read as zero
+#pragma unroll
+      for (int k = 0; k < P; k++)
+      {
+        ux[k + 1] = (double)nux[k];
+        uy[k + 1] = (double)nuy[k];
+        uz[k] = (double)nuz[k];
+      }
+      // PEC DOFs act as zero; their values go to LDS
+      const bool stash = wave_ess || (z == 0 && (pec & 16));
+      if (stash)
+      {
+#pragma unroll
+        for (int k = 0; k < P; k++)
+        {
+          sE[EZ + k][eN] = uz[k];
+          uz[k] = essz ? 0.0 : uz[k];
+          if (k < P - 1)
+          {
+            sE[EX + k][eN] = ux[k + 1];
+            sE[EY + k][eT] = uy[k + 1];
+          }
+          else
+          {
+            sE[EX0 + ((z + 1) & 1)][eN] = ux[P];
+            sE[EY0 + ((z + 1) & 1)][eT] = uy[P];
+          }
+          ux[k + 1] = essx ? 0.0 : ux[k + 1];
+          uy[k + 1] = essyT ? 0.0 : uy[k + 1];
+        }
+      }
+      ux[P] = ztop ? 0.0 : ux[P];
+      uy[P] = ztop ? 0.0 : uy[P];
+      const double nuN = (double)nq[0], sgN = (double)nq[1];
+      const double nuT = (P == 1) ? (double)nq[P == 1 ? 2 : 0] : nuN, sgT = (P == 1) ? (double)nq[P == 1 ? 3 : 1] : sgN;
+      if (z + 1 < z1)
+        load_layer(bx + P * plx, by + P * ply, bz + P * plz, z + 1);
+
+      double yx[P + 1], yy[P + 1], yz[P];
+      {
+        // In phases (the scheduler keeps to them: the order holds the number of
+        // live registers below the 128 that four waves per SIMD leave each)
+        auto phase = []() { __builtin_amdgcn_sched_barrier(0); };
+        // curl components (c_y with reversed sign)
+        const double kcx = ck0 * (nuT * wf), kcy = ck1 * (nuN * wf), kcz = ck2 * (nuN * wfs);
+        const double kmx = mk0 * (sgN * wf), kmy = mk1 * (sgT * wf), kmz = mk2 * sgN;
+        double cxs[P], cys[P], ut[P];
+#pragma unroll
+        for (int q = 0; q < P; q++)
+          ut[q] = mm(uz[q], opI, 0.0); // u_z, T
+#pragma unroll
+        for (int q = 0; q < P; q++)
+        {
+          double dx = 0.0, dy = 0.0;
+#pragma unroll
+          for (int k = 0; k <= P; k++)
+          {
+            dx = __builtin_fma(-tb.D[q][k], ux[k], dx);
+            dy = __builtin_fma(-tb.D[q][k], uy[k], dy);
+          }
+          cxs[q] = mm(uz[q], opD, dy); // T: D_y u_z - D_z u_y
+          cys[q] = mm(ut[q], opD, dx); // N: D_x u_z - D_z u_x
+        }
+#pragma unroll
+        for (int q = 0; q < P; q++)
+        {
+          cys[q] *= kcy;
+          cxs[q] *= kcx;
+          uz[q] *= kmz;
+        }
+        phase();
+        // y_z = w (Mc_x Mc_y (sigma mk u_z) + D_x^T Mc_y cys + D_y^T Mc_x cxs),
+        // and the z contractions that y_x and y_y take from u_x, u_y and the curl
+#pragma unroll
+        for (int q = 0; q < P; q++)
+        {
+          const double p1 = mm(uz[q], opM, 0.0);  // T
+          const double p2 = mm(cys[q], opM, 0.0); // T
+          const double p3 = mm(cxs[q], opM, 0.0); // N
+          yz[q] = mm(p1, opM, 0.0);
+          yz[q] = mm(p2, opDt, yz[q]);
+          yz[q] = mm(opDt, p3, yz[q]);
+        }
+#pragma unroll
+        for (int k = 0; k <= P; k++)
+        {
+          double mx = 0.0, my = 0.0, ax = 0.0, ay = 0.0;
+#pragma unroll
+          for (int m = 0; m <= P; m++)
+          {
+            mx = __builtin_fma(tb.M[k][m], ux[m], mx);
+            my = __builtin_fma(tb.M[k][m], uy[m], my);
+          }
+#pragma unroll
+          for (int q = 0; q < P; q++)
+          {
+            ax = __builtin_fma(-(tb.w[q] * tb.D[q][k]), cys[q], ax);
+            ay = __builtin_fma(-(tb.w[q] * tb.D[q][k]), cxs[q], ay);
+          }
+          yx[k] = __builtin_fma(kmx, mx, ax);
+          yy[k] = __builtin_fma(kmy, my, ay);
+        }
+#pragma unroll
+        for (int q = 0; q < P; q++)
+          yz[q] *= tb.w[q];
+        phase();
+        double cz[P + 1];
+#pragma unroll
+        for (int k = 0; k <= P; k++)
+          cz[k] = mm(uy[k], opD, 0.0); // D_x u_y, N
+#pragma unroll
+        for (int k = 0; k <= P; k++)
+          cz[k] = mm<1>(opD, ux[k], cz[k]); // - D_y u_x
+        phase();
+        double f[P + 1], ft[P + 1];
+#pragma unroll
+        for (int k = 0; k <= P; k++)
+        {
+          double fk = 0.0;
+#pragma unroll
+          for (int m = 0; m <= P; m++)
+            fk = __builtin_fma(tb.M[k][m], cz[m], fk);
+          f[k] = kcz * fk; // - f_z, N
+        }
+#pragma unroll
+        for (int k = 0; k <= P; k++)
+          ft[k] = mm(f[k], opI, 0.0); // - f_z, T
+#pragma unroll
+        for (int k = 0; k <= P; k++)
+          f[k] = mm(opDt, f[k], 0.0); // - D_y^T f_z, N
+#pragma unroll
+        for (int k = 0; k <= P; k++)
+          ft[k] = mm<1>(ft[k], opDt, 0.0); // D_x^T f_z, N
+#pragma unroll
+        for (int k = 0; k <= P; k++)
+          yx[k] = mm(opM, yx[k], f[k]);
+#pragma unroll
+        for (int k = 0; k <= P; k++)
+          yy[k] = mm(yy[k], opM, ft[k]);
+      }
+      yx[0] = yx[0] + carx;
+      yy[0] = yy[0] + cary;
+      carx = yx[P];
+      cary = yy[P];
+      // the top plane becomes the bottom plane of the next layer
+      ux[0] = ux[P];
+      uy[0] = uy[P];
+      const int64_t cbx = bx, cby = by, cbz = bz;
+      bx += P * plx;
+      by += P * ply;
+      bz += P * plz;
+      // the lower halo layer of a chunk stores nothing (its top plane is
+      // carried); no branch around the stores: on a path without them the next
+      // layer's wait for its loads would have to wait for every store too
+      const bool zout = z >= z0;
+      const uint32_t jsx = (ownx && zout) ? ilx : OOB, jsy = (owny && zout) ? oyN : OOB;
+      const uint32_t jsz = (ownz && zout) ? ilz : OOB;
+
+      // face values to LDS; meanwhile b of the residual mode is on its way
+      if (ps == P)
+      {
+#pragma unroll
+        for (int k = 0; k < P; k++)
+        {
+          sX[buf][k][wR] = yx[k];
+          sZR[buf][k][wR] = yz[k];
+        }
+      }
+      if (pf == P)
+      {
+#pragma unroll
+        for (int k = 0; k < P; k++)
+        {
+          sY[buf][k][wC] = yy[k];
+          sZC[buf][k][wC] = yz[k];
+        }
+      }
+      T rbx[P], rby[P], rbz[P];
+      if constexpr (RES)
+      {
+        const T * bv = (const T *)ad.resid + rof;
+#pragma unroll
+        for (int k = 0; k < P; k++)
+        {
+          rbx[k] = ldb(bv + cbx, jsx, k * spx);
+          rby[k] = ldb(bv + cby, jsy, k * spy);
+          rbz[k] = ldb(bv + cbz, jsz, k * spz);
+        }
+      }
+      __syncthreads();
+      // left, then diagonal, then below: a fixed order for every tile shape
+#pragma unroll
+      for (int k = 0; k < P; k++)
+      {
+        yx[k] += sX[buf][k][rB];
+        yy[k] += sY[buf][k][rL];
+        yz[k] = ((yz[k] + sZC[buf][k][rL]) + sZR[buf][k][rD]) + sZR[buf][k][rB];
+      }
+      // PEC DOFs: y = x
+      if (stash)
+      {
+        const bool zf = z == 0 && (pec & 16);
+#pragma unroll
+        for (int k = 0; k < P; k++)
+        {
+          const double vx = k ? sE[EX + (k ? k - 1 : 0)][eN] : sE[EX0 + (z & 1)][eN];
+          const double vy = k ? sE[EY + (k ? k - 1 : 0)][eN] : sE[EY0 + (z & 1)][eN];
+          const double vz = sE[EZ + k][eN];
+          yx[k] = (essx || (zf && k == 0)) ? vx : yx[k];
+          yy[k] = (essy || (zf && k == 0)) ? vy : yy[k];
+          yz[k] = essz ? vz : yz[k];
+        }
+      }
+      if constexpr (RES)
+      {
+#pragma unroll
+        for (int k = 0; k < P; k++)
+        {
+          yx[k] = (double)rbx[k] - yx[k];
+          yy[k] = (double)rby[k] - yy[k];
+          yz[k] = (double)rbz[k] - yz[k];
+        }
+      }
+      T * yv = (T *)ad.y + rof;
+#pragma unroll
+      for (int k = 0; k < P; k++)
+      {
+        stb(yv + cbx, jsx, (T)yx[k], k * spx);
+        stb(yv + cby, jsy, (T)yy[k], k * spy);
+        stb(yv + cbz, jsz, (T)yz[k], k * spz);
+      }
+      buf ^= 1;
+    }
+    if (z1 == nz)
+    {
+      // top plane of the mesh (components x and y)
+      const bool zf = (pec & 32) != 0;
+      if (ps == P)
+        sX[buf][0][wR] = carx;
+      if (pf == P)
+        sY[buf][0][wC] = cary;
+      __syncthreads();
+      carx += sX[buf][0][rB];
+      cary += sY[buf][0][rL];
+      T * yv = (T *)ad.y + rof;
+      const uint32_t isx = ownx ? oxN : OOB, isy = owny ? oyN : OOB;
+      const T vx = ldb(xv + bx, isx), vy = ldb(xv + by, isy);
+      carx = (essx || zf) ? (double)vx : carx;
+      cary = (essy || zf) ? (double)vy : cary;
+      if constexpr (RES)
+      {
+        const T * bv = (const T *)ad.resid + rof;
+        carx = (double)ldb(bv + bx, isx) - carx;
+        cary = (double)ldb(bv + by, isy) - cary;
+      }
+      stb(yv + bx, isx, (T)carx);
+      stb(yv + by, isy, (T)cary);
+    }
+    if (TABLE && rhs + 1 < r_end)
+      __syncthreads(); // the next rhs starts over with buffer 0
+  }
+}
+
+// ---------------------------------------------------------------------------
+// tiles and launch
+// ---------------------------------------------------------------------------
+
+// Decomposition: for each number of slots the tile with the fewest tiles (ties:
+// the widest rows) and the chunk of layers with the least modelled time.  A
+// layer takes about 0.9 + 1.25 w us at order 3 with w waves per SIMD (measured:
+// 2.2 us alone, 5.9 us with four; the other orders scale alike), so a mesh that
+// leaves CUs idle takes small workgroups and short chunks (12^3 order 3: 7.8 us
+// with 16 slots, 14.6 us with 64), one that fills them the fewest duplicated
+// elements (48^3 order 3: 63 us with 64 slots, 78 us with 16).
+BoxTile
+box_tile(const Geom & g, int nrhs, int ns_only)
+{
+  const int ej = g.p == 1 ? 2 : 1;
+  auto tiles = [&](int n, int c) { return n <= c * ej ? 1 : (n - 1 + c * ej - 2) / (c * ej - 1); };
+  constexpr int CUS = 256;
+  BoxTile best{};
+  double cost = 1e300;
+  for (int ns = 16; ns <= 64; ns *= 2)
+  {
+    if (ns_only && ns != ns_only)
+      continue;
+    BoxTile b{};
+    b.ns = ns;
+    int64_t least = -1;
+    for (int cy = 1; cy <= ns; cy++)
+    {
+      const int cx = ns / cy;
+      if ((cy * ej < 2 && g.n[1] > 1) || (cx * ej < 2 && g.n[0] > 1))
+        continue;
+      const int ntx = tiles(g.n[0], cx), nty = tiles(g.n[1], cy);
+      const int64_t t = (int64_t)ntx * nty;
+      if (least < 0 || t < least || (t == least && cx > b.cx))
+      {
+        least = t;
+        b.cx = cx;
+        b.cy = cy;
+        b.ntx = ntx;
+        b.nty = nty;
+      }
+    }
+    const int bpc = 64 / ns, wpb = ns / 16; // workgroups per CU, waves per SIMD of one
+    const int64_t cap = (int64_t)CUS * bpc;
+    for (int zc = g.n[2];;)
+    {
+      const int nzc = (g.n[2] + zc - 1) / zc;
+      const int64_t blocks = least * nrhs * nzc, rem = blocks % cap;
+      double t = (double)(blocks / cap) * (0.9 + 1.25 * bpc * wpb);
+      if (rem)
+        t += 0.9 + 1.25 * wpb * (double)((rem + CUS - 1) / CUS);
+      t *= zc + (nzc > 1 ? 1.8 : 0.8);
+      if (t < cost)
+      {
+        cost = t;
+        best = b;
+        best.zc = zc;
+        best.nzc = nzc;
+      }
+      if (zc == 1)
+        break;
+      zc = std::min(zc - 1, (g.n[2] + nzc) / (nzc + 1)); // the next chunk length with more chunks
+    }
+  }
+  return best;
+}
+
+// The 32-bit offsets of the kernel: p planes of a component beyond a tile's
+// first row.
+bool
+box_fits(const Geom & g)
+{
+  int64_t pl = 0;
+  for (int c = 0; c < 3; c++)
+    pl = std::max(pl, g.cd[c][0] * g.cd[c][1]);
+  return (g.p + 1) * pl * (int64_t)sizeof(double) < (int64_t)0xFFFFF000;
+}
+
+template <typename T>
+hipError_t
+apply_box(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, int p, int ns, hipStream_t st)
+{
+  if (nwork <= 0)
+    return hipSuccess;
+  auto go = [&](auto pc, auto nc) {
+    constexpr int P = decltype(pc)::value, NS = decltype(nc)::value;
+    if (descs)
+      hipLaunchKernelGGL((k_apply_box<P, T, NS, true, false>), dim3(nwork), dim3(16 * NS), 0, st, d0, descs, ndesc);
+    else if (d0.resid)
+      hipLaunchKernelGGL((k_apply_box<P, T, NS, false, true>), dim3(nwork), dim3(16 * NS), 0, st, d0, descs, ndesc);
+    else
+      hipLaunchKernelGGL((k_apply_box<P, T, NS, false, false>), dim3(nwork), dim3(16 * NS), 0, st, d0, descs, ndesc);
+  };
+  auto by_ns = [&](auto pc) {
+    if (ns == 16)
+      go(pc, std::integral_constant<int, 16>{});
+    else if (ns == 32)
+      go(pc, std::integral_constant<int, 32>{});
+    else
+      go(pc, std::integral_constant<int, 64>{});
+  };
+  switch (p)
+  {
+  case 1:
+    by_ns(std::integral_constant<int, 1>{});
+    break;
+  case 2:
+    by_ns(std::integral_constant<int, 2>{});
+    break;
+  case 3:
+    by_ns(std::integral_constant<int, 3>{});
+    break;
+  default:
+    return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+template hipError_t apply_box<double>(const ApplyDesc &, const ApplyDesc *, int, int, int, int, hipStream_t);
+template hipError_t apply_box<float>(const ApplyDesc &, const ApplyDesc *, int, int, int, int, hipStream_t);
+
+} // namespace hc

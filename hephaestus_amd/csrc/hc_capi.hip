@@ -317,7 +317,7 @@ try
   if (op->box)
   {
     // element factors: J = diag(h), |det J| = h0 h1 h2
-    if ((rc = op->alloc(op->qc64, 2 * op->E)) || (op->qd32 && (rc = op->alloc(op->qc32, 2 * op->E))))
+    if (hc::box_fits(g) && ((rc = op->alloc(op->qc64, 2 * op->E)) || (op->qd32 && (rc = op->alloc(op->qc32, 2 * op->E)))))
     {
       delete op;
       return rc;
@@ -770,9 +770,13 @@ try
     hc::ApplyPlan & pl = prec == 64 ? op->plan64 : op->plan32;
     float best = 1e30f;
     const hc::TileCandidate * bestc = pl.cand;
-    for (int i = 0; i < n; i++)
+    // element factors: the box apply runs whatever the tile variant, which is
+    // kept; its time alone is measured
+    const bool box = op->ef(prec == 32).qc != nullptr;
+    for (int i = 0; i < (box ? 1 : n); i++)
     {
-      set_plan(op, pl, &c[i]);
+      if (!box)
+        set_plan(op, pl, &c[i]);
       auto run = [&]() -> int {
         return prec == 64 ? apply_t<double>(op, op->ws.r64, op->ws.q64, 1, nullptr, st)
                           : apply_t<float>(op, op->ws.r32, op->ws.q32, 1, nullptr, st);
@@ -791,7 +795,8 @@ try
       if (ms < best)
       {
         best = ms;
-        bestc = &c[i];
+        if (!box)
+          bestc = &c[i];
       }
     }
     set_plan(op, pl, bestc);
@@ -850,6 +855,9 @@ try
   d.nrhs = 1;
   d.rb = 1;
   d.ntiles = pl.g.nt[0] * pl.g.nt[1] * pl.g.nt[2];
+  const bool box = d.ef.qc != nullptr;
+  if (box)
+    hc::set_box_tile(d, hc::box_tile(pl.g, 1));
   const void * tb = f32 ? (const void *)&op->tb32 : (const void *)&op->tb64;
   std::vector<hipEvent_t> ev(3 * reps);
   for (auto & e : ev)
@@ -857,10 +865,15 @@ try
   for (int r = 0; r < reps; r++)
   {
     HC_TRY_HIP(hipEventRecord(ev[3 * r], st));
-    HC_TRY_HIP(pl.cand->launch(d, nullptr, 1, d.ntiles, 0, tb, prec_bits, st));
+    if (box)
+      HC_TRY_HIP(f32 ? hc::apply_box<float>(d, nullptr, 1, d.ntiles, pl.g.p, d.bt.ns, st)
+                     : hc::apply_box<double>(d, nullptr, 1, d.ntiles, pl.g.p, d.bt.ns, st));
+    else
+      HC_TRY_HIP(pl.cand->launch(d, nullptr, 1, d.ntiles, 0, tb, prec_bits, st));
     HC_TRY_HIP(hipEventRecord(ev[3 * r + 1], st));
-    HC_TRY_HIP(f32 ? hc::assemble_planes<float>(d, nullptr, 1, d.prows, st)
-                   : hc::assemble_planes<double>(d, nullptr, 1, d.prows, st));
+    if (!box)
+      HC_TRY_HIP(f32 ? hc::assemble_planes<float>(d, nullptr, 1, d.prows, st)
+                     : hc::assemble_planes<double>(d, nullptr, 1, d.prows, st));
     HC_TRY_HIP(hipEventRecord(ev[3 * r + 2], st));
   }
   HC_TRY_HIP(hipEventSynchronize(ev[3 * reps - 1]));
@@ -871,7 +884,7 @@ try
     HC_TRY_HIP(hipEventElapsedTime(&a, ev[3 * r], ev[3 * r + 1]));
     HC_TRY_HIP(hipEventElapsedTime(&b, ev[3 * r + 1], ev[3 * r + 2]));
     t_tile += a;
-    t_plane += b;
+    t_plane += box ? 0.0 : b;
   }
   for (auto & e : ev)
     (void)hipEventDestroy(e);

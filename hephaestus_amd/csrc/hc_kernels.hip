@@ -140,8 +140,10 @@ k_cast_f32(const double * __restrict__ a, float * __restrict__ b, int64_t n)
 // row is (plane k, position along the second in-plane axis); the threads
 // stride the first in-plane axis.  DOFs on the intersection of two plane
 // families are summed by the lower-numbered axis; fixed summation order.
+constexpr int PLANE_THREADS = 64;
+
 template <typename T, bool MULTI>
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(PLANE_THREADS)
 k_assemble_planes(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc)
 {
   const int w = blockIdx.x;
@@ -174,27 +176,20 @@ k_assemble_planes(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc)
   const int step2 = g.T[a2] * g.p;
   const int dlo = (c == 0) ? 1 : 0;
   const int64_t ebase = d.segs.eoff[c][a] + (int64_t)row * n0;
-  for (int j0 = threadIdx.x; j0 < n0; j0 += blockDim.x)
+  for (int j0 = threadIdx.x; j0 < n0; j0 += PLANE_THREADS)
   {
-    int gi[3];
-    gi[a] = k * g.T[a] * g.p;
-    gi[b0] = j0;
-    gi[b1] = j1;
-    const bool on2 = gi[a2] > 0 && gi[a2] < g.n[a2] * g.p && (gi[a2] % step2) == 0;
+    // grid indices by selects: an array indexed by the uniform axes would be
+    // moved to LDS with a stride read from the dispatch packet in host memory
+    // (12 us per launch)
+    const int ka = k * g.T[a] * g.p;
+    const int g0 = a == 0 ? ka : j0, g1 = a == 1 ? ka : (a == 0 ? j0 : j1), g2 = a == 2 ? ka : j1;
+    const int ga2 = a2 == 0 ? g0 : (a2 == 1 ? g1 : g2);
+    const bool on2 = ga2 > 0 && ga2 < g.n[a2] * g.p && (ga2 % step2) == 0;
     if (on2 && a2 < a)
       continue; // summed by the lower-numbered axis
-    bool ess = false;
-#pragma unroll
-    for (int q = 0; q < 3; q++)
-    {
-      if (q == c)
-        continue;
-      const int dim = (int)g.cd[c][q];
-      ess = ess || (gi[q] == 0 && ((g.pec >> (2 * q)) & 1)) || (gi[q] == dim - 1 && ((g.pec >> (2 * q + 1)) & 1));
-    }
-    if (ess)
+    if (is_ess(g, c, g0, g1, g2))
       continue; // written by the owning tile
-    const int64_t gid = g.off[c] + ((int64_t)gi[2] * g.cd[c][1] + gi[1]) * g.cd[c][0] + gi[0];
+    const int64_t gid = g.off[c] + ((int64_t)g2 * g.cd[c][1] + g1) * g.cd[c][0] + g0;
     // slot bits: bit 0 = lower-numbered closed axis, bit 1 = the other
     const bool on_lo = (a == dlo) ? true : on2;
     const bool on_hi = (a == dlo) ? on2 : true;
@@ -344,9 +339,9 @@ assemble_planes(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int np
   if (npwork <= 0)
     return hipSuccess;
   if (descs)
-    hipLaunchKernelGGL((k_assemble_planes<T, true>), dim3(npwork), dim3(64), 0, st, d0, descs, ndesc);
+    hipLaunchKernelGGL((k_assemble_planes<T, true>), dim3(npwork), dim3(PLANE_THREADS), 0, st, d0, descs, ndesc);
   else
-    hipLaunchKernelGGL((k_assemble_planes<T, false>), dim3(npwork), dim3(64), 0, st, d0, descs, ndesc);
+    hipLaunchKernelGGL((k_assemble_planes<T, false>), dim3(npwork), dim3(PLANE_THREADS), 0, st, d0, descs, ndesc);
   return hipGetLastError();
 }
 

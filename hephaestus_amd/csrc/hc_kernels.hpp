@@ -38,7 +38,7 @@ struct PlaneSegs
 // curl_a = dt nu_e w_q h_a^2 / |det J| (no off-diagonal terms), so a box
 // operator needs two numbers per element, qc[2e] = dt nu_e, qc[2e+1] =
 // sigma_e (element type of the launch), plus the axis constants
-// ck[a] = h_a^2 / |det J| and mk[a] = |det J| / h_a^2 and the 1D weights.
+// ck[a] = h_a^2 / |det J| and mk[a] = |det J| / h_a^2 (hc_apply_box.hip).
 // qc == nullptr: the quadrature-point factors qd are used.
 struct ElemFactors
 {
@@ -47,9 +47,18 @@ struct ElemFactors
   double mk[3] = {0, 0, 0};
 };
 
+// Decomposition of a box apply (hc_apply_box.hip): ns element slots per
+// workgroup, cx by cy of them per tile, ntx by nty tiles, nzc chunks of zc
+// element layers.
+struct BoxTile
+{
+  int ns, cx, cy, ntx, nty, zc, nzc;
+};
+
 struct ApplyDesc
 {
   Geom g;
+  BoxTile bt{};    // box apply only
   PlaneSegs segs;
   const void * qd; // quadrature data (element type of the launch)
   ElemFactors ef;  // element factors (box meshes), used instead of qd when set
@@ -174,9 +183,6 @@ xcd_remap(int b, int nb)
 // A compiled tile variant of the apply kernel (shape + load mode).
 // descs == nullptr: the single instance d0; otherwise ndesc instances.
 // grouped != 0 (with descs): work items are groups of rb right-hand sides.
-// grouped bit 0: rhs groups; bit 1 (LAUNCH_EF): every instance of descs carries
-// element factors (the single instance d0 is read from d0.ef.qc).
-constexpr int LAUNCH_EF = 2;
 using TileLaunch = hipError_t (*)(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, int grouped,
                                   const void * tables, int prec_bits, hipStream_t st);
 struct TileCandidate
@@ -253,6 +259,20 @@ hipError_t apply_op(const Geom & g,
                     int rb = 1,
                     ApplyDesc * desc_dev = nullptr,
                     const T * resid_b = nullptr);
+// The box apply (every instance reads element factors; ApplyDesc::bt set, ns
+// common to the launch), and its decomposition of a mesh for nrhs vectors
+// (ns_only: with that many slots).  The results do not depend on it.
+template <typename T>
+hipError_t apply_box(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, int p, int ns,
+                     hipStream_t st);
+bool box_fits(const Geom & g); // (32-bit offsets within a plane)
+BoxTile box_tile(const Geom & g, int nrhs, int ns_only = 0);
+inline void
+set_box_tile(ApplyDesc & d, const BoxTile & b)
+{
+  d.bt = b;
+  d.ntiles = b.ntx * b.nty * b.nzc;
+}
 // Right-hand sides per work item for a batch of nrhs on ntiles tiles.
 int default_rhs_block(int ntiles, int nrhs);
 // y = (mscale M + cscale K') x (K' = the curl part of the quadrature data,
@@ -267,10 +287,11 @@ hipError_t apply_scaled(const Geom & g, const PlaneSegs & segs, const Tables<T> 
 void plane_rows(ApplyDesc & d);
 
 // Apply over a device table of instances (all of one order, one tile variant).
-// nwork = sum of ntiles*nrhs, npwork = sum of prows*nrhs.
+// nwork = sum of ntiles*nrhs, npwork = sum of prows*nrhs.  box_ns != 0: every
+// instance reads element factors and runs the box apply with box_ns slots.
 template <typename T>
 hipError_t apply_multi(const TileCandidate * cand, const Tables<T> & tb, const ApplyDesc * descs_dev, int ndesc,
-                       int nwork, int npwork, int grouped, hipStream_t st);
+                       int nwork, int npwork, int grouped, int box_ns, hipStream_t st);
 
 // Sum of the tile-face partials (fixed order) into y.
 template <typename T>

@@ -122,6 +122,12 @@ try
   d.w0 = 0;
   d.pw0 = 0;
   d.ntiles = pl.g.nt[0] * pl.g.nt[1] * pl.g.nt[2];
+  if (d.ef.qc)
+  {
+    hc::set_box_tile(d, hc::box_tile(pl.g, 1));
+    HC_TRY_HIP(hc::apply_box<double>(d, nullptr, 1, d.ntiles, pl.g.p, d.bt.ns, st));
+    return HC_OK;
+  }
   HC_TRY_HIP(pl.cand->launch(d, nullptr, 1, d.ntiles, 0, &op->tb64, 64, st));
   HC_TRY_HIP(hc::assemble_planes<double>(d, nullptr, 1, d.prows, st));
   return HC_OK;

@@ -341,8 +341,8 @@ private:
     ApplyDesc single;  // by-value descriptor (batched == false)
     const ApplyDesc * descs; // device
     int ndesc, nwork, npwork;
-    int grouped; // bit 0: some instance groups rb > 1 right-hand sides per work item;
-                 // LAUNCH_EF: every instance reads element factors
+    int grouped; // some instance groups rb > 1 right-hand sides per work item
+    int box_ns;  // every instance reads element factors: slots of the box apply (0: tile kernels)
     const TileCandidate * cand;
     const void * tables; // Tables<double> or Tables<float>
     int prec;

@@ -269,7 +269,16 @@ Engine::set(const std::vector<EngineInst> & inst, int mode, int rhs_block, bool 
       G.ndesc = (int)ids.size();
       G.grouped = 0;
       int w0 = 0, pw0 = 0;
-      bool all_ef = true; // every instance has element factors: one launch reads them all
+      // every instance has element factors: one launch of the box apply;
+      // mixed: every instance reads its quadrature-point factors
+      bool all_ef = true;
+      int vecs = 0;
+      for (int i : ids)
+      {
+        all_ef = all_ef && inst_[i].op->ef(prec32).qc;
+        vecs += inst_[i].nrhs;
+      }
+      G.box_ns = all_ef ? box_tile(op0->g, vecs).ns : 0;
       for (int i : ids)
       {
         const EngineInst & e = inst_[i];
@@ -279,12 +288,13 @@ Engine::set(const std::vector<EngineInst> & inst, int mode, int rhs_block, bool 
         geom_for(op, G.cand, d.g, d.segs);
         d.prows = (int)d.segs.start[d.segs.nseg];
         d.ntiles = d.g.nt[0] * d.g.nt[1] * d.g.nt[2];
+        if (all_ef)
+          set_box_tile(d, box_tile(d.g, vecs, G.box_ns));
         d.nrhs = e.nrhs;
         d.rb = G.batched ? (rhs_block > 0 ? std::min(rhs_block, e.nrhs) : default_rhs_block(d.ntiles, e.nrhs)) : 1;
         d.qd = prec32 ? (const void *)op->qd32 : (const void *)op->qd64;
-        d.ef = op->ef(prec32);
-        if (!d.ef.qc)
-          all_ef = false;
+        if (all_ef)
+          d.ef = op->ef(prec32);
         if (k == K_PQ32)
         {
           d.x = w.p32;
@@ -320,13 +330,6 @@ Engine::set(const std::vector<EngineInst> & inst, int mode, int rhs_block, bool 
           G.single = d;
         hd[dpos++] = d;
       }
-      if (all_ef)
-        G.grouped |= LAUNCH_EF;
-      else // mixed: every instance reads its quadrature-point factors
-        for (size_t q = dpos - ids.size(); q < dpos; q++)
-          hd[q].ef = ElemFactors{};
-      if (!G.batched)
-        G.single = hd[dpos - 1];
       G.nwork = w0;
       G.npwork = pw0;
       groups_[k].push_back(G);
@@ -358,9 +361,12 @@ Engine::apply(Kind k, hipStream_t st)
     hipError_t e;
     if (G.batched)
       e = G.prec == 64 ? apply_multi<double>(G.cand, *(const Tables<double> *)G.tables, G.descs, G.ndesc, G.nwork,
-                                             G.npwork, G.grouped, st)
+                                             G.npwork, G.grouped, G.box_ns, st)
                        : apply_multi<float>(G.cand, *(const Tables<float> *)G.tables, G.descs, G.ndesc, G.nwork,
-                                            G.npwork, G.grouped, st);
+                                            G.npwork, G.grouped, G.box_ns, st);
+    else if (G.box_ns)
+      e = G.prec == 64 ? apply_box<double>(G.single, nullptr, 1, G.nwork, G.order, G.box_ns, st)
+                       : apply_box<float>(G.single, nullptr, 1, G.nwork, G.order, G.box_ns, st);
     else
     {
       e = G.cand->launch(G.single, nullptr, 1, G.nwork, 0, G.tables, G.prec, st);

@@ -178,13 +178,14 @@ int hc_op_precond_apply(hc_op_t op, int mode, const double * r, double * z, void
 int hc_op_term_ratio(hc_op_t op, double * ratio);
 
 /* Factor storage read by the apply kernels.  mode 1 (default): on an
- * axis-aligned box mesh (hc_mesh_desc.vert == NULL) the kernels read two
- * factors per element, dt nu_e and sigma_e, and form the quadrature-point
- * factors from them (J = diag(h): mass sigma_e w |det J| / h_a^2, curl
- * dt nu_e w h_a^2 / |det J|, no off-diagonal terms); other meshes read the
- * 12 (p+1)^3 quadrature-point factors per element of the partial assembly.
- * mode 0: the quadrature-point factors on every mesh.  The two agree to
- * round-off (a few units in the last place of each factor).  No counterpart
+ * axis-aligned box mesh (hc_mesh_desc.vert == NULL) the apply reads two
+ * factors per element, dt nu_e and sigma_e, and contracts with the exact 1-D
+ * matrices that the quadrature reduces to (J = diag(h)); its arithmetic is
+ * FP64 whatever the precision of the vectors, its results do not depend on
+ * a tile shape, and the tile variant (hc_op_set_tile) is not used.  Other
+ * meshes read the 12 (p+1)^3 quadrature-point factors per element of the
+ * partial assembly.  mode 0: the quadrature-point factors on every mesh.
+ * The two agree to round-off.  No counterpart
  * in the reference (MFEM's partial assembly stores the quadrature-point
  * factors).  hc_op_factor_mode: the storage the kernels read (0 or 1) or a
  * negative status. */
@@ -287,6 +288,8 @@ int hc_tile_list(int order, int * out, int max);
 int hc_op_get_tile(hc_op_t op, int prec_bits, int * tx, int * ty, int * tz, int * mode);
 /* Autotuner: times every compiled tile variant on this operator (after
  * hc_op_setup), `reps` applies each, and keeps the fastest per precision.
+ * With element factors (hc_op_set_factor_mode 1 on a box mesh) there is
+ * nothing to choose: the apply is timed and the variant kept.
  * best_us (optional, 2 entries): the winning FP64 / FP32 apply times.
  * No reference counterpart (the reference applies a CSR matrix). */
 int hc_op_autotune(hc_op_t op, int reps, double * best_us, void * stream);
@@ -434,7 +437,8 @@ int hc_fill_uniform(hc_op_t op, uint64_t seed, double * v, int64_t n, void * str
 /* Timing of `reps` single-RHS applies y = A x (prec_bits 64 or 32, x/y of
  * that precision) with HIP events around each kernel on `stream`: out_us[0] =
  * mean duration of the tile kernel, out_us[1] = of the tile-face assembly
- * kernel.  No reference counterpart (measurement entry point). */
+ * kernel (element factors: the whole apply, and zero).  No reference
+ * counterpart (measurement entry point). */
 int hc_op_profile_apply(hc_op_t op, int prec_bits, const void * x, void * y, int reps, double * out_us,
                         void * stream);
 /* Device vector helpers of the host layer.

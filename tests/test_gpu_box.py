@@ -1,0 +1,59 @@
+"""The box apply (element factors, needs an MI355X) at the edges of its
+decomposition.
+
+Its workgroups march columns of 16, 32 or 64 element slots along z, duplicate
+the elements of tile and chunk faces and choose slots, tile and chunk from the
+mesh and the number of right-hand sides.  Against the quadrature-point factors
+of the same operator (the tile kernels that the oracle tests pin): meshes of one
+element per direction, edges just below, at and above tile and chunk sizes, the
+block pairs of order 1 split by an odd edge, partial PEC, and sizes that take
+each number of slots.  Both sides carry rounding errors of a few units of
+2^-53 (1e-15 .. 3e-15 relative to 64-bit references), so 2e-14 bounds their
+difference with a margin; FP32 vectors differ by their own rounding, 2^-24 per
+entry of x and y, and the tile kernel's FP32 sums (1e-7 measured).  A result
+must not depend on the decomposition: several right-hand sides in one launch
+(another tile and chunk) are bitwise those of single launches.
+"""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def env():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    import hephaestus_amd as H
+    H.load()
+    return torch, H
+
+
+SIZES = [(1, 1, 1), (2, 1, 1), (1, 5, 2), (1, 1, 40), (3, 4, 5), (4, 4, 4), (5, 7, 9), (7, 8, 2), (8, 9, 17), (64, 2, 3),
+         (65, 1, 2), (9, 63, 5), (16, 15, 33), (48, 48, 11)]
+
+
+@pytest.mark.parametrize("p", [1, 2, 3])
+@pytest.mark.parametrize("n", SIZES)
+def test_box_apply_edges(env, p, n):
+    torch, H = env
+    pec = (0x3F, 0x19, 0x00, 0x26)[sum(n) % 4]
+    print(f"case box edges p={p} n={n} pec={pec:#x}", flush=True)
+    g = torch.Generator().manual_seed(sum(n) + p)
+    E = n[0] * n[1] * n[2]
+    nu = (0.5 + torch.rand(E, generator=g, dtype=torch.float64)).numpy()
+    sig = (10.0 ** (2.0 * torch.rand(E, generator=g, dtype=torch.float64))).numpy()
+    op = H.Operator(n, p, nu, sig, pec_faces=pec, length=(1.0, 0.7, 1.3)).setup(0.37)
+    X = (2.0 * torch.rand((5, op.ndofs), generator=g, dtype=torch.float64) - 1.0).cuda()
+    Y = op.apply(X)
+    y32 = op.apply_f32(X.float())
+    k = op.apply_curl(X[0].contiguous())
+    for r in range(5):
+        assert torch.equal(op.apply(X[r].contiguous()), Y[r]), r
+        assert torch.equal(op.apply_f32(X[r].float().contiguous()), y32[r]), r
+    op.set_factor_mode(0)
+    Yq, kq = op.apply(X), op.apply_curl(X[0].contiguous())
+    assert float((Y - Yq).norm()) <= 2e-14 * float(Yq.norm())
+    assert float((k - kq).norm()) <= 2e-14 * float(kq.norm())
+    assert float((y32.double() - Yq).norm()) <= 4e-7 * float(Yq.norm())
+    op.close()
