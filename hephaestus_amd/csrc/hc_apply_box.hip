@@ -59,51 +59,6 @@ namespace hc
 namespace
 {
 
-template <int P>
-struct BoxTab
-{
-  double M[P + 1][P + 1] = {}; // closed mass matrix
-  double D[P][P + 1] = {};     // derivative of the closed basis at the open points
-  double w[P] = {};            // open weights
-};
-
-template <int P>
-constexpr BoxTab<P>
-box_tab()
-{
-  BoxTab<P> t{};
-  const basis::Tab<double> b = basis::make_tab(P);
-  double on[PMAX] = {}, ow[PMAX] = {}, cn[PMAX + 1] = {};
-  basis::gauss_legendre01(P, on, ow);
-  basis::gauss_lobatto01(P + 1, cn);
-  for (int i = 0; i < P; i++)
-  {
-    double v[PMAX + 1] = {}, d[PMAX + 1] = {};
-    basis::lagrange(P + 1, cn, on[i], v, d);
-    t.w[i] = ow[i];
-    for (int m = 0; m <= P; m++)
-      t.D[i][m] = d[m];
-  }
-  // entries that are equal by symmetry get one value (one scalar register pair)
-  for (int a = 0; a <= P; a++)
-    for (int c = 0; c <= P; c++)
-    {
-      const int m = a < c ? a : c, n = a < c ? c : a;       // M[a][c] = M[c][a]
-      const bool flip = m + n > P; // = M[P-c][P-a]
-      const int i = flip ? P - n : m, j = flip ? P - m : n;
-      for (int q = 0; q <= P; q++)
-        t.M[a][c] += b.qw[q] * b.Bc[q * (P + 1) + i] * b.Bc[q * (P + 1) + j];
-    }
-  for (int i = 0; i < P; i++)
-  {
-    t.w[i] = ow[i <= P - 1 - i ? i : P - 1 - i];
-    for (int m = 0; m <= P; m++)
-      if (2 * i > P - 1 || (2 * i == P - 1 && 2 * m > P))
-        t.D[i][m] = -t.D[P - 1 - i][P - m];
-  }
-  return t;
-}
-
 // a b + c; NEG: bit 0 negates a (operand modifier of the FP64 form)
 template <int NEG = 0>
 __device__ inline double
@@ -153,7 +108,7 @@ __global__ void __launch_bounds__(16 * NS, 4)
 k_apply_box(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc)
 {
 #pragma clang fp contract(off)
-  constexpr BoxTab<P> tb = box_tab<P>();
+  constexpr basis::BoxTab<P> tb = basis::box_tab<P>();
   constexpr int EJ = (P == 1) ? 2 : 1; // elements per axis in a 16-lane block
   constexpr int FS = 4 * EJ;           // face values per block, plane and array
   constexpr uint32_t SZ = sizeof(T);

@@ -179,7 +179,7 @@ try
     // diagonal and the node diagonal of G^T M G
     hipLaunchKernelGGL(hc::k_fill_value, dim3(256), dim3(256), 0, st, E, 0.0, c0);
     hipLaunchKernelGGL(hc::k_fill_value, dim3(256), dim3(256), 0, st, E, 1.0, c1);
-    HC_TRY_HIP(hc::pa_setup(op->g, op->tb64, op->d_vert, op->h, c0, c1, 1.0, qdu, st));
+    HC_TRY_HIP(hc::pa_setup(op->g, op->tb64, op->d_vert, op->h, c0, c1, 1.0, qdu, nullptr, st));
     HC_TRY_HIP(hc::diagonal(g0, op->tb64, qdu, dM, st));
     HC_TRY_HIP(hc::invert_diag(dM, dM, nullptr, N, st));
     HC_TRY_HIP(hc::aux_diag_inv(g0, op->ag, op->tb64, qdu, dS, dS, nullptr, st));

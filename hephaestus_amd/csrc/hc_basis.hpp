@@ -199,5 +199,52 @@ tab()
   return cast_tab<T>(make_tab(P));
 }
 
+// Exact 1-D matrices of order P on [0, 1], which the integrals over a box
+// element separate into (the p + 1 point rule integrates them exactly).
+template <int P>
+struct BoxTab
+{
+  double M[P + 1][P + 1] = {}; // closed mass matrix
+  double D[P][P + 1] = {};     // derivative of the closed basis at the open points
+  double w[P] = {};            // open weights
+};
+
+template <int P>
+__host__ __device__ constexpr BoxTab<P>
+box_tab()
+{
+  BoxTab<P> t{};
+  const Tab<double> b = make_tab(P);
+  double on[PMAX] = {}, ow[PMAX] = {}, cn[PMAX + 1] = {};
+  gauss_legendre01(P, on, ow);
+  gauss_lobatto01(P + 1, cn);
+  for (int i = 0; i < P; i++)
+  {
+    double v[PMAX + 1] = {}, d[PMAX + 1] = {};
+    lagrange(P + 1, cn, on[i], v, d);
+    t.w[i] = ow[i];
+    for (int m = 0; m <= P; m++)
+      t.D[i][m] = d[m];
+  }
+  // entries that are equal by symmetry get one value (one scalar register pair)
+  for (int a = 0; a <= P; a++)
+    for (int c = 0; c <= P; c++)
+    {
+      const int m = a < c ? a : c, n = a < c ? c : a;       // M[a][c] = M[c][a]
+      const bool flip = m + n > P; // = M[P-c][P-a]
+      const int i = flip ? P - n : m, j = flip ? P - m : n;
+      for (int q = 0; q <= P; q++)
+        t.M[a][c] += b.qw[q] * b.Bc[q * (P + 1) + i] * b.Bc[q * (P + 1) + j];
+    }
+  for (int i = 0; i < P; i++)
+  {
+    t.w[i] = ow[i <= P - 1 - i ? i : P - 1 - i];
+    for (int m = 0; m <= P; m++)
+      if (2 * i > P - 1 || (2 * i == P - 1 && 2 * m > P))
+        t.D[i][m] = -t.D[P - 1 - i][P - m];
+  }
+  return t;
+}
+
 } // namespace basis
 } // namespace hc

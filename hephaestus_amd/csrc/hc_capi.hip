@@ -393,18 +393,31 @@ try
     HC_TRY_HIP(hipMemcpyAsync(op->d_nu, op->nu.data(), op->E * sizeof(double), hipMemcpyHostToDevice, st));
     HC_TRY_HIP(hipMemcpyAsync(op->d_sig, op->sig.data(), op->E * sizeof(double), hipMemcpyHostToDevice, st));
   }
-  HC_TRY_HIP(hc::pa_setup(op->g, op->tb64, op->d_vert, op->h, op->d_nu, op->d_sig, dt, op->qd64, st));
-  const int Q = op->p + 1;
-  if (op->qd32)
-    HC_TRY_HIP(hc::cast_f32(op->qd64, op->qd32, op->E * 12 * Q * Q * Q, st));
+  HC_TRY_HIP(hc::pa_setup(op->g, op->tb64, op->d_vert, op->h, op->d_nu, op->d_sig, dt, op->qd64, op->qd32, st));
+  // element factors of a box mesh; sigma h^2 / nu per element (block minima)
   if (op->qc64)
-    HC_TRY_HIP(hc::elem_factors(op->E, op->d_nu, op->d_sig, dt, op->qc64, op->qc32, st));
-  HC_TRY_HIP(hc::diagonal(op->g, op->tb64, op->qd64, op->diag, st));
-  HC_TRY_HIP(hc::invert_diag(op->diag, op->dinv64, op->dinv32, op->N, st));
-  // node diagonal of the gradient-space correction (computed in place)
-  HC_TRY_HIP(hc::aux_diag_inv(op->g, op->ag, op->tb64, op->qd64, op->ginv64, op->ginv64, op->ginv32, st));
-  // sigma h^2 / nu per element (block minima)
-  HC_TRY_HIP(hc::term_ratio_blocks(op->qd64, op->E, op->p, op->d_ratio, st));
+    HC_TRY_HIP(hc::elem_factors(op->E, op->d_nu, op->d_sig, dt, op->ck, op->mk, op->qc64, op->qc32, op->d_ratio, st));
+  else
+    HC_TRY_HIP(hc::term_ratio_blocks(op->qd64, op->E, op->p, op->d_ratio, st));
+  // Jacobi diagonal, and the node diagonal of the gradient-space correction
+  // (in closed form on box meshes, whatever storage the apply reads)
+  if (op->qc64 && (int64_t)op->g.n[2] * op->p + 1 < 65536)
+  {
+    hc::ElemFactors ef;
+    ef.qc = op->qc64;
+    for (int a = 0; a < 3; a++)
+    {
+      ef.ck[a] = op->ck[a];
+      ef.mk[a] = op->mk[a];
+    }
+    HC_TRY_HIP(hc::diagonals_box(op->g, ef, op->diag, op->dinv64, op->dinv32, op->ginv64, op->ginv32, st));
+  }
+  else
+  {
+    HC_TRY_HIP(hc::diagonal(op->g, op->tb64, op->qd64, op->diag, st));
+    HC_TRY_HIP(hc::invert_diag(op->diag, op->dinv64, op->dinv32, op->N, st));
+    HC_TRY_HIP(hc::aux_diag_inv(op->g, op->ag, op->tb64, op->qd64, op->ginv64, op->ginv64, op->ginv32, st));
+  }
   double rmin[hc::TERM_RATIO_BLOCKS];
   HC_TRY_HIP(hipMemcpyAsync(rmin, op->d_ratio, sizeof(rmin), hipMemcpyDeviceToHost, st));
   HC_TRY_HIP(hipStreamSynchronize(st));

@@ -10,6 +10,7 @@
 // The apply is the operator EquationSystem::Mult (equation_system.cpp:200-204)
 // on the PEC-eliminated system of FormLinearSystem (equation_system.cpp:132-190):
 // y_free = (A x_free)_free, y_ess = x_ess.
+#include "hc_basis.hpp"
 #include "hc_kernels.hpp"
 
 #include <algorithm>
@@ -67,7 +68,8 @@ k_pa_setup(Geom g,
            const double * __restrict__ curl_coef,
            const double * __restrict__ mass_coef,
            double curl_scale,
-           double * __restrict__ qd)
+           double * __restrict__ qd,
+           float * __restrict__ qd32) // FP32 copy, may be null
 {
   const int Q = g.p + 1, Q3 = Q * Q * Q;
   const int64_t E = (int64_t)g.n[0] * g.n[1] * g.n[2];
@@ -125,7 +127,12 @@ k_pa_setup(Geom g,
   point_factors(J, w * mass_coef[e], w * curl_scale * curl_coef[e], f);
 #pragma unroll
   for (int k = 0; k < 12; k++)
-    qd[((e * Q + qz) * 12 + k) * Q * Q + qy * Q + qx] = f[k];
+  {
+    const int64_t o = ((e * Q + qz) * 12 + k) * Q * Q + qy * Q + qx;
+    qd[o] = f[k];
+    if (qd32)
+      qd32[o] = (float)f[k];
+  }
 }
 
 __global__ void
@@ -350,21 +357,25 @@ template hipError_t assemble_planes<float>(const ApplyDesc &, const ApplyDesc *,
 
 hipError_t
 pa_setup(const Geom & g, const Tables<double> & tb, const double * vert, const double h[3],
-         const double * curl_coef, const double * mass_coef, double curl_scale, double * qd, hipStream_t st)
+         const double * curl_coef, const double * mass_coef, double curl_scale, double * qd, float * qd32,
+         hipStream_t st)
 {
   const int Q = g.p + 1;
   const int64_t n = (int64_t)g.n[0] * g.n[1] * g.n[2] * Q * Q * Q;
   hipLaunchKernelGGL(k_pa_setup, dim3(div_up(n, 256)), dim3(256), 0, st, g, tb, vert, h[0], h[1], h[2], curl_coef,
-                     mass_coef, curl_scale, qd);
+                     mass_coef, curl_scale, qd, qd32);
   return hipGetLastError();
 }
 
 // Element factors of a box mesh: qc[2e] = dt nu_e, qc[2e+1] = sigma_e (and
-// their FP32 copies when qc32 is set).
-__global__ void
-k_elem_factors(int64_t E, const double * __restrict__ nu, const double * __restrict__ sig, double dt,
-               double * __restrict__ qc, float * __restrict__ qc32)
+// their FP32 copies when qc32 is set), and per block the minimum of
+// ratio sigma_e / (dt nu_e), the term ratio of k_term_ratio.
+__global__ void __launch_bounds__(256)
+k_elem_factors(int64_t E, const double * __restrict__ nu, const double * __restrict__ sig, double dt, double ratio,
+               double * __restrict__ qc, float * __restrict__ qc32, double * __restrict__ rmin)
 {
+  __shared__ double sh[256];
+  double v = 1.0e300;
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < E; e += (int64_t)gridDim.x * blockDim.x)
   {
     const double a = dt * nu[e], b = sig[e];
@@ -375,13 +386,177 @@ k_elem_factors(int64_t E, const double * __restrict__ nu, const double * __restr
       qc32[2 * e] = (float)a;
       qc32[2 * e + 1] = (float)b;
     }
+    const double r = a > 0.0 ? ratio * (b / a) : 1.0e300;
+    v = r < v ? r : v;
   }
+  sh[threadIdx.x] = v;
+  __syncthreads();
+  for (int s2 = 128; s2 > 0; s2 >>= 1)
+  {
+    if ((int)threadIdx.x < s2 && sh[threadIdx.x + s2] < sh[threadIdx.x])
+      sh[threadIdx.x] = sh[threadIdx.x + s2];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0)
+    rmin[blockIdx.x] = sh[0];
 }
 
 hipError_t
-elem_factors(int64_t E, const double * nu, const double * sig, double dt, double * qc, float * qc32, hipStream_t st)
+elem_factors(int64_t E, const double * nu, const double * sig, double dt, const double ck[3], const double mk[3],
+             double * qc, float * qc32, double * rmin, hipStream_t st)
 {
-  hipLaunchKernelGGL(k_elem_factors, dim3(1024), dim3(256), 0, st, E, nu, sig, dt, qc, qc32);
+  const double ratio = (mk[0] + mk[1] + mk[2]) / (ck[0] + ck[1] + ck[2]);
+  hipLaunchKernelGGL(k_elem_factors, dim3(TERM_RATIO_BLOCKS), dim3(256), 0, st, E, nu, sig, dt, ratio, qc, qc32, rmin);
+  return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// Diagonals of a box mesh in closed form.  With the exact 1-D matrices
+// (hc_basis.hpp) the diagonal entry of a DOF of component c (open index i along
+// c, closed indices j, k along the axes a1 < a2) sums, over its at most four
+// elements,
+//   w_i (sigma mk_c M_jj M_kk + dt nu (ck_a1 M_jj K_kk + ck_a2 K_jj M_kk)),
+// K = D^T W D, and the node diagonal of G^T M_sigma G, over at most eight,
+//   sigma (mk_0 K M M + mk_1 M K M + mk_2 M M K).
+// One thread per entry reads the factors of its elements and writes the entry,
+// its inverse and the FP32 copies: bound by those writes.  At 32^3 order 2 the
+// element-coloured sums over the quadrature-point factors (k_diag_elem,
+// k_aux_diag, which other meshes keep) took 362 of the 512 us of a set-up with
+// its first product; the same pass takes 110 us now.
+// ---------------------------------------------------------------------------
+struct DiagTab
+{
+  double M[PMAX + 1], K[PMAX + 1], w[PMAX];
+};
+
+template <int P>
+static DiagTab
+diag_tab()
+{
+  constexpr basis::BoxTab<P> t = basis::box_tab<P>();
+  DiagTab d{};
+  for (int j = 0; j <= P; j++)
+  {
+    d.M[j] = t.M[j][j];
+    for (int q = 0; q < P; q++)
+      d.K[j] += t.w[q] * t.D[q][j] * t.D[q][j];
+  }
+  for (int q = 0; q < P; q++)
+    d.w[q] = t.w[q];
+  return d;
+}
+
+static DiagTab
+diag_tab(int p)
+{
+  return p == 1 ? diag_tab<1>() : (p == 2 ? diag_tab<2>() : diag_tab<3>());
+}
+
+// elements that share closed point gi of an axis of n elements: first, count;
+// local point in the first (the other holds it as its point 0)
+__device__ inline void
+closed_elems(int gi, int n, int p, int & e0, int & cnt, int & m0)
+{
+  const int e = gi / p, m = gi - e * p;
+  const bool lower = m == 0 && gi > 0;
+  e0 = lower ? e - 1 : e;
+  m0 = lower ? p : m;
+  cnt = (lower && e < n) ? 2 : 1;
+}
+
+__global__ void __launch_bounds__(256)
+k_diag_box(Geom g, ElemFactors ef, DiagTab tab, double * __restrict__ d, double * __restrict__ d64,
+           float * __restrict__ d32)
+{
+  __shared__ DiagTab t;
+  if (threadIdx.x == 0)
+    t = tab;
+  __syncthreads();
+  const int c = blockIdx.z, a1 = c == 0 ? 1 : 0, a2 = c == 2 ? 1 : 2;
+  const int n0 = (int)g.cd[c][0], n1 = (int)g.cd[c][1], n2 = (int)g.cd[c][2];
+  const unsigned pt = blockIdx.x * 256 + threadIdx.x;
+  const int i2 = blockIdx.y;
+  if (pt >= (unsigned)n0 * (unsigned)n1 || i2 >= n2)
+    return;
+  const int i1 = (int)(pt / (unsigned)n0), i0 = (int)(pt - (unsigned)i1 * (unsigned)n0);
+  const double * __restrict__ qc = (const double *)ef.qc;
+  const int ic = c == 0 ? i0 : (c == 1 ? i1 : i2), j = a1 == 0 ? i0 : i1, k = a2 == 1 ? i1 : i2;
+  const int ec = ic / g.p, l = ic - ec * g.p;
+  int ej, nj, mj, ek, nk, mk;
+  closed_elems(j, a1 == 0 ? g.n[0] : g.n[1], g.p, ej, nj, mj);
+  closed_elems(k, a2 == 1 ? g.n[1] : g.n[2], g.p, ek, nk, mk);
+  const double mkc = c == 0 ? ef.mk[0] : (c == 1 ? ef.mk[1] : ef.mk[2]);
+  const double ck1 = a1 == 0 ? ef.ck[0] : ef.ck[1], ck2 = a2 == 1 ? ef.ck[1] : ef.ck[2];
+  const int64_t st[3] = {1, g.n[0], (int64_t)g.n[0] * g.n[1]};
+  const int64_t sc = c == 0 ? st[0] : (c == 1 ? st[1] : st[2]), s1 = a1 == 0 ? st[0] : st[1];
+  const int64_t s2 = a2 == 1 ? st[1] : st[2];
+  double v = 0.0;
+  for (int bk = 0; bk < nk; bk++)
+    for (int bj = 0; bj < nj; bj++)
+    {
+      const int64_t e = ec * sc + (ej + bj) * s1 + (ek + bk) * s2;
+      const double Mj = t.M[bj ? 0 : mj], Kj = t.K[bj ? 0 : mj], Mk = t.M[bk ? 0 : mk], Kk = t.K[bk ? 0 : mk];
+      v += qc[2 * e + 1] * (mkc * (Mj * Mk)) + qc[2 * e] * (ck1 * (Mj * Kk) + ck2 * (Kj * Mk));
+    }
+  v = is_ess(g, c, i0, i1, i2) ? 1.0 : v * t.w[l];
+  const int64_t o = g.off[c] + ((int64_t)i2 * n1 + i1) * n0 + i0;
+  const double r = 1.0 / v;
+  d[o] = v;
+  d64[o] = r;
+  if (d32)
+    d32[o] = (float)r;
+}
+
+__global__ void __launch_bounds__(256)
+k_node_diag_box(Geom g, ElemFactors ef, DiagTab tab, double * __restrict__ g64, float * __restrict__ g32)
+{
+  __shared__ DiagTab t;
+  if (threadIdx.x == 0)
+    t = tab;
+  __syncthreads();
+  const int n0 = g.n[0] * g.p + 1, n1 = g.n[1] * g.p + 1, n2 = g.n[2] * g.p + 1;
+  const unsigned pt = blockIdx.x * 256 + threadIdx.x;
+  const int i2 = blockIdx.y;
+  if (pt >= (unsigned)n0 * (unsigned)n1)
+    return;
+  const int i1 = (int)(pt / (unsigned)n0), i0 = (int)(pt - (unsigned)i1 * (unsigned)n0);
+  const double * __restrict__ qc = (const double *)ef.qc;
+  int e0, c0, m0, e1, c1, m1, e2, c2, m2;
+  closed_elems(i0, g.n[0], g.p, e0, c0, m0);
+  closed_elems(i1, g.n[1], g.p, e1, c1, m1);
+  closed_elems(i2, g.n[2], g.p, e2, c2, m2);
+  double v = 0.0;
+  for (int b2 = 0; b2 < c2; b2++)
+    for (int b1 = 0; b1 < c1; b1++)
+      for (int b0 = 0; b0 < c0; b0++)
+      {
+        const int64_t e = ((int64_t)(e2 + b2) * g.n[1] + (e1 + b1)) * g.n[0] + e0 + b0;
+        const double Mx = t.M[b0 ? 0 : m0], My = t.M[b1 ? 0 : m1], Mz = t.M[b2 ? 0 : m2];
+        v += qc[2 * e + 1] * (ef.mk[0] * (t.K[b0 ? 0 : m0] * (My * Mz)) + ef.mk[1] * (Mx * (t.K[b1 ? 0 : m1] * Mz)) +
+                              ef.mk[2] * (Mx * (My * t.K[b2 ? 0 : m2])));
+      }
+  bool ess = false;
+  const int idx[3] = {i0, i1, i2}, dim[3] = {n0, n1, n2};
+#pragma unroll
+  for (int a = 0; a < 3; a++)
+    ess = ess || (idx[a] == 0 && ((g.pec >> (2 * a)) & 1)) || (idx[a] == dim[a] - 1 && ((g.pec >> (2 * a + 1)) & 1));
+  const double inv = (ess || !(v > 0.0)) ? 0.0 : 1.0 / v;
+  const int64_t o = ((int64_t)i2 * n1 + i1) * n0 + i0;
+  g64[o] = inv;
+  if (g32)
+    g32[o] = (float)inv;
+}
+
+hipError_t
+diagonals_box(const Geom & g, const ElemFactors & ef, double * d, double * dinv64, float * dinv32, double * ginv64,
+              float * ginv32, hipStream_t st)
+{
+  const DiagTab tab = diag_tab(g.p);
+  const int64_t m0 = (int64_t)g.n[0] * g.p + 1, m1 = (int64_t)g.n[1] * g.p + 1, m2 = (int64_t)g.n[2] * g.p + 1;
+  // the planes of z go over a grid dimension limited to 65535: the coloured sums serve longer meshes
+  const dim3 grid((unsigned)((m0 * m1 + 255) / 256), (unsigned)m2, 3);
+  hipLaunchKernelGGL(k_diag_box, grid, dim3(256), 0, st, g, ef, tab, d, dinv64, dinv32);
+  hipLaunchKernelGGL(k_node_diag_box, dim3(grid.x, grid.y), dim3(256), 0, st, g, ef, tab, ginv64, ginv32);
   return hipGetLastError();
 }
 

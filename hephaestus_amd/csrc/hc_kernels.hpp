@@ -211,12 +211,18 @@ hipError_t pa_setup(const Geom & g,
                     const double * mass_coef,
                     double curl_scale,
                     double * qd,
+                    float * qd32, // FP32 copy, or null
                     hipStream_t st);
 hipError_t cast_f32(const double * a, float * b, int64_t n, hipStream_t st);
 // Element factors of a box mesh (ElemFactors::qc): dt nu_e, sigma_e per
-// element, FP64 and (qc32 != nullptr) FP32.
-hipError_t elem_factors(int64_t E, const double * nu, const double * sig, double dt, double * qc, float * qc32,
-                        hipStream_t st);
+// element, FP64 and (qc32 != nullptr) FP32, and the block minima of the term
+// ratio (TERM_RATIO_BLOCKS doubles, as term_ratio_blocks).
+hipError_t elem_factors(int64_t E, const double * nu, const double * sig, double dt, const double ck[3],
+                        const double mk[3], double * qc, float * qc32, double * rmin, hipStream_t st);
+// Jacobi diagonal and node diagonal of a box mesh (ef.qc: the FP64 factors)
+// with their inverses; dinv32, ginv32 may be null.  z planes below 65536.
+hipError_t diagonals_box(const Geom & g, const ElemFactors & ef, double * d, double * dinv64, float * dinv32,
+                         double * ginv64, float * ginv32, hipStream_t st);
 
 // Coil-like current J = curl psi, psi = sum_k a_k exp(-|x - c_k|^2 / (2 s_k^2)),
 // with its Gauss rule (p + 2 points) and the ND basis at those points.

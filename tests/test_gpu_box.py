@@ -57,3 +57,33 @@ def test_box_apply_edges(env, p, n):
     assert float((k - kq).norm()) <= 2e-14 * float(kq.norm())
     assert float((y32.double() - Yq).norm()) <= 4e-7 * float(Yq.norm())
     op.close()
+
+
+@pytest.mark.parametrize("p", [1, 2, 3])
+@pytest.mark.parametrize("n,pec", [((1, 1, 1), 0x3F), ((1, 1, 1), 0x00), ((2, 1, 3), 0x15), ((5, 4, 6), 0x2A), ((7, 33, 2), 0x3F)])
+def test_box_diagonals(env, p, n, pec):
+    """The closed-form Jacobi and node diagonals of a box mesh (the latter
+    through the gradient-corrected preconditioner) and its term ratio equal
+    those of the same mesh given by its vertices, which are summed over the
+    quadrature-point factors.  Every entry is a sum of positive terms, so both
+    are within some 50 roundings of the exact value: 1e-13."""
+    torch, H = env
+    import numpy as np
+    print(f"case box diagonals p={p} n={n} pec={pec:#x}", flush=True)
+    rng = np.random.default_rng(11 * p + sum(n))
+    E = n[0] * n[1] * n[2]
+    nu, sig = rng.uniform(0.5, 2.0, E), 10.0 ** rng.uniform(-3, 3, E)
+    L = (1.0, 0.6, 1.5)
+    Z, Y, X = np.meshgrid(*[L[a] * np.arange(n[a] + 1) / n[a] for a in (2, 1, 0)], indexing="ij")
+    vert = np.stack([X, Y, Z], -1).reshape(-1, 3)
+    box = H.Operator(n, p, nu, sig, pec_faces=pec, length=L).setup(0.25)
+    ref = H.Operator(n, p, nu, sig, pec_faces=pec, vert=vert).setup(0.25)
+    d, dr = box.diagonal(), ref.diagonal()
+    assert float(((d - dr) / dr).abs().max()) <= 1e-13
+    r = torch.from_numpy(rng.uniform(-1, 1, box.ndofs)).cuda()
+    for mode in (H.SOLVE_FP64, H.SOLVE_FP64 | H.SOLVE_AUX):
+        z, zr = box.precond_apply(r, mode), ref.precond_apply(r, mode)
+        assert float((z - zr).norm()) <= 1e-12 * float(zr.norm()), mode
+    assert abs(box.term_ratio / ref.term_ratio - 1.0) <= 1e-13
+    box.close()
+    ref.close()
