@@ -206,9 +206,9 @@ k_aux_z_single(AuxGeom a, const double * __restrict__ dinv, const double * __res
 }
 
 // One smoothing step after t = Dg^-1 G^T r: z = D^-1 r + G t, then the
-// Chebyshev (or damped) update d = ca z + cb d, x += d, in one pass
-// (flags 1: fresh d, d = ca z; 2: fresh x, x = d).  The same arithmetic as z
-// followed by the separate update, with z kept in a register.
+// Chebyshev (or damped) update d = ca z + cb d, x += d, in one pass (flags
+// SMOOTH_*: vectors that need not be read or written).  The same arithmetic as
+// z followed by the separate update, with z kept in a register.
 __global__ void
 k_aux_z_cheb(AuxGeom a, const double * __restrict__ dinv, const double * __restrict__ r,
              const double * __restrict__ t, double ca, double cb, double * __restrict__ d, double * __restrict__ x,
@@ -225,9 +225,12 @@ k_aux_z_cheb(AuxGeom a, const double * __restrict__ dinv, const double * __restr
          i += (int64_t)gridDim.x * blockDim.x)
     {
       const double z = dinv[i] * r[i] + aux_g<P>(a, tab, t, i);
-      const double di = (flags & 1) ? ca * z : ca * z + cb * d[i];
-      d[i] = di;
-      x[i] = (flags & 2) ? di : x[i] + di;
+      const double dold = (flags & SMOOTH_FRESH_D) ? 0.0 : d[i];
+      const double di = (flags & SMOOTH_FRESH_D) ? ca * z : ca * z + cb * dold;
+      if (!(flags & SMOOTH_NO_D))
+        d[i] = di;
+      if (!(flags & SMOOTH_NO_X))
+        x[i] = (flags & SMOOTH_FRESH_X) ? di : ((flags & SMOOTH_X_IS_D) ? dold : x[i]) + di;
     }
   });
 }

@@ -275,8 +275,12 @@ hipError_t grad_apply(const AuxGeom & a, const double * v, double * y, hipStream
 hipError_t grad_transpose(const AuxGeom & a, const double * w, double * yv, hipStream_t st);
 // z = D^-1 r + G Dg^-1 G^T r for one vector (t: node scratch, NN entries).
 // One step of the Chebyshev iteration with the hybrid smoother B = D^-1 + G Dg^-1 G^T:
-// t = Dg^-1 G^T r, then d = ca B r + cb d and x += d in one pass (flags 1:
-// fresh d; 2: fresh x, x = d).
+// t = Dg^-1 G^T r, then d = ca B r + cb d and x += d in one pass.
+constexpr int SMOOTH_FRESH_D = 1; // d is not read: d = ca B r
+constexpr int SMOOTH_FRESH_X = 2; // x is not read: x = d
+constexpr int SMOOTH_NO_D = 4;    // the new d is not stored
+constexpr int SMOOTH_NO_X = 8;    // x is neither read nor stored
+constexpr int SMOOTH_X_IS_D = 16; // x before the step is the old d (x is not read)
 hipError_t aux_smooth_step(const AuxGeom & a, const double * dinv, const double * ginv, const double * r, double * t,
                            double ca, double cb, double * d, double * x, int flags, hipStream_t st, int nrhs = 1,
                            int64_t sn = 0, int64_t snn = 0);

@@ -72,97 +72,141 @@ constexpr int DOT_THREADS = 256;
 // kernels
 // ---------------------------------------------------------------------------
 
-// One 1-D pass of a tensor-product transfer: out = scale * M (along axis) in,
-// + out when accumulate.  in: dims d[0..2] (x fastest); out: the same dims but
-// d[axis] -> m (the rows of M, CSR rp/ci/w).  Grid: x over the (i0, i1)
-// plane of the output, y over i2.
-__global__ void __launch_bounds__(256)
-k_pass1d(const double * __restrict__ in, double * __restrict__ out, int d0, int d1, int d2, int axis, int m,
-         const int * __restrict__ rp, const int * __restrict__ ci, const double * __restrict__ w, double scale,
-         int accumulate, int64_t sin, int64_t sout)
+// Local 1-D transfer matrices of a level pair: W[kind][row][k] = coarse basis
+// function k (of the open, kind 0, or closed, kind 1, points) at the point of
+// fine row `row` of the coarse element.  The same for every element and axis.
+constexpr int XFER_ROWS = 2 * PMAX;
+struct XferTab
 {
-  in += blockIdx.z * sin; // right-hand side blockIdx.z (strides 0 for one)
-  out += blockIdx.z * sout;
-  const unsigned o0 = axis == 0 ? m : d0, o1 = axis == 1 ? m : d1;
-  const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= o0 * o1)
-    return;
-  const int i1 = (int)(t / o0);
-  const int i0 = (int)(t - (unsigned)i1 * o0);
-  const int i2 = (int)blockIdx.y;
-  const int row = axis == 0 ? i0 : (axis == 1 ? i1 : i2);
-  // input offset of (j, i) along the axis: base + j * stride
-  const int64_t stride = axis == 0 ? 1 : (axis == 1 ? (int64_t)d0 : (int64_t)d0 * d1);
-  const int64_t base = ((int64_t)(axis == 2 ? 0 : i2) * d1 + (axis == 1 ? 0 : i1)) * d0 + (axis == 0 ? 0 : i0);
-  double s = 0.0;
-  for (int k = rp[row]; k < rp[row + 1]; k++)
-    s += w[k] * in[base + ci[k] * stride];
-  s *= scale;
-  const int64_t o = ((int64_t)i2 * o1 + i1) * o0 + i0;
-  out[o] = accumulate ? out[o] + s : s;
-}
+  double W[2][XFER_ROWS][PMAX + 1];
+};
 
-// The same pass for the three components of an ND transfer in one launch
-// (blockIdx.z = 3 rhs + component): each component has its own dims, 1-D
-// matrix, scale and input/output vectors; the per-entry arithmetic is that
-// of k_pass1d.
-struct Pass3
+// One 1-D pass of a tensor-product transfer along `axis`, for up to three
+// components in one launch (blockIdx.z = ncomp rhs + component).
+struct Xfer
 {
   const double * in[3];
   double * out[3];
-  int d[3][3]; // input dims per component
-  int m[3];    // rows of the component's 1-D matrix
-  const int * rp[3];
-  const int * ci[3];
-  const double * w[3];
+  int d[3][3];       // input dims per component (x fastest)
+  int closed[3];     // the component's points along the axis are closed
   double scale[3];
   int64_t sin, sout; // right-hand-side strides
-  int axis, accumulate;
-  int zero_pec; // PEC bits (HC_FACE_*) whose entries of the output are set to zero, or 0
+  int ncomp, axis, ne; // ne: coarse elements along the axis
+  int accumulate;
+  int zero_pec;      // PEC bits (HC_FACE_*) whose entries of the output are set to zero, or 0
+  XferTab t;
 };
 
+// A thread takes one coarse element of one line: the PC (+ 1) coarse and NR fine
+// values of the element are read once and every output of the element is
+// formed from registers (a fine row read by each of the outputs that need it,
+// through CSR, took 2-2.5 TB/s: 87 us for the last pass of a 48^3 order-3
+// prolongation).  Order of every sum: ascending input index.
+template <int NR, int PC, bool PROLONG>
 __global__ void __launch_bounds__(256)
-k_pass3(Pass3 q)
+k_xfer(Xfer q)
 {
-  const int comp = (int)(blockIdx.z % 3), rhs = (int)(blockIdx.z / 3);
-  const int axis = q.axis, m = q.m[comp];
+  const int comp = (int)(blockIdx.z % q.ncomp), rhs = (int)(blockIdx.z / q.ncomp);
+  const int axis = q.axis, ne = q.ne;
   const int d0 = q.d[comp][0], d1 = q.d[comp][1], d2 = q.d[comp][2];
-  const unsigned o0 = axis == 0 ? m : d0, o1 = axis == 1 ? m : d1, o2 = axis == 2 ? m : d2;
-  const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= o0 * o1 || blockIdx.y >= o2)
+  const unsigned w0 = axis == 0 ? ne : d0, w1 = axis == 1 ? ne : d1, w2 = axis == 2 ? ne : d2;
+  const unsigned t = blockIdx.x * 256 + threadIdx.x;
+  if (t >= w0 * w1 || blockIdx.y >= w2)
     return;
-  const double * __restrict__ in = q.in[comp] + rhs * q.sin;
-  double * __restrict__ out = q.out[comp] + rhs * q.sout;
-  const int * __restrict__ rp = q.rp[comp];
-  const int * __restrict__ ci = q.ci[comp];
-  const double * __restrict__ w = q.w[comp];
-  const int i1 = (int)(t / o0);
-  const int i0 = (int)(t - (unsigned)i1 * o0);
-  const int i2 = (int)blockIdx.y;
-  const int row = axis == 0 ? i0 : (axis == 1 ? i1 : i2);
-  const int64_t stride = axis == 0 ? 1 : (axis == 1 ? (int64_t)d0 : (int64_t)d0 * d1);
-  const int64_t base = ((int64_t)(axis == 2 ? 0 : i2) * d1 + (axis == 1 ? 0 : i1)) * d0 + (axis == 0 ? 0 : i0);
-  double s = 0.0;
-  for (int k = rp[row]; k < rp[row + 1]; k++)
-    s += w[k] * in[base + ci[k] * stride];
-  s *= q.scale[comp];
-  const int64_t o = ((int64_t)i2 * o1 + i1) * o0 + i0;
-  if (q.zero_pec)
-  {
-    // PEC entries of the output (a restriction's last pass): tangential DOFs
-    // on a PEC face of one of the component's closed axes
-    const int ii[3] = {i0, i1, i2};
-    const unsigned od[3] = {o0, o1, o2};
-    bool ess = false;
+  const int u1 = (int)(t / w0), u0 = (int)(t - (unsigned)u1 * w0), u2 = (int)blockIdx.y;
+  const int ec = axis == 0 ? u0 : (axis == 1 ? u1 : u2);
+  auto body = [&](auto cc) {
+    constexpr bool C = decltype(cc)::value;
+    constexpr int OUT = PROLONG ? NR : PC, KC = C ? PC + 1 : PC; // coarse points of an element
+    const int m = ne * OUT + (C ? 1 : 0);
+    const int e0 = axis == 0 ? m : d0, e1 = axis == 1 ? m : d1, e2 = axis == 2 ? m : d2;
+    const int64_t si = axis == 0 ? 1 : (axis == 1 ? (int64_t)d0 : (int64_t)d0 * d1);
+    const int64_t so = axis == 0 ? 1 : (axis == 1 ? (int64_t)e0 : (int64_t)e0 * e1);
+    const int64_t v0 = axis == 0 ? 0 : u0, v1 = axis == 1 ? 0 : u1, v2 = axis == 2 ? 0 : u2;
+    const double * __restrict__ in = q.in[comp] + rhs * q.sin + (v2 * d1 + v1) * d0 + v0;
+    double * __restrict__ out = q.out[comp] + rhs * q.sout + (v2 * e1 + v1) * e0 + v0;
+    const bool last = C && ec == ne - 1; // the thread of the last element also takes the end point
+    double r[OUT + 1];
 #pragma unroll
-    for (int b = 0; b < 3; b++)
-      if (b != comp)
-        ess = ess || (ii[b] == 0 && ((q.zero_pec >> (2 * b)) & 1)) ||
-              ((unsigned)ii[b] == od[b] - 1 && ((q.zero_pec >> (2 * b + 1)) & 1));
-    if (ess)
-      s = 0.0;
-  }
-  out[o] = q.accumulate ? out[o] + s : s;
+    for (int j = 0; j <= OUT; j++)
+      r[j] = 0.0;
+    if constexpr (PROLONG)
+    {
+      double v[PC + 1];
+#pragma unroll
+      for (int k = 0; k < KC; k++)
+        v[k] = in[((int64_t)ec * PC + k) * si];
+#pragma unroll
+      for (int j = 0; j < NR; j++)
+#pragma unroll
+        for (int k = 0; k < KC; k++)
+          r[j] += q.t.W[C][j][k] * v[k];
+      if constexpr (C)
+        r[NR] = v[PC];
+    }
+    else
+    {
+      double f[NR], l[NR];
+#pragma unroll
+      for (int j = 0; j < NR; j++)
+      {
+        f[j] = in[((int64_t)ec * NR + j) * si];
+        l[j] = (C && ec > 0) ? in[((int64_t)(ec - 1) * NR + j) * si] : 0.0;
+      }
+      // the closed point shared with the element before collects both
+      if constexpr (C)
+      {
+#pragma unroll
+        for (int j = 0; j < NR; j++)
+          r[0] += q.t.W[1][j][PC] * l[j];
+      }
+#pragma unroll
+      for (int k = 0; k < PC; k++)
+#pragma unroll
+        for (int j = 0; j < NR; j++)
+          r[k] += q.t.W[C][j][k] * f[j];
+      if (last)
+      {
+#pragma unroll
+        for (int j = 0; j < NR; j++)
+          r[PC] += q.t.W[1][j][PC] * f[j];
+        r[PC] += in[(int64_t)ne * NR * si];
+      }
+    }
+    const double scale = q.scale[comp];
+    double old[OUT + 1];
+#pragma unroll
+    for (int j = 0; j <= OUT; j++)
+      old[j] = (q.accumulate && (j < OUT || last)) ? out[((int64_t)ec * OUT + j) * so] : 0.0;
+#pragma unroll
+    for (int j = 0; j <= OUT; j++)
+    {
+      if (j == OUT && !last)
+        break;
+      double v = r[j] * scale;
+      if (q.zero_pec)
+      {
+        // PEC entries of the output (a restriction's last pass): tangential
+        // DOFs on a PEC face of one of the component's closed axes
+        const int o = ec * OUT + j;
+        const int ii[3] = {axis == 0 ? o : u0, axis == 1 ? o : u1, axis == 2 ? o : u2};
+        const int od[3] = {e0, e1, e2};
+        bool ess = false;
+#pragma unroll
+        for (int b = 0; b < 3; b++)
+          if (b != comp)
+            ess = ess || (ii[b] == 0 && ((q.zero_pec >> (2 * b)) & 1)) ||
+                  (ii[b] == od[b] - 1 && ((q.zero_pec >> (2 * b + 1)) & 1));
+        if (ess)
+          v = 0.0;
+      }
+      out[((int64_t)ec * OUT + j) * so] = old[j] + v;
+    }
+  };
+  if (q.closed[comp])
+    body(std::integral_constant<bool, true>{});
+  else
+    body(std::integral_constant<bool, false>{});
 }
 
 // Block partials of (a, b) and (a, a) (fixed grid and order).
@@ -186,15 +230,26 @@ k_dot2(const double * __restrict__ a, const double * __restrict__ b, int64_t n, 
   }
 }
 
-// x += alpha p; r -= alpha q (one pass)
-__global__ void
+// x += alpha p; r -= alpha q, and the block partials of (r, r) in the blocks and
+// order of k_dot2 (the first of each pair is zero): one pass instead of two
+__global__ void __launch_bounds__(DOT_THREADS)
 k_xr_update(int64_t n, double alpha, const double * __restrict__ p, const double * __restrict__ q,
-            double * __restrict__ x, double * __restrict__ r)
+            double * __restrict__ x, double * __restrict__ r, double * __restrict__ part)
 {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+  __shared__ double sh[DOT_THREADS];
+  double s = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * DOT_THREADS + threadIdx.x; i < n; i += (int64_t)DOT_BLOCKS * DOT_THREADS)
   {
     x[i] += alpha * p[i];
-    r[i] -= alpha * q[i];
+    const double ri = r[i] - alpha * q[i];
+    r[i] = ri;
+    s += ri * ri;
+  }
+  s = group_sum<DOT_THREADS>(s, sh);
+  if (threadIdx.x == 0)
+  {
+    part[2 * blockIdx.x] = 0.0;
+    part[2 * blockIdx.x + 1] = s;
   }
 }
 
@@ -349,76 +404,26 @@ points01(int n, bool lobatto, double * x)
   basis::gauss_legendre01(n, x, w);
 }
 
-struct Csr1
+// Local transfer matrices from coarse elements of order pc to their r (1 or 2)
+// fine elements per axis of order pf >= pc (the coarse field is in the fine
+// space: ND_pc on a mesh is contained in ND_pf on its refinement).
+XferTab
+xfer_tab(int pc, int pf, int r)
 {
-  std::vector<int> rp, ci;
-  std::vector<double> w;
-  int rows = 0, cols = 0;
-};
-
-// Prolongation of 1-D DOFs from nc coarse elements of order pc to nf = r nc
-// fine elements (r = 1 or 2) of order pf >= pc: open (p Gauss-Legendre points
-// per element) or closed (p+1 Gauss-Lobatto, shared at element ends).  Row =
-// fine DOF, entries = the coarse basis at its point (the coarse field is in
-// the fine space: ND_pc on a mesh is contained in ND_pf on its refinement).
-Csr1
-prolong_1d(int nc, int pc, int nf, int pf, bool closed)
-{
-  double gf[PMAX + 2], gc[PMAX + 2];
-  points01(closed ? pf + 1 : pf, closed, gf);
-  points01(closed ? pc + 1 : pc, closed, gc);
-  Csr1 m;
-  const int r = nf / nc;
-  const int kc = closed ? pc + 1 : pc; // coarse local nodes per element
-  m.rows = closed ? nf * pf + 1 : nf * pf;
-  m.cols = closed ? nc * pc + 1 : nc * pc;
-  m.rp.push_back(0);
-  for (int g = 0; g < m.rows; g++)
+  XferTab t{};
+  for (int kind = 0; kind < 2; kind++)
   {
-    const int ef = std::min(g / pf, nf - 1);
-    const int jf = g - ef * pf;
-    const int ec = ef / r, sub = ef % r;
-    const double t = (sub + gf[jf]) / r; // position in the coarse element
-    for (int jc = 0; jc < kc; jc++)
-    {
-      m.ci.push_back(ec * pc + jc);
-      m.w.push_back(lagrange1(kc, gc, jc, t));
-    }
-    m.rp.push_back((int)m.ci.size());
-  }
-  return m;
-}
-
-Csr1
-transpose(const Csr1 & a)
-{
-  Csr1 t;
-  t.rows = a.cols;
-  t.cols = a.rows;
-  std::vector<std::vector<std::pair<int, double>>> rows(t.rows);
-  for (int i = 0; i < a.rows; i++)
-    for (int k = a.rp[i]; k < a.rp[i + 1]; k++)
-      rows[a.ci[k]].push_back({i, a.w[k]}); // ascending fine index: a fixed summation order
-  t.rp.push_back(0);
-  for (auto & r : rows)
-  {
-    for (auto & e : r)
-    {
-      t.ci.push_back(e.first);
-      t.w.push_back(e.second);
-    }
-    t.rp.push_back((int)t.ci.size());
+    const bool closed = kind == 1;
+    double gf[PMAX + 2], gc[PMAX + 2];
+    points01(closed ? pf + 1 : pf, closed, gf);
+    points01(closed ? pc + 1 : pc, closed, gc);
+    const int kc = closed ? pc + 1 : pc;
+    for (int row = 0; row < r * pf; row++)
+      for (int k = 0; k < kc; k++)
+        t.W[kind][row][k] = lagrange1(kc, gc, k, (row / pf + gf[row % pf]) / r);
   }
   return t;
 }
-
-// device copy of a CSR 1-D matrix (carved out of a DevBlock)
-struct Csr1Dev
-{
-  const int *rp = nullptr, *ci = nullptr;
-  const double * w = nullptr;
-  int rows = 0, cols = 0;
-};
 
 } // namespace
 
@@ -433,8 +438,10 @@ struct MgLevel
   double omega = 1.0; // Richardson damping 1 / (1.05 lambda_max)
   double lam = 1.0;   // lambda_max(B A) estimate
   double cheb = 0.0;  // Chebyshev range lam_hi / lam_lo of the smoother (<= 1: Richardson)
-  // transfers to this level from the next coarser one: [axis][open=0/closed=1]
-  Csr1Dev P[3][2], R[3][2];
+  // transfers between this level and the next coarser one: local matrices,
+  // fine rows and coarse order per coarse element
+  XferTab xt{};
+  int xnr = 0, xpc = 0;
 };
 
 struct NodeHier;
@@ -505,13 +512,11 @@ comp_dims(const int n[3], int p, int c, int d[3])
     d[a] = (a == c) ? n[a] * p : n[a] * p + 1;
 }
 
+// sums of the block partials in h.part (synchronises)
 hipError_t
-dot2(MgHier & h, const double * a, const double * b, int64_t n, double & ab, double & aa, hipStream_t st)
+dot2_sums(MgHier & h, double & ab, double & aa, hipStream_t st)
 {
-  hipLaunchKernelGGL(k_dot2, dim3(DOT_BLOCKS), dim3(DOT_THREADS), 0, st, a, b, n, h.part);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess)
-    return e;
+  hipError_t e;
   if ((e = hipMemcpyAsync(h.hpart, h.part, sizeof(double) * 2 * DOT_BLOCKS, hipMemcpyDeviceToHost, st)) != hipSuccess)
     return e;
   if ((e = hipStreamSynchronize(st)) != hipSuccess)
@@ -523,6 +528,44 @@ dot2(MgHier & h, const double * a, const double * b, int64_t n, double & ab, dou
     aa += h.hpart[2 * i + 1];
   }
   return hipSuccess;
+}
+
+hipError_t
+dot2(MgHier & h, const double * a, const double * b, int64_t n, double & ab, double & aa, hipStream_t st)
+{
+  hipLaunchKernelGGL(k_dot2, dim3(DOT_BLOCKS), dim3(DOT_THREADS), 0, st, a, b, n, h.part);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? dot2_sums(h, ab, aa, st) : e;
+}
+
+hipError_t
+xfer_pass(const Xfer & q, int nr, int pc, bool prolong, int nrhs, hipStream_t st)
+{
+  int64_t plane = 0, o2 = 0;
+  for (int comp = 0; comp < q.ncomp; comp++)
+  {
+    plane = std::max(plane, (int64_t)(q.axis == 0 ? q.ne : q.d[comp][0]) * (q.axis == 1 ? q.ne : q.d[comp][1]));
+    o2 = std::max(o2, (int64_t)(q.axis == 2 ? q.ne : q.d[comp][2]));
+  }
+  const dim3 grid((unsigned)((plane + 255) / 256), (unsigned)o2, (unsigned)(q.ncomp * nrhs));
+  auto go = [&](auto kp, auto kr) {
+    if (prolong)
+      hipLaunchKernelGGL(kp, grid, dim3(256), 0, st, q);
+    else
+      hipLaunchKernelGGL(kr, grid, dim3(256), 0, st, q);
+  };
+  // halving of orders 1, 2, 3; orders 2 and 3 to 1 on the same mesh
+  if (nr == 2 && pc == 1)
+    go(k_xfer<2, 1, true>, k_xfer<2, 1, false>);
+  else if (nr == 4 && pc == 2)
+    go(k_xfer<4, 2, true>, k_xfer<4, 2, false>);
+  else if (nr == 6 && pc == 3)
+    go(k_xfer<6, 3, true>, k_xfer<6, 3, false>);
+  else if (nr == 3 && pc == 1)
+    go(k_xfer<3, 1, true>, k_xfer<3, 1, false>);
+  else
+    return hipErrorInvalidValue;
+  return hipGetLastError();
 }
 
 // y (level l) += P x (level l+1)   (prolong = true), or
@@ -568,49 +611,44 @@ transfer(MgHier & h, int l, bool prolong, const double * x, double * y, hipStrea
   // pass a over every component: x (src -> t1), y (t1 -> t2), z (t2 -> dst)
   for (int a = 0; a < 3; a++)
   {
-    Pass3 q{};
-    int64_t plane = 0, o2 = 0;
+    Xfer q{};
     for (int comp = 0; comp < 3; comp++)
     {
-      const int kind = (a == comp) ? 0 : 1;
-      const Csr1Dev & m = prolong ? f.P[a][kind] : f.R[a][kind];
+      q.closed[comp] = a != comp;
       q.in[comp] = (a == 0) ? src[comp] : (a == 1 ? t1[comp] : t2[comp]);
       q.out[comp] = (a == 2) ? dst[comp] : (a == 0 ? t1[comp] : t2[comp]);
-      for (int b = 0; b < 3; b++)
-        q.d[comp][b] = d[comp][b];
-      q.m[comp] = m.rows;
-      q.rp[comp] = m.rp;
-      q.ci[comp] = m.ci;
-      q.w[comp] = m.w;
       q.scale[comp] = a == 2 ? scale[comp] : 1.0;
-      plane = std::max(plane, (int64_t)(a == 0 ? m.rows : d[comp][0]) * (a == 1 ? m.rows : d[comp][1]));
-      o2 = std::max(o2, (int64_t)(a == 2 ? m.rows : d[comp][2]));
-      d[comp][a] = m.rows;
+      std::memcpy(q.d[comp], d[comp], sizeof(d[comp]));
+      d[comp][a] = c.n[a] * (prolong ? f.xnr : f.xpc) + q.closed[comp];
     }
+    q.ncomp = 3;
     q.axis = a;
+    q.ne = c.n[a];
     q.accumulate = (a == 2 && prolong) ? 1 : 0;
     q.zero_pec = (a == 2 && !prolong) ? c.op->g.pec : 0;
     q.sin = a == 0 ? sx : sT;
     q.sout = a == 2 ? sy : sT;
-    hipLaunchKernelGGL(k_pass3, dim3((unsigned)((plane + 255) / 256), (unsigned)o2, (unsigned)(3 * nrhs)), dim3(256),
-                       0, st, q);
-    hipError_t e = hipGetLastError();
+    q.t = f.xt;
+    hipError_t e = xfer_pass(q, f.xnr, f.xpc, prolong, nrhs, st);
     if (e != hipSuccess)
       return e;
   }
   return hipSuccess; // (a restriction's PEC entries are zeroed by its last pass)
 }
 
-// r = b - A x on level l (x == nullptr: r = b)
+// Flags of aux_smooth_step for smoothing step s: `first` the step from x = 0,
+// `xd` the one after it (x is in d), `final` the last.
 int
-residual(MgLevel & L, const double * b, const double * x, double * r, hipStream_t st)
+smooth_flags(int s, bool first, bool xd, bool final)
 {
-  if (!x)
-  {
-    HC_TRY_HIP(hipMemcpyAsync(r, b, sizeof(double) * L.N, hipMemcpyDeviceToDevice, st));
-    return HC_OK;
-  }
-  return op_residual(L.op, b, x, r, st);
+  int f = s == 0 ? SMOOTH_FRESH_D : 0;
+  if (first)
+    f |= final ? SMOOTH_FRESH_X : SMOOTH_NO_X;
+  if (xd)
+    f |= SMOOTH_X_IS_D;
+  if (final)
+    f |= SMOOTH_NO_D;
+  return f;
 }
 
 // h.nsmooth steps of the smoother on a level, from x = 0 when zero_start.
@@ -636,9 +674,14 @@ smooth(MgHier & h, MgLevel & L, bool zero_start, hipStream_t st, int steps = -1)
   }
   for (int s = 0; s < nsteps; s++)
   {
-    const bool first = zero_start && s == 0;
-    if (int rc = residual(L, L.b, first ? nullptr : L.x, L.r, st))
-      return rc;
+    const bool first = zero_start && s == 0, final = s == nsteps - 1;
+    // from zero the first residual is b itself, and the first step leaves x =
+    // d, stored once
+    const bool xd = zero_start && s == 1 && L.cheb > 1.0;
+    const double * r = first ? L.b : L.r;
+    if (!first)
+      if (int rc = op_residual(L.op, L.b, xd ? L.d : L.x, L.r, st))
+        return rc;
     if (L.cheb > 1.0)
     {
       double a, b;
@@ -657,12 +700,12 @@ smooth(MgHier & h, MgLevel & L, bool zero_start, hipStream_t st, int steps = -1)
       // z = B r and the update in one pass after the node stage
       if (int rc = L.op->ensure_ws(1, false))
         return rc;
-      HC_TRY_HIP(aux_smooth_step(L.op->ag, L.op->dinv64, L.op->ginv64, L.r, L.op->ws.t64, a, b, L.d, L.x,
-                                 (s == 0 ? 1 : 0) | (first ? 2 : 0), st));
+      HC_TRY_HIP(aux_smooth_step(L.op->ag, L.op->dinv64, L.op->ginv64, r, L.op->ws.t64, a, b, L.d, L.x,
+                                 smooth_flags(s, first, xd, final), st));
     }
     else
     {
-      if (int rc = hc_op_precond_apply(L.op, HC_SOLVE_FP64 | HC_SOLVE_AUX, L.r, L.z, st))
+      if (int rc = hc_op_precond_apply(L.op, HC_SOLVE_FP64 | HC_SOLVE_AUX, r, L.z, st))
         return rc;
       HC_TRY_HIP(axpby(L.N, L.omega, L.z, first ? 0.0 : 1.0, L.x, st));
     }
@@ -687,7 +730,7 @@ vcycle(MgHier & h, int l, hipStream_t st)
   }
   if (int rc = smooth(h, L, true, st)) // pre-smoothing from x = 0
     return rc;
-  if (int rc = residual(L, L.b, L.x, L.r, st))
+  if (int rc = op_residual(L.op, L.b, L.x, L.r, st))
     return rc;
   HC_TRY_HIP(transfer(h, l, false, L.r, h.lev[l + 1].b, st));
   if (int rc = vcycle(h, l + 1, st))
@@ -882,11 +925,13 @@ smooth_k(MgHier & h, MgMulti & mm, int l, bool zero_start, int k, hipStream_t st
   }
   for (int s = 0; s < nsteps; s++)
   {
-    const bool first = zero_start && s == 0;
-    if (first)
-      HC_TRY_HIP(hipMemcpyAsync(r, b, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
-    else if (int rc = op_residual(L.op, b, x, r, st, k))
-      return rc;
+    // as in smooth()
+    const bool first = zero_start && s == 0, final = s == nsteps - 1;
+    const bool xd = zero_start && s == 1 && L.cheb > 1.0;
+    double * rs = first ? b : r;
+    if (!first)
+      if (int rc = op_residual(L.op, b, xd ? d : x, r, st, k))
+        return rc;
     if (L.cheb > 1.0)
     {
       double a, bb;
@@ -903,12 +948,12 @@ smooth_k(MgHier & h, MgMulti & mm, int l, bool zero_start, int k, hipStream_t st
         rho0 = rho1;
       }
       // z = B r and the update in one pass after the node stage
-      HC_TRY_HIP(aux_smooth_step(L.op->ag, L.op->dinv64, L.op->ginv64, r, L.op->ws.t64, a, bb, d, x,
-                                 (s == 0 ? 1 : 0) | (first ? 2 : 0), st, k, L.N, L.op->ws.NNC));
+      HC_TRY_HIP(aux_smooth_step(L.op->ag, L.op->dinv64, L.op->ginv64, rs, L.op->ws.t64, a, bb, d, x,
+                                 smooth_flags(s, first, xd, final), st, k, L.N, L.op->ws.NNC));
     }
     else
     {
-      HC_TRY_HIP(aux_precond_apply(L.op->ag, L.op->dinv64, L.op->ginv64, r, L.op->ws.t64, z, st, k, L.N,
+      HC_TRY_HIP(aux_precond_apply(L.op->ag, L.op->dinv64, L.op->ginv64, rs, L.op->ws.t64, z, st, k, L.N,
                                    L.op->ws.NNC));
       HC_TRY_HIP(axpby(n, L.omega, z, first ? 0.0 : 1.0, x, st));
     }
@@ -938,32 +983,6 @@ vcycle_k(MgHier & h, MgMulti & mm, int l, int k, hipStream_t st)
     return rc;
   HC_TRY_HIP(transfer(h, l, true, mm.x[l + 1], mm.x[l], st, k, mm.tmp1, mm.tmp2));
   return smooth_k(h, mm, l, false, k, st);
-}
-
-Csr1Dev
-upload(const Csr1 & m, char *& p)
-{
-  Csr1Dev d;
-  d.rows = m.rows;
-  d.cols = m.cols;
-  const size_t a = align256(sizeof(int) * m.rp.size()), b = align256(sizeof(int) * m.ci.size());
-  (void)hipMemcpy(p, m.rp.data(), sizeof(int) * m.rp.size(), hipMemcpyHostToDevice);
-  d.rp = (const int *)p;
-  p += a;
-  (void)hipMemcpy(p, m.ci.data(), sizeof(int) * m.ci.size(), hipMemcpyHostToDevice);
-  d.ci = (const int *)p;
-  p += b;
-  (void)hipMemcpy(p, m.w.data(), sizeof(double) * m.w.size(), hipMemcpyHostToDevice);
-  d.w = (const double *)p;
-  p += align256(sizeof(double) * m.w.size());
-  return d;
-}
-
-size_t
-csr_bytes(const Csr1 & m)
-{
-  return align256(sizeof(int) * m.rp.size()) + align256(sizeof(int) * m.ci.size()) +
-         align256(sizeof(double) * m.w.size());
 }
 
 // lambda_max of B A on a level by power iteration (from a seeded vector)
@@ -1120,18 +1139,16 @@ mg_build(hc_op_t op, hipStream_t st)
                                " DOFs and the mesh cannot be coarsened (odd element counts at order 1; at most " +
                                std::to_string(MG_COARSE_MAX) + " DOFs for a single level)");
   // transfer matrices
-  std::vector<Csr1> mats; // per level pair: [axis][kind] P then R
   size_t bytes = 0;
   for (int l = 0; l + 1 < nl; l++)
-    for (int a = 0; a < 3; a++)
-      for (int kind = 0; kind < 2; kind++)
-      {
-        Csr1 P = prolong_1d(h->lev[l + 1].n[a], h->lev[l + 1].op->p, h->lev[l].n[a], h->lev[l].op->p, kind == 1);
-        Csr1 R = transpose(P);
-        bytes += csr_bytes(P) + csr_bytes(R);
-        mats.push_back(std::move(P));
-        mats.push_back(std::move(R));
-      }
+  {
+    MgLevel & f = h->lev[l];
+    const MgLevel & c = h->lev[l + 1];
+    const int r = f.n[0] / c.n[0];
+    f.xpc = c.op->p;
+    f.xnr = r * f.op->p;
+    f.xt = xfer_tab(f.xpc, f.op->p, r);
+  }
   // vectors: x, b, r, z per level; two temporaries of the finest size; dot partials
   for (auto & L : h->lev)
     bytes += 5 * align256(sizeof(double) * L.N);
@@ -1139,14 +1156,6 @@ mg_build(hc_op_t op, hipStream_t st)
   if (int rc = h->mem.alloc(bytes))
     return rc;
   char * q = (char *)h->mem.base;
-  size_t mi = 0;
-  for (int l = 0; l + 1 < nl; l++)
-    for (int a = 0; a < 3; a++)
-      for (int kind = 0; kind < 2; kind++)
-      {
-        h->lev[l].P[a][kind] = upload(mats[mi++], q);
-        h->lev[l].R[a][kind] = upload(mats[mi++], q);
-      }
   for (auto & L : h->lev)
   {
     double ** v[5] = {&L.x, &L.b, &L.r, &L.z, &L.d};
@@ -1274,9 +1283,8 @@ mg_pcg_solve(hc_op_t op, const double * b, double * x, double rtol, int maxit, h
   for (outer = 1; outer <= 1 + MAX_RESTARTS && !conv && status == HC_OK; outer++)
   {
     // r = b - A x
-    if (int rc = hc_op_apply(op, x, r, 1, st))
+    if (int rc = op_residual(op, b, x, r, st))
       return rc;
-    HC_TRY_HIP(axpby(N, 1.0, b, -1.0, r, st));
     HC_TRY_HIP(dot2(h, r, r, N, dummy, rr, st));
     if (rr <= tol2)
     {
@@ -1301,10 +1309,10 @@ mg_pcg_solve(hc_op_t op, const double * b, double * x, double rtol, int maxit, h
         break;
       }
       const double alpha = gam / pq;
-      hipLaunchKernelGGL(k_xr_update, dim3(grid_for(N)), dim3(256), 0, st, N, alpha, pv, q, x, r);
+      hipLaunchKernelGGL(k_xr_update, dim3(DOT_BLOCKS), dim3(DOT_THREADS), 0, st, N, alpha, pv, q, x, r, h.part);
       HC_TRY_HIP(hipGetLastError());
       iters++;
-      HC_TRY_HIP(dot2(h, r, r, N, dummy, rr, st));
+      HC_TRY_HIP(dot2_sums(h, dummy, rr, st));
       if (rr <= tol2)
         break;
       if (int rc = precond(r, zz))
@@ -1318,9 +1326,8 @@ mg_pcg_solve(hc_op_t op, const double * b, double * x, double rtol, int maxit, h
     if (status != HC_OK)
       break;
     // true residual of the result
-    if (int rc = hc_op_apply(op, x, r, 1, st))
+    if (int rc = op_residual(op, b, x, r, st))
       return rc;
-    HC_TRY_HIP(axpby(N, 1.0, b, -1.0, r, st));
     HC_TRY_HIP(dot2(h, r, r, N, dummy, rr, st));
     conv = rr <= tol2;
     if (iters >= maxit)
@@ -1402,9 +1409,8 @@ mg_pcg_solve_multi(hc_op_t op, const double * B, double * X, int k, double rtol,
     return hipMemcpyAsync(mm.coef, mm.hcoef, sizeof(double) * k, hipMemcpyHostToDevice, st);
   };
   auto resid = [&]() -> int {
-    if (int rc = hc_op_apply(op, X, R, k, st))
+    if (int rc = op_residual(op, B, X, R, st, k))
       return rc;
-    HC_TRY_HIP(axpby(n, 1.0, B, -1.0, R, st));
     HC_TRY_HIP(dot2_k(mm, R, R, N, k, dummy, rr, st));
     return HC_OK;
   };
@@ -1543,7 +1549,6 @@ struct NodeLevel
   double *x = nullptr, *b = nullptr, *r = nullptr, *z = nullptr, *d = nullptr, *dinv = nullptr;
   double *t1 = nullptr, *t2 = nullptr; // ND-size temporaries of the S apply
   double lam = 1.0;
-  Csr1Dev P[3], R[3]; // from the next coarser level, per axis
 };
 
 struct NodeHier
@@ -1604,23 +1609,28 @@ node_transfer(MgHier & h, NodeHier & nh, int l, bool prolong, const double * x, 
 {
   const NodeLevel & f = nh.lev[l];
   const NodeLevel & c = nh.lev[l + 1];
+  const MgLevel & fl = h.lev[l];
+  const MgLevel & cl = h.lev[l + 1];
   int d[3];
   for (int a = 0; a < 3; a++)
     d[a] = prolong ? c.op->ag.M[a] : f.op->ag.M[a];
   for (int a = 0; a < 3; a++)
   {
-    const Csr1Dev & m = prolong ? f.P[a] : f.R[a];
-    double * out = (a == 2) ? y : (a == 0 ? h.tmp1 : h.tmp2);
-    const double * in = (a == 0) ? x : (a == 1 ? h.tmp1 : h.tmp2);
-    const int64_t plane = (int64_t)(a == 0 ? m.rows : d[0]) * (a == 1 ? m.rows : d[1]);
-    const int o2 = a == 2 ? m.rows : d[2];
-    hipLaunchKernelGGL(k_pass1d, dim3((unsigned)((plane + 255) / 256), (unsigned)o2), dim3(256), 0, st, in, out, d[0],
-                       d[1], d[2], a, m.rows, m.rp, m.ci, m.w, 1.0, (a == 2 && prolong) ? 1 : 0, (int64_t)0,
-                       (int64_t)0);
-    hipError_t e = hipGetLastError();
+    Xfer q{};
+    q.closed[0] = 1;
+    q.out[0] = (a == 2) ? y : (a == 0 ? h.tmp1 : h.tmp2);
+    q.in[0] = (a == 0) ? x : (a == 1 ? h.tmp1 : h.tmp2);
+    q.scale[0] = 1.0;
+    std::memcpy(q.d[0], d, sizeof(d));
+    q.ncomp = 1;
+    q.axis = a;
+    q.ne = cl.n[a];
+    q.accumulate = (a == 2 && prolong) ? 1 : 0;
+    q.t = fl.xt;
+    hipError_t e = xfer_pass(q, fl.xnr, fl.xpc, prolong, 1, st);
     if (e != hipSuccess)
       return e;
-    d[a] = m.rows;
+    d[a] = cl.n[a] * (prolong ? fl.xnr : fl.xpc) + 1;
   }
   return hipSuccess;
 }
@@ -1700,7 +1710,6 @@ node_build(MgHier & h, hipStream_t st)
   auto * nh = new NodeHier();
   std::unique_ptr<NodeHier> guard(nh);
   size_t bytes = 0;
-  std::vector<Csr1> mats;
   for (int l = 0; l < nl; l++)
   {
     NodeLevel L;
@@ -1714,27 +1723,9 @@ node_build(MgHier & h, hipStream_t st)
     nh->lev.push_back(L);
     bytes += 6 * align256(sizeof(double) * L.NN) + 2 * align256(sizeof(double) * L.N);
   }
-  for (int l = 0; l + 1 < nl; l++)
-    for (int a = 0; a < 3; a++)
-    {
-      const MgLevel & f = h.lev[l];
-      const MgLevel & c = h.lev[l + 1];
-      Csr1 P = prolong_1d(c.n[a], c.op->p, f.n[a], f.op->p, true);
-      Csr1 R = transpose(P);
-      bytes += csr_bytes(P) + csr_bytes(R);
-      mats.push_back(std::move(P));
-      mats.push_back(std::move(R));
-    }
   if (int rc = nh->mem.alloc(bytes))
     return rc;
   char * q = (char *)nh->mem.base;
-  size_t mi = 0;
-  for (int l = 0; l + 1 < nl; l++)
-    for (int a = 0; a < 3; a++)
-    {
-      nh->lev[l].P[a] = upload(mats[mi++], q);
-      nh->lev[l].R[a] = upload(mats[mi++], q);
-    }
   for (auto & L : nh->lev)
   {
     double ** v[6] = {&L.x, &L.b, &L.r, &L.z, &L.d, &L.dinv};
