@@ -31,7 +31,11 @@ make_aux_geom(const Geom & g, const double * dg1d)
     a.dg[i] = dg1d[i];
   for (int c = 0; c < 3; c++)
     for (int d = 0; d < 2; d++)
+    {
       a.rcd[c][d] = 1.0 / (double)a.cd[c][d];
+      a.ed[c][d] = (d == c) ? a.n[d] : a.cd[c][d];
+      a.red[c][d] = 1.0 / (double)a.ed[c][d];
+    }
   return a;
 }
 
@@ -172,7 +176,7 @@ term_ratio_blocks(const double * qd, int64_t E, int p, double * out, hipStream_t
 }
 
 // Standalone z = B r: t = Dg^-1 G^T r at the nodes, then z = D^-1 r + G t.
-__global__ void
+__global__ void __launch_bounds__(256)
 k_aux_nodes_single(AuxGeom a, const double * __restrict__ ginv, const double * __restrict__ r,
                    double * __restrict__ t, int64_t sr, int64_t st_)
 {
@@ -181,15 +185,15 @@ k_aux_nodes_single(AuxGeom a, const double * __restrict__ ginv, const double * _
   with_order(a, [&](auto pc) {
     constexpr int P = decltype(pc)::value;
     const DgTab<P> tab = load_dg<P>(a);
-    const int S = gridDim.x * blockDim.x;
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
+    const int S = gridDim.x * 256;
+    int k = blockIdx.x * 256 + threadIdx.x;
     NodeWalk nw(a, k, S);
     for (; k < a.NN; k += S, nw.step(a))
       t[k] = ginv[k] * aux_gt<P>(a, tab, r, nw.I, nw.J, nw.K);
   });
 }
 
-__global__ void
+__global__ void __launch_bounds__(256)
 k_aux_z_single(AuxGeom a, const double * __restrict__ dinv, const double * __restrict__ r,
                const double * __restrict__ t, double * __restrict__ z, int64_t sr, int64_t st_)
 {
@@ -199,9 +203,8 @@ k_aux_z_single(AuxGeom a, const double * __restrict__ dinv, const double * __res
   with_order(a, [&](auto pc) {
     constexpr int P = decltype(pc)::value;
     const DgTab<P> tab = load_dg<P>(a);
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.off[3];
-         i += (int64_t)gridDim.x * blockDim.x)
-      z[i] = dinv[i] * r[i] + aux_g<P>(a, tab, t, i);
+    for (int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x; k < a.off[3] / P; k += (int64_t)gridDim.x * 256)
+      aux_g_edge<P>(a, tab, t, k, [&](int64_t i, double g) { z[i] = dinv[i] * r[i] + g; });
   });
 }
 
@@ -209,7 +212,7 @@ k_aux_z_single(AuxGeom a, const double * __restrict__ dinv, const double * __res
 // Chebyshev (or damped) update d = ca z + cb d, x += d, in one pass (flags
 // SMOOTH_*: vectors that need not be read or written).  The same arithmetic as
 // z followed by the separate update, with z kept in a register.
-__global__ void
+__global__ void __launch_bounds__(256)
 k_aux_z_cheb(AuxGeom a, const double * __restrict__ dinv, const double * __restrict__ r,
              const double * __restrict__ t, double ca, double cb, double * __restrict__ d, double * __restrict__ x,
              int flags, int64_t sr, int64_t st_)
@@ -221,17 +224,16 @@ k_aux_z_cheb(AuxGeom a, const double * __restrict__ dinv, const double * __restr
   with_order(a, [&](auto pc) {
     constexpr int P = decltype(pc)::value;
     const DgTab<P> tab = load_dg<P>(a);
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.off[3];
-         i += (int64_t)gridDim.x * blockDim.x)
-    {
-      const double z = dinv[i] * r[i] + aux_g<P>(a, tab, t, i);
-      const double dold = (flags & SMOOTH_FRESH_D) ? 0.0 : d[i];
-      const double di = (flags & SMOOTH_FRESH_D) ? ca * z : ca * z + cb * dold;
-      if (!(flags & SMOOTH_NO_D))
-        d[i] = di;
-      if (!(flags & SMOOTH_NO_X))
-        x[i] = (flags & SMOOTH_FRESH_X) ? di : ((flags & SMOOTH_X_IS_D) ? dold : x[i]) + di;
-    }
+    for (int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x; k < a.off[3] / P; k += (int64_t)gridDim.x * 256)
+      aux_g_edge<P>(a, tab, t, k, [&](int64_t i, double g) {
+        const double z = dinv[i] * r[i] + g;
+        const double dold = (flags & SMOOTH_FRESH_D) ? 0.0 : d[i];
+        const double di = (flags & SMOOTH_FRESH_D) ? ca * z : ca * z + cb * dold;
+        if (!(flags & SMOOTH_NO_D))
+          d[i] = di;
+        if (!(flags & SMOOTH_NO_X))
+          x[i] = (flags & SMOOTH_FRESH_X) ? di : ((flags & SMOOTH_X_IS_D) ? dold : x[i]) + di;
+      });
   });
 }
 
@@ -274,75 +276,33 @@ aux_precond_apply(const AuxGeom & a, const double * dinv, const double * ginv, c
 // M G is exact (G maps into the ND space) and K G = 0, so the mixed and
 // diffusion blocks are M G and G^T M G.
 // ---------------------------------------------------------------------------
-// Row segments of the ND DOFs: one work item per element edge along a
-// component's open axis (the p DOFs that share the p + 1 nodes of that edge),
-// items of a component in the memory order of its DOFs with the open axis
-// counted in elements.
-struct RowItems
-{
-  int64_t ioff[4]; // first item of each component, ioff[3] = N / p
-  int dim[3][2];   // items along the first two axes of each component
-  double rd[3][2]; // their reciprocals (fast_divmod)
-};
-
-static RowItems
-row_items(const AuxGeom & a)
-{
-  RowItems ri{};
-  for (int c = 0; c < 4; c++)
-    ri.ioff[c] = a.off[c] / a.p;
-  for (int c = 0; c < 3; c++)
-    for (int d = 0; d < 2; d++)
-    {
-      ri.dim[c][d] = (d == c) ? a.n[d] : a.cd[c][d];
-      ri.rd[c][d] = 1.0 / (double)ri.dim[c][d];
-    }
-  return ri;
-}
-
-// s = a0 + G v (ADD_A, a0 = a with its PEC DOFs zeroed) or s = G v, one row
-// segment per item: the p + 1 node values of the edge are loaded once for
-// its p DOFs; each DOF sums its p + 1 terms in node order, as aux_g_at does.
+// s = a0 + G v (ADD_A, a0 = a with its PEC DOFs zeroed) or s = G v, one element
+// edge per work item.
 template <bool ADD_A>
-__global__ void
-k_g_rows(Geom g, AuxGeom a, RowItems ri, const double * __restrict__ av, const double * __restrict__ v,
-         double * __restrict__ s)
+__global__ void __launch_bounds__(256)
+k_g_rows(int pec, AuxGeom a, const double * __restrict__ av, const double * __restrict__ v, double * __restrict__ s)
 {
   with_order(a, [&](auto pc) {
     constexpr int P = decltype(pc)::value;
     const DgTab<P> tab = load_dg<P>(a);
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < ri.ioff[3];
-         t += (int64_t)gridDim.x * blockDim.x)
+    for (int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x; k < a.off[3] / P; k += (int64_t)gridDim.x * 256)
     {
-      const int c = (t < ri.ioff[1]) ? 0 : ((t < ri.ioff[2]) ? 1 : 2);
-      int i[3], rest;
-      fast_divmod((int)(t - ri.ioff[c]), ri.dim[c][0], ri.rd[c][0], rest, i[0]);
-      fast_divmod(rest, ri.dim[c][1], ri.rd[c][1], i[2], i[1]);
-      i[c] *= P; // first DOF of the edge, and its first node along c
-      const int64_t d0 = a.off[c] + ((int64_t)i[2] * a.cd[c][1] + i[1]) * a.cd[c][0] + i[0];
-      const int64_t dstride = (c == 0) ? 1 : ((c == 1) ? (int64_t)a.cd[1][0] : (int64_t)a.cd[2][0] * a.cd[2][1]);
-      const int64_t nstride = (c == 0) ? 1 : ((c == 1) ? (int64_t)a.M[0] : (int64_t)a.M[0] * a.M[1]);
-      const double * tl = v + ((int64_t)i[2] * a.M[1] + i[1]) * a.M[0] + i[0];
-      double nv[P + 1];
-#pragma unroll
-      for (int m = 0; m <= P; m++)
-        nv[m] = tl[m * nstride];
-      const bool ess = ADD_A && is_ess(g, c, i[0], i[1], i[2]); // the same for the edge's DOFs
-#pragma unroll
-      for (int l = 0; l < P; l++)
-      {
-        double gv = 0.0;
-#pragma unroll
-        for (int m = 0; m <= P; m++)
-          gv += tab.d[l][m] * nv[m];
+      bool first = true, ess = false;
+      aux_g_edge<P>(a, tab, v, k, [&](int64_t i, double g) {
         if constexpr (ADD_A)
         {
-          const double a0 = ess ? 0.0 : av[d0 + l * dstride];
-          s[d0 + l * dstride] = a0 + gv;
+          if (first) // the same for the edge's DOFs
+          {
+            int c, i0, i1, i2;
+            aux_dof_coords(a, i, c, i0, i1, i2);
+            ess = aux_ess(a, pec, c, i0, i1, i2);
+            first = false;
+          }
+          s[i] = (ess ? 0.0 : av[i]) + g;
         }
         else
-          s[d0 + l * dstride] = gv;
-      }
+          s[i] = g;
+      });
     }
   });
 }
@@ -359,14 +319,14 @@ k_av_finish(Geom g, AuxGeom a, const double * __restrict__ av, const double * __
   }
 }
 
-__global__ void
+__global__ void __launch_bounds__(256)
 k_grad_transpose(AuxGeom a, const double * __restrict__ w, double * __restrict__ yv)
 {
   with_order(a, [&](auto pc) {
     constexpr int P = decltype(pc)::value;
     const DgTab<P> tab = load_dg<P>(a);
-    const int S = gridDim.x * blockDim.x;
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
+    const int S = gridDim.x * 256;
+    int k = blockIdx.x * 256 + threadIdx.x;
     NodeWalk nw(a, k, S);
     for (; k < a.NN; k += S, nw.step(a))
       yv[k] = aux_gt<P>(a, tab, w, nw.I, nw.J, nw.K);
@@ -376,15 +336,14 @@ k_grad_transpose(AuxGeom a, const double * __restrict__ w, double * __restrict__
 hipError_t
 grad_apply(const AuxGeom & a, const double * v, double * y, hipStream_t st)
 {
-  Geom g{}; // unused without ADD_A
-  hipLaunchKernelGGL(k_g_rows<false>, dim3(4096), dim3(256), 0, st, g, a, row_items(a), nullptr, v, y);
+  hipLaunchKernelGGL(k_g_rows<false>, dim3(4096), dim3(256), 0, st, 0, a, nullptr, v, y);
   return hipGetLastError();
 }
 
 hipError_t
 av_gather(const Geom & g, const AuxGeom & a, const double * av, const double * v, double * s, hipStream_t st)
 {
-  hipLaunchKernelGGL(k_g_rows<true>, dim3(4096), dim3(256), 0, st, g, a, row_items(a), av, v, s);
+  hipLaunchKernelGGL(k_g_rows<true>, dim3(4096), dim3(256), 0, st, g.pec, a, av, v, s);
   return hipGetLastError();
 }
 

@@ -325,8 +325,8 @@ k_pcg_update_p(SlotTable t, const int * __restrict__ git)
     with_order(sl.ag, [&](auto pc) {
       constexpr int P = decltype(pc)::value;
       const DgTab<P> tab = load_dg<P>(sl.ag);
-      HC_SLOT_LOOP(i, sl.n, nb)
-      p[i] = (dinv[i] * r[i] + (T)aux_g<P>(sl.ag, tab, tv, i)) + beta * p[i];
+      HC_SLOT_LOOP(k, sl.n / P, nb)
+      aux_g_edge<P>(sl.ag, tab, tv, k, [&](int64_t i, double g) { p[i] = (dinv[i] * r[i] + (T)g) + beta * p[i]; });
     });
   }
   else
@@ -407,8 +407,8 @@ k_aux_pset(SlotTable t, int which)
   with_order(sl.ag, [&](auto pc) {
     constexpr int P = decltype(pc)::value;
     const DgTab<P> tab = load_dg<P>(sl.ag);
-    HC_SLOT_LOOP(i, sl.n, nb)
-    p[i] = dinv[i] * r[i] + (T)aux_g<P>(sl.ag, tab, tv, i);
+    HC_SLOT_LOOP(k, sl.n / P, nb)
+    aux_g_edge<P>(sl.ag, tab, tv, k, [&](int64_t i, double g) { p[i] = dinv[i] * r[i] + (T)g; });
   });
 }
 
