@@ -1087,11 +1087,9 @@ template hipError_t apply_op<float>(const Geom &, const PlaneSegs &, const Table
 template <typename T>
 hipError_t
 apply_multi(const TileCandidate * cand, const Tables<T> & tb, const ApplyDesc * descs_dev, int ndesc, int nwork,
-            int npwork, int grouped, int box_ns, hipStream_t st)
+            int npwork, int grouped, hipStream_t st)
 {
   ApplyDesc dummy{};
-  if (box_ns)
-    return apply_box<T>(dummy, descs_dev, ndesc, nwork, cand->p, box_ns, st);
   hipError_t e = cand->launch(dummy, descs_dev, ndesc, nwork, grouped, &tb, sizeof(T) == 8 ? 64 : 32, st);
   if (e != hipSuccess)
     return e;
@@ -1099,8 +1097,8 @@ apply_multi(const TileCandidate * cand, const Tables<T> & tb, const ApplyDesc * 
 }
 
 template hipError_t apply_multi<double>(const TileCandidate *, const Tables<double> &, const ApplyDesc *, int, int, int,
-                                        int, int, hipStream_t);
+                                        int, hipStream_t);
 template hipError_t apply_multi<float>(const TileCandidate *, const Tables<float> &, const ApplyDesc *, int, int, int, int,
-                                       int, hipStream_t);
+                                       hipStream_t);
 
 } // namespace hc

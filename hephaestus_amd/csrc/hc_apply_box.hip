@@ -103,27 +103,25 @@ stb(T * base, uint32_t off, T v, uint32_t sof = 0)
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rsrc(base), (int)off, (int)sof, 0);
 }
 
+// LDS of the apply in doubles: 4 face arrays of 2 buffers and P planes, and the
+// PEC values
+template <int P, int NS>
+constexpr int
+box_lds()
+{
+  return 8 * P * (NS * (P == 1 ? 8 : 4) + 1) + (3 * P + 2) * 16 * NS;
+}
+
+// The right-hand sides [r_begin, r_end) of tile `tile` of one instance.
 template <int P, typename T, int NS, bool TABLE, bool RES>
-__global__ void __launch_bounds__(16 * NS, 4)
-k_apply_box(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc)
+__device__ __forceinline__ void
+box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
 {
 #pragma clang fp contract(off)
   constexpr basis::BoxTab<P> tb = basis::box_tab<P>();
   constexpr int EJ = (P == 1) ? 2 : 1; // elements per axis in a 16-lane block
   constexpr int FS = 4 * EJ;           // face values per block, plane and array
   constexpr uint32_t SZ = sizeof(T);
-
-  const int wi = xcd_remap(blockIdx.x, gridDim.x);
-  int di = 0;
-  if constexpr (TABLE)
-    di = __builtin_amdgcn_readfirstlane(find_instance(wi, ndesc, [&](int i) { return descs[i].w0; }));
-  const ApplyDesc & ad = TABLE ? descs[di] : d0;
-  const int rb = TABLE ? ad.rb : 1;
-  const int ngrp = (ad.nrhs + rb - 1) / rb;
-  const int wl = wi - ad.w0;
-  const int r_begin = (wl % ngrp) * rb;
-  const int r_end = TABLE ? min(ad.nrhs, r_begin + rb) : r_begin + 1;
-  int tile = wl / ngrp;
   const Geom & g = ad.g;
   const int bcx = ad.bt.cx, bcy = ad.bt.cy;
   const int tx = tile % ad.bt.ntx;
@@ -132,7 +130,8 @@ k_apply_box(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc)
 
   // face values; entry NS * FS is the zero that lanes without a neighbour add
   constexpr int FZ = NS * FS;
-  __shared__ double sX[2][P][FZ + 1], sY[2][P][FZ + 1], sZR[2][P][FZ + 1], sZC[2][P][FZ + 1];
+  using Face = double[P][FZ + 1];
+  Face * const sX = (Face *)lds, * const sY = sX + 2, * const sZR = sX + 4, * const sZC = sX + 6;
   if (threadIdx.x < 2 * P)
   {
     const int b = threadIdx.x / P, k = threadIdx.x % P;
@@ -174,7 +173,8 @@ k_apply_box(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc)
   // 1 .. p-1 of x and y and p planes of z of the layer, and the lowest plane of
   // x and y of the layer (by parity of z: the one above is known a layer early)
   const bool wave_ess = __any((vN && essz) || (vT && essyT)) != 0;
-  __shared__ double sE[3 * P + 2][16 * NS];
+  using PecRow = double[16 * NS];
+  PecRow * const sE = (PecRow *)(sX + 8);
   constexpr int EX = 0, EY = P - 1, EZ = 2 * P - 2, EX0 = 3 * P - 2, EY0 = 3 * P;
   const int eN = threadIdx.x, eT = (threadIdx.x & ~51) | (lf << 4) | ls;
   // byte offsets inside a plane of each component, from the tile's first row
@@ -551,6 +551,37 @@ k_apply_box(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc)
   }
 }
 
+// P = 0: the instances of the table may have any order (one launch, and the
+// small instances of one order run beside the large ones of another)
+template <int P, typename T, int NS, bool TABLE, bool RES>
+__global__ void __launch_bounds__(16 * NS, 4)
+k_apply_box(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc)
+{
+  __shared__ double lds[box_lds<P == 0 ? PMAX : P, NS>()];
+  const int wi = xcd_remap(blockIdx.x, gridDim.x);
+  int di = 0;
+  if constexpr (TABLE)
+    di = __builtin_amdgcn_readfirstlane(find_instance(wi, ndesc, [&](int i) { return descs[i].w0; }));
+  const ApplyDesc & ad = TABLE ? descs[di] : d0;
+  const int rb = TABLE ? ad.rb : 1;
+  const int ngrp = (ad.nrhs + rb - 1) / rb;
+  const int wl = wi - ad.w0;
+  const int r_begin = (wl % ngrp) * rb;
+  const int r_end = TABLE ? min(ad.nrhs, r_begin + rb) : r_begin + 1;
+  const int tile = wl / ngrp;
+  if constexpr (P == 0)
+  {
+    if (ad.g.p == 1)
+      box_body<1, T, NS, TABLE, RES>(ad, tile, r_begin, r_end, lds);
+    else if (ad.g.p == 2)
+      box_body<2, T, NS, TABLE, RES>(ad, tile, r_begin, r_end, lds);
+    else
+      box_body<3, T, NS, TABLE, RES>(ad, tile, r_begin, r_end, lds);
+  }
+  else
+    box_body<P, T, NS, TABLE, RES>(ad, tile, r_begin, r_end, lds);
+}
+
 // ---------------------------------------------------------------------------
 // tiles and launch
 // ---------------------------------------------------------------------------
@@ -637,7 +668,9 @@ apply_box(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, i
     return hipSuccess;
   auto go = [&](auto pc, auto nc) {
     constexpr int P = decltype(pc)::value, NS = decltype(nc)::value;
-    if (descs)
+    if constexpr (P == 0)
+      hipLaunchKernelGGL((k_apply_box<0, T, NS, true, false>), dim3(nwork), dim3(16 * NS), 0, st, d0, descs, ndesc);
+    else if (descs)
       hipLaunchKernelGGL((k_apply_box<P, T, NS, true, false>), dim3(nwork), dim3(16 * NS), 0, st, d0, descs, ndesc);
     else if (d0.resid)
       hipLaunchKernelGGL((k_apply_box<P, T, NS, false, true>), dim3(nwork), dim3(16 * NS), 0, st, d0, descs, ndesc);
@@ -654,6 +687,11 @@ apply_box(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, i
   };
   switch (p)
   {
+  case 0:
+    if (!descs)
+      return hipErrorInvalidValue;
+    by_ns(std::integral_constant<int, 0>{});
+    break;
   case 1:
     by_ns(std::integral_constant<int, 1>{});
     break;

@@ -266,7 +266,7 @@ hipError_t apply_op(const Geom & g,
                     ApplyDesc * desc_dev = nullptr,
                     const T * resid_b = nullptr);
 // The box apply (every instance reads element factors; ApplyDesc::bt set, ns
-// common to the launch), and its decomposition of a mesh for nrhs vectors
+// common to the launch; p = 0: a table of instances of any orders), and its decomposition of a mesh for nrhs vectors
 // (ns_only: with that many slots).  The results do not depend on it.
 template <typename T>
 hipError_t apply_box(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, int p, int ns,
@@ -293,11 +293,10 @@ hipError_t apply_scaled(const Geom & g, const PlaneSegs & segs, const Tables<T> 
 void plane_rows(ApplyDesc & d);
 
 // Apply over a device table of instances (all of one order, one tile variant).
-// nwork = sum of ntiles*nrhs, npwork = sum of prows*nrhs.  box_ns != 0: every
-// instance reads element factors and runs the box apply with box_ns slots.
+// nwork = sum of ntiles*nrhs, npwork = sum of prows*nrhs.
 template <typename T>
 hipError_t apply_multi(const TileCandidate * cand, const Tables<T> & tb, const ApplyDesc * descs_dev, int ndesc,
-                       int nwork, int npwork, int grouped, int box_ns, hipStream_t st);
+                       int nwork, int npwork, int grouped, hipStream_t st);
 
 // Sum of the tile-face partials (fixed order) into y.
 template <typename T>

@@ -336,7 +336,7 @@ private:
   void drop_graphs();
   struct ApplyGroup
   {
-    int order;
+    int order;         // 0: several orders (box apply)
     bool batched;      // descriptor table (BATCH kernel) or by-value single instance
     ApplyDesc single;  // by-value descriptor (batched == false)
     const ApplyDesc * descs; // device

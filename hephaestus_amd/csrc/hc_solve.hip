@@ -241,11 +241,13 @@ Engine::set(const std::vector<EngineInst> & inst, int mode, int rhs_block, bool 
     if (k == K_PQ32 && !ir)
       continue;
     const bool prec32 = (k == K_PQ32);
+    // the FP32 group holds the instances whose slots may run FP32 inner
+    // solves (work items of the others would only be gated off)
+    std::vector<std::vector<int>> members(PMAX + 1);
+    bool all_box = true; // of every order: one launch of the box apply
+    int orders = 0;
     for (int p = 1; p <= PMAX; p++)
     {
-      // the FP32 group holds the instances whose slots may run FP32 inner
-      // solves (work items of the others would only be gated off)
-      std::vector<int> ids;
       for (int i : by_order[p])
       {
         const bool may32 = ir && inst_[i].op->fp32_inner_ok();
@@ -253,13 +255,29 @@ Engine::set(const std::vector<EngineInst> & inst, int mode, int rhs_block, bool 
         // FP32 + refinement: the others and those promoted after a slot
         // continued in FP64 (the residual group K_XQ holds every instance)
         if (prec32 ? may32 : (k != K_PQ64 || !may32 || inst_[i].fp64))
-          ids.push_back(i);
+        {
+          members[p].push_back(i);
+          all_box = all_box && inst_[i].op->ef(prec32).qc;
+        }
       }
+      orders += !members[p].empty();
+    }
+    if (all_box && orders > 1)
+    {
+      for (int p = 2; p <= PMAX; p++)
+      {
+        members[1].insert(members[1].end(), members[p].begin(), members[p].end());
+        members[p].clear();
+      }
+    }
+    for (int p = 1; p <= PMAX; p++)
+    {
+      const std::vector<int> & ids = members[p];
       if (ids.empty())
         continue;
       const hc_op_s * op0 = inst_[ids[0]].op;
       ApplyGroup G{};
-      G.order = p;
+      G.order = all_box && orders > 1 ? 0 : p;
       G.prec = prec32 ? 32 : 64;
       const TileCandidate * over = prec32 ? (cands32 ? cands32[p] : nullptr) : (cands64 ? cands64[p] : nullptr);
       G.cand = over ? over : (prec32 ? op0->plan32.cand : op0->plan64.cand);
@@ -271,14 +289,23 @@ Engine::set(const std::vector<EngineInst> & inst, int mode, int rhs_block, bool 
       int w0 = 0, pw0 = 0;
       // every instance has element factors: one launch of the box apply;
       // mixed: every instance reads its quadrature-point factors
+      // (decomposition: as if all the work were vectors of one instance)
       bool all_ef = true;
-      int vecs = 0;
+      int64_t work = 0, big = 0;
+      const hc_op_s * opb = op0;
       for (int i : ids)
       {
-        all_ef = all_ef && inst_[i].op->ef(prec32).qc;
-        vecs += inst_[i].nrhs;
+        const hc_op_s * op = inst_[i].op;
+        all_ef = all_ef && op->ef(prec32).qc;
+        work += op->N * inst_[i].nrhs;
+        if (op->N > big)
+        {
+          big = op->N;
+          opb = op;
+        }
       }
-      G.box_ns = all_ef ? box_tile(op0->g, vecs).ns : 0;
+      auto vecs = [&](const hc_op_s * op) { return (int)std::min<int64_t>((work + op->N / 2) / op->N, 4096); };
+      G.box_ns = all_ef ? box_tile(opb->g, vecs(opb)).ns : 0;
       for (int i : ids)
       {
         const EngineInst & e = inst_[i];
@@ -289,7 +316,7 @@ Engine::set(const std::vector<EngineInst> & inst, int mode, int rhs_block, bool 
         d.prows = (int)d.segs.start[d.segs.nseg];
         d.ntiles = d.g.nt[0] * d.g.nt[1] * d.g.nt[2];
         if (all_ef)
-          set_box_tile(d, box_tile(d.g, vecs, G.box_ns));
+          set_box_tile(d, box_tile(d.g, vecs(op), G.box_ns));
         d.nrhs = e.nrhs;
         d.rb = G.batched ? (rhs_block > 0 ? std::min(rhs_block, e.nrhs) : default_rhs_block(d.ntiles, e.nrhs)) : 1;
         d.qd = prec32 ? (const void *)op->qd32 : (const void *)op->qd64;
@@ -359,14 +386,17 @@ Engine::apply(Kind k, hipStream_t st)
   for (const ApplyGroup & G : groups_[k])
   {
     hipError_t e;
-    if (G.batched)
+    if (G.box_ns)
+    {
+      const ApplyDesc * descs = G.batched ? G.descs : nullptr;
+      e = G.prec == 64 ? apply_box<double>(G.single, descs, G.ndesc, G.nwork, G.order, G.box_ns, st)
+                       : apply_box<float>(G.single, descs, G.ndesc, G.nwork, G.order, G.box_ns, st);
+    }
+    else if (G.batched)
       e = G.prec == 64 ? apply_multi<double>(G.cand, *(const Tables<double> *)G.tables, G.descs, G.ndesc, G.nwork,
-                                             G.npwork, G.grouped, G.box_ns, st)
+                                             G.npwork, G.grouped, st)
                        : apply_multi<float>(G.cand, *(const Tables<float> *)G.tables, G.descs, G.ndesc, G.nwork,
-                                            G.npwork, G.grouped, G.box_ns, st);
-    else if (G.box_ns)
-      e = G.prec == 64 ? apply_box<double>(G.single, nullptr, 1, G.nwork, G.order, G.box_ns, st)
-                       : apply_box<float>(G.single, nullptr, 1, G.nwork, G.order, G.box_ns, st);
+                                            G.npwork, G.grouped, st);
     else
     {
       e = G.cand->launch(G.single, nullptr, 1, G.nwork, 0, G.tables, G.prec, st);
