@@ -1003,7 +1003,7 @@ apply_op(const Geom & g, const PlaneSegs & segs, const Tables<T> & tb, const T *
   if (ef.qc)
   {
     // box mesh: one launch, results independent of rb (one rhs per work item)
-    set_box_tile(d, box_tile(g, nrhs));
+    set_box_tile(d, nrhs);
     return apply_box<T>(d, nullptr, 1, d.ntiles * nrhs, g.p, d.bt.ns, st);
   }
   if (rb > 1 && nrhs > 1)
@@ -1044,7 +1044,7 @@ apply_scaled(const Geom & g, const PlaneSegs & segs, const Tables<T> & tb, const
   d.cscale = cscale;
   if (ef.qc)
   {
-    set_box_tile(d, box_tile(g, 1));
+    set_box_tile(d, 1);
     return apply_box<T>(d, nullptr, 1, d.ntiles, g.p, d.bt.ns, st);
   }
   // term weights are honoured by the batched kernel (descriptor in device memory)

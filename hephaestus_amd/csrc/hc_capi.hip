@@ -322,6 +322,7 @@ try
       delete op;
       return rc;
     }
+    op->box_one = hc::box_tile(g, 1);
     const double det = op->h[0] * (op->h[1] * op->h[2]);
     for (int a = 0; a < 3; a++)
     {
@@ -870,7 +871,7 @@ try
   d.ntiles = pl.g.nt[0] * pl.g.nt[1] * pl.g.nt[2];
   const bool box = d.ef.qc != nullptr;
   if (box)
-    hc::set_box_tile(d, hc::box_tile(pl.g, 1));
+    hc::set_box_tile(d, 1);
   const void * tb = f32 ? (const void *)&op->tb32 : (const void *)&op->tb64;
   std::vector<hipEvent_t> ev(3 * reps);
   for (auto & e : ev)

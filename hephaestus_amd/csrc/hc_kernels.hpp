@@ -28,6 +28,14 @@ struct PlaneSegs
   int64_t eoff[3][3];
 };
 
+// Decomposition of a box apply (hc_apply_box.hip): ns element slots per
+// workgroup, cx by cy of them per tile, ntx by nty tiles, nzc chunks of zc
+// element layers.
+struct BoxTile
+{
+  int ns, cx, cy, ntx, nty, zc, nzc;
+};
+
 // One operator instance of an apply launch.  Work items are (tile, rhs group)
 // with the group index fastest; a group is rb consecutive right-hand sides (the
 // single-instance kernel uses rb = 1).  The items of instance i occupy
@@ -45,14 +53,7 @@ struct ElemFactors
   const void * qc = nullptr;
   double ck[3] = {0, 0, 0};
   double mk[3] = {0, 0, 0};
-};
-
-// Decomposition of a box apply (hc_apply_box.hip): ns element slots per
-// workgroup, cx by cy of them per tile, ntx by nty tiles, nzc chunks of zc
-// element layers.
-struct BoxTile
-{
-  int ns, cx, cy, ntx, nty, zc, nzc;
+  const BoxTile * one = nullptr; // host: the operator's decomposition for one vector
 };
 
 struct ApplyDesc
@@ -278,6 +279,11 @@ set_box_tile(ApplyDesc & d, const BoxTile & b)
 {
   d.bt = b;
   d.ntiles = b.ntx * b.nty * b.nzc;
+}
+inline void
+set_box_tile(ApplyDesc & d, int nrhs)
+{
+  set_box_tile(d, nrhs == 1 && d.ef.one ? *d.ef.one : box_tile(d.g, nrhs));
 }
 // Right-hand sides per work item for a batch of nrhs on ntiles tiles.
 int default_rhs_block(int ntiles, int nrhs);

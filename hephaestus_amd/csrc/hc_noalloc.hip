@@ -124,7 +124,7 @@ try
   d.ntiles = pl.g.nt[0] * pl.g.nt[1] * pl.g.nt[2];
   if (d.ef.qc)
   {
-    hc::set_box_tile(d, hc::box_tile(pl.g, 1));
+    hc::set_box_tile(d, 1);
     HC_TRY_HIP(hc::apply_box<double>(d, nullptr, 1, d.ntiles, pl.g.p, d.bt.ns, st));
     return HC_OK;
   }

@@ -182,6 +182,7 @@ struct hc_op_s
   double * qc64 = nullptr;
   float * qc32 = nullptr;
   double ck[3] = {0, 0, 0}, mk[3] = {0, 0, 0};
+  hc::BoxTile box_one{}; // decomposition of the box apply for one vector
   int ef_mode = 1;
   hc::ElemFactors ef(bool f32) const
   {
@@ -189,6 +190,7 @@ struct hc_op_s
     if (ef_mode && qc64)
     {
       f.qc = f32 ? (const void *)qc32 : (const void *)qc64;
+      f.one = &box_one;
       for (int a = 0; a < 3; a++)
       {
         f.ck[a] = ck[a];
