@@ -1004,7 +1004,7 @@ apply_op(const Geom & g, const PlaneSegs & segs, const Tables<T> & tb, const T *
   {
     // box mesh: one launch, results independent of rb (one rhs per work item)
     set_box_tile(d, nrhs);
-    return apply_box<T>(d, nullptr, 1, d.ntiles * nrhs, g.p, d.bt.ns, st);
+    return apply_box<T>(d, nullptr, 1, d.ntiles * nrhs, g.p, d.bt.ns, ef.vert != nullptr, st);
   }
   if (rb > 1 && nrhs > 1)
   {
@@ -1045,7 +1045,7 @@ apply_scaled(const Geom & g, const PlaneSegs & segs, const Tables<T> & tb, const
   if (ef.qc)
   {
     set_box_tile(d, 1);
-    return apply_box<T>(d, nullptr, 1, d.ntiles, g.p, d.bt.ns, st);
+    return apply_box<T>(d, nullptr, 1, d.ntiles, g.p, d.bt.ns, ef.vert != nullptr, st);
   }
   // term weights are honoured by the batched kernel (descriptor in device memory)
   hipError_t e = hipMemcpyAsync(desc_dev, &d, sizeof(d), hipMemcpyHostToDevice, st);

@@ -1,5 +1,5 @@
-// Apply of dt*nu K + sigma M on axis-aligned box meshes from two factors per
-// element (ApplyDesc::ef), on the FP64 matrix units (gfx950).
+// Apply of dt*nu K + sigma M on structured meshes from two factors per element
+// (ApplyDesc::ef), on the FP64 matrix units (gfx950).  First box elements:
 //
 // The operator is that of hc_apply.hip (EquationSystem::Mult,
 // src/equation_systems/equation_system.cpp:200-204, on the system of
@@ -41,8 +41,25 @@
 // one launch, no partial sums in memory, and the same bits for every tile
 // shape.
 //
-// Measured at 48^3 order 3 (9.08 M DOFs): 195 us per FP64 apply with the
-// LDS-staged tile kernel and its face assembly, 63 us here (FP32 vectors: 115
+// Trilinear elements (HEX; ApplyDesc::ef with vertices) march the same way, but
+// their integrals do not separate: u is interpolated to the (p + 1)^3 points by
+// matrix products along y and x and register arithmetic along z, the lane keeps
+// its (x, y) point, takes the Jacobian there from the corners of the lower and
+// upper vertex plane (the upper is carried to the next layer), applies mass and
+// curl factors (adj(J^T J) sigma w / |det J| and J^T J dt nu w / |det J|) and the
+// transposed stages follow.  Against 12 (p + 1)^3 stored factors per element
+// read by the tile kernel of hc_apply_qp.hip this reads 24 bytes a vertex and 16
+// an element.  About 700 vector instructions and 86 matrix products a layer at
+// order 3 keep 244 registers, so two waves per SIMD and tiles of at most 32
+// elements, of whose work 1.5 x 1.1 is duplicated: bound by the FP64 pipe and
+// its latencies.  Measured, stored factors -> here: 48^3 order 3 223 -> 157 us,
+// 48^3 order 2 118 -> 106 us, 33x26x19 order 2 30 -> 24 us, 64^3 order 1
+// 80 -> 39 us, 16^3 order 1 12 -> 7.7 us.  Error against extended precision over
+// 40 meshes of 6x5x4 to 44x34x20: 9.1e-16 -> 7.2e-16 in the mean (the stored
+// factors take the Jacobian from sums of coordinates, here from differences).
+//
+// Measured on boxes at 48^3 order 3 (9.08 M DOFs): 194 us per FP64 apply with the
+// LDS-staged tile kernel and its face assembly, 69 us here (FP32 vectors: 114
 // and 60 us).  Memory traffic is 164 MB (147 MB algorithmic, 30 us at the copy
 // rate); the bound is the FP64 pipe -- one 4 x 4 x 4 product takes 7 ns per SIMD
 // and a vector FMA 2.3 ns, and they do not overlap -- at about 65 % use, the
@@ -112,8 +129,102 @@ box_lds()
   return 8 * P * (NS * (P == 1 ? 8 : 4) + 1) + (3 * P + 2) * 16 * NS;
 }
 
+// What a lane (f, s) of a block keeps of the 1-D matrices, by f * 4 + s.  (As
+// selects over the entries this took 300 to 500 instructions of every launch.)
+// Entry [f][s] of a matrix is its A operand, [s][f] its B operand; at order 1,
+// where a block is 2 x 2 elements, the matrices are block-diagonal.
+template <int N>
+struct LaneTab
+{
+  double v[16][N];
+};
+template <int P>
+constexpr LaneTab<6>
+make_box_lanes()
+{
+  LaneTab<6> t{};
+  const basis::BoxTab<P> b = basis::box_tab<P>();
+  for (int f = 0; f < 4; f++)
+    for (int s = 0; s < 4; s++)
+    {
+      const int pf = P == 1 ? f % 2 : f, ps = P == 1 ? s % 2 : s;
+      double * v = t.v[f * 4 + s];
+      if (pf > P || ps > P)
+        continue;
+      if (P > 1 || f / 2 == s / 2)
+      {
+        v[0] = b.M[pf][ps];
+        v[1] = pf < P ? b.D[pf < P ? pf : 0][ps] : 0.0;
+        v[2] = ps < P ? b.D[ps < P ? ps : 0][pf] : 0.0;
+      }
+      v[3] = pf < P ? b.w[pf < P ? pf : 0] : 0.0;
+      v[4] = ps < P ? b.w[ps < P ? ps : 0] : 0.0;
+    }
+  return t;
+}
+// interpolation to the quadrature points (open, closed, derivative of closed),
+// [f][s] and [s][f]; the lane's point (f, s) and its weight
+template <int P>
+constexpr LaneTab<10>
+make_hex_lanes()
+{
+  LaneTab<10> t{};
+  const basis::Tab<double> b = basis::tab<P, double>();
+  for (int f = 0; f < 4; f++)
+    for (int s = 0; s < 4; s++)
+    {
+      const int pf = P == 1 ? f % 2 : f, ps = P == 1 ? s % 2 : s;
+      double * v = t.v[f * 4 + s];
+      if (pf > P || ps > P)
+        continue;
+      if (P > 1 || f / 2 == s / 2)
+      {
+        v[0] = ps < P ? b.Bo[pf * P + (ps < P ? ps : 0)] : 0.0;
+        v[1] = b.Bc[pf * (P + 1) + ps];
+        v[2] = b.Gc[pf * (P + 1) + ps];
+        v[3] = pf < P ? b.Bo[ps * P + (pf < P ? pf : 0)] : 0.0;
+        v[4] = b.Bc[ps * (P + 1) + pf];
+        v[5] = b.Gc[ps * (P + 1) + pf];
+      }
+      v[6] = b.qp[pf];
+      v[7] = b.qp[ps];
+      v[8] = b.qw[pf] * b.qw[ps];
+    }
+  return t;
+}
+template <int P>
+__device__ constexpr LaneTab<6> box_lanes = make_box_lanes<P>();
+template <int P>
+__device__ constexpr LaneTab<10> hex_lanes = make_hex_lanes<P>();
+
+// The corners (x, y) of an element on one vertex plane as they enter the
+// trilinear map at reference point (a, b): the point, relative to corner (0, 0),
+// and the two in-plane derivatives.  (Differences of coordinates are taken
+// first throughout, so that the relative error does not grow with 1 / h.)
+struct PlaneGeom
+{
+  double p[3], dx[3], dy[3];
+};
+__device__ inline PlaneGeom
+plane_geom(const double * v, double a, double b)
+{
+#pragma clang fp contract(off)
+  PlaneGeom g;
+#pragma unroll
+  for (int r = 0; r < 3; r++)
+  {
+    const double v00 = v[r], v10 = v[3 + r], v01 = v[6 + r], v11 = v[9 + r];
+    const double e0 = v10 - v00, e1 = v11 - v01; // along x at y = 0, 1
+    g.dx[r] = __builtin_fma(b, e1 - e0, e0);
+    const double f0 = v01 - v00, f1 = v11 - v10; // along y at x = 0, 1
+    g.dy[r] = __builtin_fma(a, f1 - f0, f0);
+    g.p[r] = __builtin_fma(b, g.dy[r], a * e0);
+  }
+  return g;
+}
+
 // The right-hand sides [r_begin, r_end) of tile `tile` of one instance.
-template <int P, typename T, int NS, bool TABLE, bool RES>
+template <int P, typename T, int NS, bool TABLE, bool RES, bool HEX>
 __device__ __forceinline__ void
 box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
 {
@@ -160,9 +271,10 @@ box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
     return (gi == 0 && ((pec >> (2 * axis)) & 1)) || (gi == n * P && ((pec >> (2 * axis + 1)) & 1));
   };
   const bool essx = face(1, eyN * P + ps, ny), essy = face(0, exN * P + pf, nx), essz = essx || essy;
-  const bool essyT = face(0, exT * P + ps, nx);
+  const bool essyL = HEX ? essy : face(0, exT * P + ps, nx); // lanes as they load u_y
   // lanes that read a DOF of the component, and those that write it
-  const bool ldx = vN && pf < P && ps <= P, ldy = vT && pf < P && ps <= P, ldz = vN && pf <= P && ps <= P;
+  const bool ldx = vN && pf < P && ps <= P, ldz = vN && pf <= P && ps <= P;
+  const bool ldy = HEX ? vN && pf <= P && ps < P : vT && pf < P && ps <= P;
   const bool outN = vN && (exN > xs || tx == 0) && (eyN > ys || ty == 0);
   const bool topx = pf == P && exN == nx - 1, topy = ps == P && eyN == ny - 1;
   const bool ownx = outN && pf < P && (ps < P || topy);
@@ -172,17 +284,17 @@ box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
   // kept in LDS from load to store (own lane, component y transposed): planes
   // 1 .. p-1 of x and y and p planes of z of the layer, and the lowest plane of
   // x and y of the layer (by parity of z: the one above is known a layer early)
-  const bool wave_ess = __any((vN && essz) || (vT && essyT)) != 0;
+  const bool wave_ess = __any((vN && essz) || (vT && essyL)) != 0;
   using PecRow = double[16 * NS];
   PecRow * const sE = (PecRow *)(sX + 8);
   constexpr int EX = 0, EY = P - 1, EZ = 2 * P - 2, EX0 = 3 * P - 2, EY0 = 3 * P;
-  const int eN = threadIdx.x, eT = (threadIdx.x & ~51) | (lf << 4) | ls;
+  const int eN = threadIdx.x, eT = HEX ? eN : (int)((threadIdx.x & ~51) | (lf << 4) | ls);
   // byte offsets inside a plane of each component, from the tile's first row
   const uint32_t cx0 = (uint32_t)g.cd[0][0], cy0 = (uint32_t)g.cd[1][0], cz0 = (uint32_t)g.cd[2][0];
   const uint32_t lxN = (sx * EJ + ef) * P + pf, lyN = (sy * EJ + es) * P + ps;
   const uint32_t oxN = (lyN * cx0 + lxN) * SZ, oyN = (lyN * cy0 + lxN) * SZ, ozN = (lyN * cz0 + lxN) * SZ;
-  const uint32_t oyT = (((sy * EJ + ef) * P + pf) * cy0 + (sx * EJ + es) * P + ps) * SZ;
-  const uint32_t ilx = ldx ? oxN : OOB, ily = ldy ? oyT : OOB, ilz = ldz ? ozN : OOB; // loads
+  const uint32_t oyL = HEX ? oyN : (((sy * EJ + ef) * P + pf) * cy0 + (sx * EJ + es) * P + ps) * SZ;
+  const uint32_t ilx = ldx ? oxN : OOB, ily = ldy ? oyL : OOB, ilz = ldz ? ozN : OOB; // loads
   // entries of a plane of each component
   const int64_t plx = g.cd[0][0] * g.cd[0][1], ply = g.cd[1][0] * g.cd[1][1], plz = g.cd[2][0] * g.cd[2][1];
   const uint32_t spx = (uint32_t)plx * SZ, spy = (uint32_t)ply * SZ, spz = (uint32_t)plz * SZ; // plane bytes
@@ -204,35 +316,58 @@ box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
   const int rD = (hasL && hasB) ? (slD * EJ + eB) * 4 + ((P == 1) ? 2 * eL + 1 : P) : FZ;
 
   // matrix operands: lane (f, s) holds entry [f][s] as A and [s][f] as B
-  const bool dia = (P > 1) || (ef == es); // block-diagonal at order 1
+  const int lane16 = lf * 4 + ls;
   double opM = 0, opD = 0, opDt = 0, wf = 0, wsl = 0;
-#pragma unroll
-  for (int i = 0; i <= P; i++)
-#pragma unroll
-    for (int j = 0; j <= P; j++)
-    {
-      if (pf == i && ps == j && dia)
-        opM = tb.M[i][j];
-      if (i < P && pf == i && ps == j && dia)
-        opD = tb.D[i][j]; // [open f][closed s]
-      if (i < P && ps == i && pf == j && dia)
-        opDt = tb.D[i][j]; // [open s][closed f]
-    }
-  const double opI = (lf == ls) ? 1.0 : 0.0;
-#pragma unroll
-  for (int i = 0; i < P; i++)
+  if constexpr (!HEX)
   {
-    if (pf == i)
-      wf = tb.w[i];
-    if (ps == i)
-      wsl = tb.w[i];
+    const double * lo = box_lanes<P>.v[lane16];
+    opM = lo[0];
+    opD = lo[1]; // [open f][closed s]
+    opDt = lo[2]; // [open s][closed f]
+    wf = lo[3];
+    wsl = lo[4];
   }
+  const double opI = (lf == ls) ? 1.0 : 0.0;
   // lane weights of the element factors (mass x, y, z; curl x, y, z): the
   // weights of x and y are equal per axis up to the axis constants
   const double msc = ad.mscale, csc = ad.cscale;
   const double mk0 = ad.ef.mk[0] * msc, mk1 = ad.ef.mk[1] * msc, mk2 = ad.ef.mk[2] * msc;
   const double ck0 = ad.ef.ck[0] * csc, ck1 = ad.ef.ck[1] * csc, ck2 = -(ad.ef.ck[2] * csc);
   const double wfs = wf * wsl;
+  // trilinear elements: interpolation to the quadrature points and its
+  // transpose (operand entries [f][s] and [s][f]), the lane's point
+  constexpr basis::Tab<double> qt = basis::tab<P, double>();
+  double fBo = 0, fBc = 0, fGc = 0, bBo = 0, bBc = 0, bGc = 0, qa = 0, qb = 0, wxy = 0;
+  if constexpr (HEX)
+  {
+    const double * lo = hex_lanes<P>.v[lane16];
+    fBo = lo[0];
+    fBc = lo[1];
+    fGc = lo[2];
+    bBo = lo[3];
+    bBc = lo[4];
+    bGc = lo[5];
+    qa = lo[6];
+    qb = lo[7];
+    wxy = lo[8];
+  }
+  // vertices: the element's corner (0, 0) on a vertex plane, from the tile's first
+  const double * vert = HEX ? ad.ef.vert + 3 * ((int64_t)ys * (nx + 1) + xs) : nullptr;
+  const int64_t vpl = 3 * (int64_t)(nx + 1) * (ny + 1);
+  const uint32_t ov = vN ? ((uint32_t)(sy * EJ + es) * (nx + 1) + sx * EJ + ef) * 24 : OOB;
+  const uint32_t ov1 = vN ? ov + (uint32_t)(nx + 1) * 24 : OOB;
+  auto load_corners = [&](int z, double (&v)[15]) { // and corner (0, 0) of the plane below
+    const double * b = vert + z * vpl;
+#pragma unroll
+    for (int r = 0; r < 3; r++)
+    {
+      v[r] = ldb(b, ov, r * 8);
+      v[3 + r] = ldb(b, ov, 24 + r * 8);
+      v[6 + r] = ldb(b, ov1, r * 8);
+      v[9 + r] = ldb(b, ov1, 24 + r * 8);
+      v[12 + r] = ldb(z > 0 ? b - vpl : b, ov, r * 8);
+    }
+  };
 
   const T * qc = (const T *)ad.ef.qc + 2 * ((int64_t)ys * nx + xs);
   const uint32_t oeN = vN ? ((uint32_t)(sy * EJ + es) * nx + sx * EJ + ef) * 2 * SZ : OOB;
@@ -262,7 +397,7 @@ box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
       const T * q = qc + z * epl;
       nq[0] = ldb(q, oeN);
       nq[1] = ldb(q + 1, oeN);
-      if constexpr (P == 1)
+      if constexpr (P == 1 && !HEX)
       {
         nq[2] = ldb(q, oeT);
         nq[3] = ldb(q + 1, oeT);
@@ -273,7 +408,7 @@ box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
       const T vx = ldb(xv + bx, ilx), vy = ldb(xv + by, ily);
       load_layer(bx, by, bz, zs);
       ux[0] = (zf || essx) ? 0.0 : (double)vx;
-      uy[0] = (zf || essyT) ? 0.0 : (double)vy;
+      uy[0] = (zf || essyL) ? 0.0 : (double)vy;
       sE[EX0 + (zs & 1)][eN] = (double)vx;
       sE[EY0 + (zs & 1)][eT] = (double)vy;
       // stores that store nothing: in the loop the loads of the next layer are
@@ -282,6 +417,14 @@ box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
 #pragma unroll
       for (int k = 0; k < 3 * P; k++)
         stb((T *)ad.y + rof, OOB, T(0), k);
+    }
+    PlaneGeom g0{}; // lower vertex plane of the layer
+    double nv[15] = {};
+    if constexpr (HEX)
+    {
+      load_corners(zs, nv);
+      g0 = plane_geom(nv, qa, qb);
+      load_corners(zs + 1, nv);
     }
     double carx = 0.0, cary = 0.0;
     int buf = 0;
@@ -316,17 +459,146 @@ box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
             sE[EY0 + ((z + 1) & 1)][eT] = uy[P];
           }
           ux[k + 1] = essx ? 0.0 : ux[k + 1];
-          uy[k + 1] = essyT ? 0.0 : uy[k + 1];
+          uy[k + 1] = essyL ? 0.0 : uy[k + 1];
         }
       }
       ux[P] = ztop ? 0.0 : ux[P];
       uy[P] = ztop ? 0.0 : uy[P];
       const double nuN = (double)nq[0], sgN = (double)nq[1];
-      const double nuT = (P == 1) ? (double)nq[P == 1 ? 2 : 0] : nuN, sgT = (P == 1) ? (double)nq[P == 1 ? 3 : 1] : sgN;
-      if (z + 1 < z1)
+      const double nuT = (P == 1 && !HEX) ? (double)nq[P == 1 ? 2 : 0] : nuN;
+      const double sgT = (P == 1 && !HEX) ? (double)nq[P == 1 ? 3 : 1] : sgN;
+      if (!HEX && z + 1 < z1)
         load_layer(bx + P * plx, by + P * ply, bz + P * plz, z + 1);
 
       double yx[P + 1], yy[P + 1], yz[P];
+      if constexpr (HEX)
+      {
+        auto phase = []() { __builtin_amdgcn_sched_barrier(0); };
+        constexpr int Q = P + 1;
+        // x, y interpolation (y first: N -> T -> N): values and x, y derivatives
+        double ux0[P + 1], uxy[P + 1], uy0[P + 1], uyx[P + 1], uz0[P], uzx[P], uzy[P];
+#pragma unroll
+        for (int k = 0; k <= P; k++)
+        {
+          const double a = mm(ux[k], fBc, 0.0), b = mm(ux[k], fGc, 0.0), c = mm(uy[k], fBo, 0.0);
+          ux0[k] = mm(a, fBo, 0.0);
+          uxy[k] = mm(b, fBo, 0.0);
+          uy0[k] = mm(c, fBc, 0.0);
+          uyx[k] = mm(c, fGc, 0.0);
+        }
+#pragma unroll
+        for (int k = 0; k < P; k++)
+        {
+          const double a = mm(uz[k], fBc, 0.0), b = mm(uz[k], fGc, 0.0);
+          uz0[k] = mm(a, fBc, 0.0);
+          uzx[k] = mm(a, fGc, 0.0);
+          uzy[k] = mm(b, fBc, 0.0);
+        }
+        phase();
+        const PlaneGeom g1 = plane_geom(nv, qa, qb);
+        double jz[3];
+#pragma unroll
+        for (int r = 0; r < 3; r++)
+          jz[r] = (nv[r] - nv[12 + r]) + (g1.p[r] - g0.p[r]);
+        const double sm0 = wxy * (sgN * msc), sc0 = wxy * (nuN * csc);
+        // sums over the quadrature points along z of the transposed stage:
+        // (value, y derivative) of x, (value, x derivative) of y, (value, x, y) of z
+        double sx0[P + 1] = {}, sxy[P + 1] = {}, sy0[P + 1] = {}, syx[P + 1] = {}, sz0[P] = {}, szx[P] = {}, szy[P] = {};
+#pragma unroll
+        for (int q = 0; q < Q; q++)
+        {
+          double w0 = 0.0, w1 = 0.0, w2 = 0.0, c0 = 0.0, c1 = 0.0, c2 = 0.0;
+#pragma unroll
+          for (int k = 0; k <= P; k++)
+          {
+            const double Bc = qt.Bc[q * (P + 1) + k], Gc = qt.Gc[q * (P + 1) + k];
+            w0 = __builtin_fma(Bc, ux0[k], w0);
+            w1 = __builtin_fma(Bc, uy0[k], w1);
+            c0 = __builtin_fma(-Gc, uy0[k], c0); // - d/dz u_y
+            c1 = __builtin_fma(Gc, ux0[k], c1);  // + d/dz u_x
+            c2 = __builtin_fma(Bc, uyx[k], c2);  // + d/dx u_y
+            c2 = __builtin_fma(-Bc, uxy[k], c2); // - d/dy u_x
+          }
+#pragma unroll
+          for (int k = 0; k < P; k++)
+          {
+            const double Bo = qt.Bo[q * P + k];
+            w2 = __builtin_fma(Bo, uz0[k], w2);
+            c0 = __builtin_fma(Bo, uzy[k], c0);  // + d/dy u_z
+            c1 = __builtin_fma(-Bo, uzx[k], c1); // - d/dx u_z
+          }
+          // J = (d/dx, d/dy, d/dz) of the map; mass adj(J^T J) / |det|, curl J^T J / |det|
+          double jx[3], jy[3];
+#pragma unroll
+          for (int r = 0; r < 3; r++)
+          {
+            jx[r] = __builtin_fma(qt.qp[q], g1.dx[r] - g0.dx[r], g0.dx[r]);
+            jy[r] = __builtin_fma(qt.qp[q], g1.dy[r] - g0.dy[r], g0.dy[r]);
+          }
+          auto dot = [](const double * u, const double * v) {
+            return __builtin_fma(u[0], v[0], __builtin_fma(u[1], v[1], u[2] * v[2]));
+          };
+          const double G00 = dot(jx, jx), G01 = dot(jx, jy), G02 = dot(jx, jz);
+          const double G11 = dot(jy, jy), G12 = dot(jy, jz), G22 = dot(jz, jz);
+          const double cr[3] = {__builtin_fma(jy[1], jz[2], -(jy[2] * jz[1])), __builtin_fma(jy[2], jz[0], -(jy[0] * jz[2])),
+                                __builtin_fma(jy[0], jz[1], -(jy[1] * jz[0]))};
+          const double det = __builtin_fabs(dot(jx, cr));
+          const double rd = qt.qw[q] / (vN ? det : 1.0); // (lanes without a point carry zeros)
+          const double sm = sm0 * rd, sc = sc0 * rd;
+          const double A00 = __builtin_fma(G11, G22, -(G12 * G12)), A01 = __builtin_fma(G02, G12, -(G01 * G22));
+          const double A02 = __builtin_fma(G01, G12, -(G02 * G11)), A11 = __builtin_fma(G00, G22, -(G02 * G02));
+          const double A12 = __builtin_fma(G01, G02, -(G00 * G12)), A22 = __builtin_fma(G00, G11, -(G01 * G01));
+          auto row = [](double a, double b, double c, double u, double v, double w) {
+            return __builtin_fma(a, u, __builtin_fma(b, v, c * w));
+          };
+          // (the diagonal term, the largest, is added last)
+          const double m0 = sm * row(A00, A01, A02, w0, w1, w2), m1 = sm * row(A11, A01, A12, w1, w0, w2);
+          const double m2 = sm * row(A22, A02, A12, w2, w0, w1);
+          const double k0 = sc * row(G00, G01, G02, c0, c1, c2), k1 = sc * row(G11, G01, G12, c1, c0, c2);
+          const double k2 = sc * row(G22, G02, G12, c2, c0, c1);
+#pragma unroll
+          for (int k = 0; k <= P; k++)
+          {
+            const double Bc = qt.Bc[q * (P + 1) + k], Gc = qt.Gc[q * (P + 1) + k];
+            sx0[k] = __builtin_fma(Gc, k1, __builtin_fma(Bc, m0, sx0[k]));
+            sxy[k] = __builtin_fma(-Bc, k2, sxy[k]);
+            sy0[k] = __builtin_fma(-Gc, k0, __builtin_fma(Bc, m1, sy0[k]));
+            syx[k] = __builtin_fma(Bc, k2, syx[k]);
+          }
+#pragma unroll
+          for (int k = 0; k < P; k++)
+          {
+            const double Bo = qt.Bo[q * P + k];
+            sz0[k] = __builtin_fma(Bo, m2, sz0[k]);
+            szy[k] = __builtin_fma(Bo, k0, szy[k]);
+            szx[k] = __builtin_fma(-Bo, k1, szx[k]);
+          }
+          phase();
+        }
+        g0 = g1;
+        // (the last layer loads itself again: a branch here would let the
+        // compiler sink the points above past it and keep the loads alive there)
+        const int64_t zn = z + 1 < z1 ? P : 0;
+        load_layer(bx + zn * plx, by + zn * ply, bz + zn * plz, min(z + 1, z1 - 1));
+        load_corners(min(z + 2, z1), nv);
+        phase();
+        // transposed x, y stages
+#pragma unroll
+        for (int k = 0; k <= P; k++)
+        {
+          const double a = mm(sxy[k], bGc, mm(sx0[k], bBc, 0.0));
+          yx[k] = mm(a, bBo, 0.0);
+          const double b = mm(sy0[k], bBo, 0.0), c = mm(syx[k], bBo, 0.0);
+          yy[k] = mm(c, bGc, mm(b, bBc, 0.0));
+        }
+#pragma unroll
+        for (int k = 0; k < P; k++)
+        {
+          const double a = mm(szy[k], bGc, mm(sz0[k], bBc, 0.0)), b = mm(szx[k], bBc, 0.0);
+          yz[k] = mm(b, bGc, mm(a, bBc, 0.0));
+        }
+      }
+      else
       {
         // In phases (the scheduler keeps to them: the order holds the number of
         // live registers below the 128 that four waves per SIMD leave each)
@@ -553,8 +825,8 @@ box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
 
 // P = 0: the instances of the table may have any order (one launch, and the
 // small instances of one order run beside the large ones of another)
-template <int P, typename T, int NS, bool TABLE, bool RES>
-__global__ void __launch_bounds__(16 * NS, 4)
+template <int P, typename T, int NS, bool TABLE, bool RES, bool HEX>
+__global__ void __launch_bounds__(16 * NS, HEX ? 2 : 4)
 k_apply_box(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc)
 {
   __shared__ double lds[box_lds<P == 0 ? PMAX : P, NS>()];
@@ -572,14 +844,14 @@ k_apply_box(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc)
   if constexpr (P == 0)
   {
     if (ad.g.p == 1)
-      box_body<1, T, NS, TABLE, RES>(ad, tile, r_begin, r_end, lds);
+      box_body<1, T, NS, TABLE, RES, HEX>(ad, tile, r_begin, r_end, lds);
     else if (ad.g.p == 2)
-      box_body<2, T, NS, TABLE, RES>(ad, tile, r_begin, r_end, lds);
+      box_body<2, T, NS, TABLE, RES, HEX>(ad, tile, r_begin, r_end, lds);
     else
-      box_body<3, T, NS, TABLE, RES>(ad, tile, r_begin, r_end, lds);
+      box_body<3, T, NS, TABLE, RES, HEX>(ad, tile, r_begin, r_end, lds);
   }
   else
-    box_body<P, T, NS, TABLE, RES>(ad, tile, r_begin, r_end, lds);
+    box_body<P, T, NS, TABLE, RES, HEX>(ad, tile, r_begin, r_end, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -594,14 +866,14 @@ k_apply_box(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc)
 // with 16 slots, 14.6 us with 64), one that fills them the fewest duplicated
 // elements (48^3 order 3: 63 us with 64 slots, 78 us with 16).
 BoxTile
-box_tile(const Geom & g, int nrhs, int ns_only)
+box_tile(const Geom & g, int nrhs, int ns_only, bool hex)
 {
   const int ej = g.p == 1 ? 2 : 1;
   auto tiles = [&](int n, int c) { return n <= c * ej ? 1 : (n - 1 + c * ej - 2) / (c * ej - 1); };
   constexpr int CUS = 256;
   BoxTile best{};
   double cost = 1e300;
-  for (int ns = 16; ns <= 64; ns *= 2)
+  for (int ns = 16; ns <= (hex ? 32 : 64); ns *= 2)
   {
     if (ns_only && ns != ns_only)
       continue;
@@ -624,7 +896,7 @@ box_tile(const Geom & g, int nrhs, int ns_only)
         b.nty = nty;
       }
     }
-    const int bpc = 64 / ns, wpb = ns / 16; // workgroups per CU, waves per SIMD of one
+    const int bpc = (hex ? 32 : 64) / ns, wpb = ns / 16; // workgroups per CU, waves per SIMD of one
     const int64_t cap = (int64_t)CUS * bpc;
     for (int zc = g.n[2];;)
     {
@@ -657,25 +929,37 @@ box_fits(const Geom & g)
   int64_t pl = 0;
   for (int c = 0; c < 3; c++)
     pl = std::max(pl, g.cd[c][0] * g.cd[c][1]);
-  return (g.p + 1) * pl * (int64_t)sizeof(double) < (int64_t)0xFFFFF000;
+  const int64_t vp = (int64_t)(g.n[0] + 1) * (g.n[1] + 1); // vertices of a plane (trilinear)
+  return std::max((g.p + 1) * pl * (int64_t)sizeof(double), 24 * vp) < (int64_t)0xFFFFF000;
 }
 
 template <typename T>
 hipError_t
-apply_box(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, int p, int ns, hipStream_t st)
+apply_box(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, int p, int ns, bool hex, hipStream_t st)
 {
   if (nwork <= 0)
     return hipSuccess;
+  const dim3 grid(nwork);
   auto go = [&](auto pc, auto nc) {
     constexpr int P = decltype(pc)::value, NS = decltype(nc)::value;
+    const dim3 blk(16 * NS);
+    auto run = [&](auto kern) { hipLaunchKernelGGL(kern, grid, blk, 0, st, d0, descs, ndesc); };
     if constexpr (P == 0)
-      hipLaunchKernelGGL((k_apply_box<0, T, NS, true, false>), dim3(nwork), dim3(16 * NS), 0, st, d0, descs, ndesc);
-    else if (descs)
-      hipLaunchKernelGGL((k_apply_box<P, T, NS, true, false>), dim3(nwork), dim3(16 * NS), 0, st, d0, descs, ndesc);
-    else if (d0.resid)
-      hipLaunchKernelGGL((k_apply_box<P, T, NS, false, true>), dim3(nwork), dim3(16 * NS), 0, st, d0, descs, ndesc);
+      run(k_apply_box<0, T, NS, true, false, false>);
     else
-      hipLaunchKernelGGL((k_apply_box<P, T, NS, false, false>), dim3(nwork), dim3(16 * NS), 0, st, d0, descs, ndesc);
+    {
+      if constexpr (NS <= 32)
+      {
+        if (hex)
+          return descs ? run(k_apply_box<P, T, NS, true, false, true>) : run(k_apply_box<P, T, NS, false, false, true>);
+      }
+      if (descs)
+        run(k_apply_box<P, T, NS, true, false, false>);
+      else if (d0.resid)
+        run(k_apply_box<P, T, NS, false, true, false>);
+      else
+        run(k_apply_box<P, T, NS, false, false, false>);
+    }
   };
   auto by_ns = [&](auto pc) {
     if (ns == 16)
@@ -685,11 +969,13 @@ apply_box(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, i
     else
       go(pc, std::integral_constant<int, 64>{});
   };
+  // residuals are formed for multigrid and tables of several orders for batches
+  // of box meshes only
+  if ((hex && (ns > 32 || d0.resid || p == 0)) || (p == 0 && !descs))
+    return hipErrorInvalidValue;
   switch (p)
   {
   case 0:
-    if (!descs)
-      return hipErrorInvalidValue;
     by_ns(std::integral_constant<int, 0>{});
     break;
   case 1:
@@ -707,7 +993,7 @@ apply_box(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, i
   return hipGetLastError();
 }
 
-template hipError_t apply_box<double>(const ApplyDesc &, const ApplyDesc *, int, int, int, int, hipStream_t);
-template hipError_t apply_box<float>(const ApplyDesc &, const ApplyDesc *, int, int, int, int, hipStream_t);
+template hipError_t apply_box<double>(const ApplyDesc &, const ApplyDesc *, int, int, int, int, bool, hipStream_t);
+template hipError_t apply_box<float>(const ApplyDesc &, const ApplyDesc *, int, int, int, int, bool, hipStream_t);
 
 } // namespace hc

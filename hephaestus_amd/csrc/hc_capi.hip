@@ -314,15 +314,23 @@ try
       return rc;
     }
   }
-  if (op->box)
+  // element factors of the box apply and of its trilinear form
+  if (hc::box_fits(g))
   {
-    // element factors: J = diag(h), |det J| = h0 h1 h2
-    if (hc::box_fits(g) && ((rc = op->alloc(op->qc64, 2 * op->E)) || (op->qd32 && (rc = op->alloc(op->qc32, 2 * op->E)))))
+    // FP32 vectors on trilinear meshes: the arithmetic is FP64 either way, which
+    // pays at order 1 only (64^3 77 -> 36 us; order 2 40^3 54 -> 63 us, order 3
+    // 32^3 51 -> 61 us against FP32 sums over the stored factors)
+    const bool f32 = op->qd32 && (op->box || op->p == 1);
+    if ((rc = op->alloc(op->qc64, 2 * op->E)) || (f32 && (rc = op->alloc(op->qc32, 2 * op->E))))
     {
       delete op;
       return rc;
     }
-    op->box_one = hc::box_tile(g, 1);
+    op->box_one = hc::box_tile(g, 1, 0, !op->box);
+  }
+  if (op->box)
+  {
+    // J = diag(h), |det J| = h0 h1 h2
     const double det = op->h[0] * (op->h[1] * op->h[2]);
     for (int a = 0; a < 3; a++)
     {
@@ -398,11 +406,11 @@ try
   // element factors of a box mesh; sigma h^2 / nu per element (block minima)
   if (op->qc64)
     HC_TRY_HIP(hc::elem_factors(op->E, op->d_nu, op->d_sig, dt, op->ck, op->mk, op->qc64, op->qc32, op->d_ratio, st));
-  else
+  if (!op->qc64 || !op->box) // (overwrites the minima above, which are those of boxes)
     HC_TRY_HIP(hc::term_ratio_blocks(op->qd64, op->E, op->p, op->d_ratio, st));
   // Jacobi diagonal, and the node diagonal of the gradient-space correction
   // (in closed form on box meshes, whatever storage the apply reads)
-  if (op->qc64 && (int64_t)op->g.n[2] * op->p + 1 < 65536)
+  if (op->box && op->qc64 && (int64_t)op->g.n[2] * op->p + 1 < 65536)
   {
     hc::ElemFactors ef;
     ef.qc = op->qc64;
@@ -604,7 +612,7 @@ try
 {
   if (!op)
     return fail(HC_EINVAL, "hc_op_factor_mode: null handle");
-  return op->ef(false).qc ? 1 : 0;
+  return op->box && op->ef(false).qc ? 1 : 0;
 }
 catch (...)
 {
@@ -880,8 +888,8 @@ try
   {
     HC_TRY_HIP(hipEventRecord(ev[3 * r], st));
     if (box)
-      HC_TRY_HIP(f32 ? hc::apply_box<float>(d, nullptr, 1, d.ntiles, pl.g.p, d.bt.ns, st)
-                     : hc::apply_box<double>(d, nullptr, 1, d.ntiles, pl.g.p, d.bt.ns, st));
+      HC_TRY_HIP(f32 ? hc::apply_box<float>(d, nullptr, 1, d.ntiles, pl.g.p, d.bt.ns, d.ef.vert != nullptr, st)
+                     : hc::apply_box<double>(d, nullptr, 1, d.ntiles, pl.g.p, d.bt.ns, d.ef.vert != nullptr, st));
     else
       HC_TRY_HIP(pl.cand->launch(d, nullptr, 1, d.ntiles, 0, tb, prec_bits, st));
     HC_TRY_HIP(hipEventRecord(ev[3 * r + 1], st));

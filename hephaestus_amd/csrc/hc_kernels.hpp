@@ -53,6 +53,7 @@ struct ElemFactors
   const void * qc = nullptr;
   double ck[3] = {0, 0, 0};
   double mk[3] = {0, 0, 0};
+  const double * vert = nullptr; // trilinear mesh: its vertices (x fastest), else null
   const BoxTile * one = nullptr; // host: the operator's decomposition for one vector
 };
 
@@ -270,10 +271,10 @@ hipError_t apply_op(const Geom & g,
 // common to the launch; p = 0: a table of instances of any orders), and its decomposition of a mesh for nrhs vectors
 // (ns_only: with that many slots).  The results do not depend on it.
 template <typename T>
-hipError_t apply_box(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, int p, int ns,
+hipError_t apply_box(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, int p, int ns, bool hex,
                      hipStream_t st);
 bool box_fits(const Geom & g); // (32-bit offsets within a plane)
-BoxTile box_tile(const Geom & g, int nrhs, int ns_only = 0);
+BoxTile box_tile(const Geom & g, int nrhs, int ns_only, bool hex);
 inline void
 set_box_tile(ApplyDesc & d, const BoxTile & b)
 {
@@ -283,7 +284,7 @@ set_box_tile(ApplyDesc & d, const BoxTile & b)
 inline void
 set_box_tile(ApplyDesc & d, int nrhs)
 {
-  set_box_tile(d, nrhs == 1 && d.ef.one ? *d.ef.one : box_tile(d.g, nrhs));
+  set_box_tile(d, nrhs == 1 && d.ef.one ? *d.ef.one : box_tile(d.g, nrhs, 0, d.ef.vert != nullptr));
 }
 // Right-hand sides per work item for a batch of nrhs on ntiles tiles.
 int default_rhs_block(int ntiles, int nrhs);

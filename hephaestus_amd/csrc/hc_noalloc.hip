@@ -125,7 +125,7 @@ try
   if (d.ef.qc)
   {
     hc::set_box_tile(d, 1);
-    HC_TRY_HIP(hc::apply_box<double>(d, nullptr, 1, d.ntiles, pl.g.p, d.bt.ns, st));
+    HC_TRY_HIP(hc::apply_box<double>(d, nullptr, 1, d.ntiles, pl.g.p, d.bt.ns, d.ef.vert != nullptr, st));
     return HC_OK;
   }
   HC_TRY_HIP(pl.cand->launch(d, nullptr, 1, d.ntiles, 0, &op->tb64, 64, st));

@@ -187,10 +187,11 @@ struct hc_op_s
   hc::ElemFactors ef(bool f32) const
   {
     hc::ElemFactors f;
-    if (ef_mode && qc64)
+    if (ef_mode && (f32 ? qc32 != nullptr : qc64 != nullptr))
     {
       f.qc = f32 ? (const void *)qc32 : (const void *)qc64;
       f.one = &box_one;
+      f.vert = box ? nullptr : d_vert;
       for (int a = 0; a < 3; a++)
       {
         f.ck[a] = ck[a];
@@ -344,6 +345,7 @@ private:
     const ApplyDesc * descs; // device
     int ndesc, nwork, npwork;
     int grouped; // some instance groups rb > 1 right-hand sides per work item
+    bool hex;    // (with box_ns) trilinear meshes
     int box_ns;  // every instance reads element factors: slots of the box apply (0: tile kernels)
     const TileCandidate * cand;
     const void * tables; // Tables<double> or Tables<float>

@@ -257,7 +257,7 @@ Engine::set(const std::vector<EngineInst> & inst, int mode, int rhs_block, bool 
         if (prec32 ? may32 : (k != K_PQ64 || !may32 || inst_[i].fp64))
         {
           members[p].push_back(i);
-          all_box = all_box && inst_[i].op->ef(prec32).qc;
+          all_box = all_box && inst_[i].op->ef(prec32).qc && inst_[i].op->box;
         }
       }
       orders += !members[p].empty();
@@ -296,7 +296,7 @@ Engine::set(const std::vector<EngineInst> & inst, int mode, int rhs_block, bool 
       for (int i : ids)
       {
         const hc_op_s * op = inst_[i].op;
-        all_ef = all_ef && op->ef(prec32).qc;
+        all_ef = all_ef && op->ef(prec32).qc && op->box == op0->box;
         work += op->N * inst_[i].nrhs;
         if (op->N > big)
         {
@@ -305,7 +305,8 @@ Engine::set(const std::vector<EngineInst> & inst, int mode, int rhs_block, bool 
         }
       }
       auto vecs = [&](const hc_op_s * op) { return (int)std::min<int64_t>((work + op->N / 2) / op->N, 4096); };
-      G.box_ns = all_ef ? box_tile(opb->g, vecs(opb)).ns : 0;
+      G.hex = !op0->box;
+      G.box_ns = all_ef ? box_tile(opb->g, vecs(opb), 0, G.hex).ns : 0;
       for (int i : ids)
       {
         const EngineInst & e = inst_[i];
@@ -316,7 +317,7 @@ Engine::set(const std::vector<EngineInst> & inst, int mode, int rhs_block, bool 
         d.prows = (int)d.segs.start[d.segs.nseg];
         d.ntiles = d.g.nt[0] * d.g.nt[1] * d.g.nt[2];
         if (all_ef)
-          set_box_tile(d, box_tile(d.g, vecs(op), G.box_ns));
+          set_box_tile(d, box_tile(d.g, vecs(op), G.box_ns, G.hex));
         d.nrhs = e.nrhs;
         d.rb = G.batched ? (rhs_block > 0 ? std::min(rhs_block, e.nrhs) : default_rhs_block(d.ntiles, e.nrhs)) : 1;
         d.qd = prec32 ? (const void *)op->qd32 : (const void *)op->qd64;
@@ -389,8 +390,8 @@ Engine::apply(Kind k, hipStream_t st)
     if (G.box_ns)
     {
       const ApplyDesc * descs = G.batched ? G.descs : nullptr;
-      e = G.prec == 64 ? apply_box<double>(G.single, descs, G.ndesc, G.nwork, G.order, G.box_ns, st)
-                       : apply_box<float>(G.single, descs, G.ndesc, G.nwork, G.order, G.box_ns, st);
+      e = G.prec == 64 ? apply_box<double>(G.single, descs, G.ndesc, G.nwork, G.order, G.box_ns, G.hex, st)
+                       : apply_box<float>(G.single, descs, G.ndesc, G.nwork, G.order, G.box_ns, G.hex, st);
     }
     else if (G.batched)
       e = G.prec == 64 ? apply_multi<double>(G.cand, *(const Tables<double> *)G.tables, G.descs, G.ndesc, G.nwork,

@@ -182,13 +182,15 @@ int hc_op_term_ratio(hc_op_t op, double * ratio);
  * factors per element, dt nu_e and sigma_e, and contracts with the exact 1-D
  * matrices that the quadrature reduces to (J = diag(h)); its arithmetic is
  * FP64 whatever the precision of the vectors, its results do not depend on
- * a tile shape, and the tile variant (hc_op_set_tile) is not used.  Other
- * meshes read the 12 (p+1)^3 quadrature-point factors per element of the
- * partial assembly.  mode 0: the quadrature-point factors on every mesh.
- * The two agree to round-off.  No counterpart
- * in the reference (MFEM's partial assembly stores the quadrature-point
- * factors).  hc_op_factor_mode: the storage the kernels read (0 or 1) or a
- * negative status. */
+ * a tile shape, and the tile variant (hc_op_set_tile) is not used.  On a
+ * trilinear mesh products with FP64 vectors (at order 1 FP32 ones too) are
+ * formed the same way, with the quadrature-point factors taken from the
+ * vertices as they are needed; what else reads factors, and the set-up, uses
+ * the 12 (p+1)^3 stored per element by the partial assembly.  mode 0: the
+ * stored quadrature-point factors in every product.  The two agree to
+ * round-off.  No counterpart in the reference (MFEM's partial assembly stores
+ * the quadrature-point factors).  hc_op_factor_mode: 1 if products read element
+ * factors only (a box mesh in mode 1), else 0, or a negative status. */
 int hc_op_set_factor_mode(hc_op_t op, int mode);
 int hc_op_factor_mode(hc_op_t op);
 
@@ -288,8 +290,8 @@ int hc_tile_list(int order, int * out, int max);
 int hc_op_get_tile(hc_op_t op, int prec_bits, int * tx, int * ty, int * tz, int * mode);
 /* Autotuner: times every compiled tile variant on this operator (after
  * hc_op_setup), `reps` applies each, and keeps the fastest per precision.
- * With element factors (hc_op_set_factor_mode 1 on a box mesh) there is
- * nothing to choose: the apply is timed and the variant kept.
+ * Where the apply takes element factors (hc_op_set_factor_mode 1) there is
+ * nothing to choose: it is timed and the variant kept.
  * best_us (optional, 2 entries): the winning FP64 / FP32 apply times.
  * No reference counterpart (the reference applies a CSR matrix). */
 int hc_op_autotune(hc_op_t op, int reps, double * best_us, void * stream);
@@ -437,7 +439,7 @@ int hc_fill_uniform(hc_op_t op, uint64_t seed, double * v, int64_t n, void * str
 /* Timing of `reps` single-RHS applies y = A x (prec_bits 64 or 32, x/y of
  * that precision) with HIP events around each kernel on `stream`: out_us[0] =
  * mean duration of the tile kernel, out_us[1] = of the tile-face assembly
- * kernel (element factors: the whole apply, and zero).  No reference
+ * kernel (applies from element factors, one launch: the whole, and zero).  No reference
  * counterpart (measurement entry point). */
 int hc_op_profile_apply(hc_op_t op, int prec_bits, const void * x, void * y, int reps, double * out_us,
                         void * stream);

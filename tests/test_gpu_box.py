@@ -87,3 +87,69 @@ def test_box_diagonals(env, p, n, pec):
     assert abs(box.term_ratio / ref.term_ratio - 1.0) <= 1e-13
     box.close()
     ref.close()
+
+
+@pytest.mark.parametrize("p", [1, 2, 3])
+@pytest.mark.parametrize("n", [(1, 1, 1), (2, 1, 3), (1, 1, 40), (4, 4, 4), (5, 7, 9), (8, 9, 17), (65, 1, 2), (9, 23, 5), (33, 26, 11)])
+def test_hex_apply_edges(env, p, n):
+    """The trilinear form of the box apply, which takes the point factors from
+    the vertices, against the stored factors: distorted elements (vertices moved
+    by up to 0.15 of an edge), also with the x axis reversed (negative
+    determinants).  The point factors are sums of products of Jacobian entries
+    with at most a few digits of cancellation on both sides: 4e-14."""
+    torch, H = env
+    import numpy as np
+    pec = (0x3F, 0x19, 0x00, 0x26)[sum(n) % 4]
+    print(f"case hex edges p={p} n={n} pec={pec:#x}", flush=True)
+    rng = np.random.default_rng(sum(n) + p)
+    E = n[0] * n[1] * n[2]
+    nu, sig = rng.uniform(0.5, 1.5, E), 10.0 ** rng.uniform(0, 2, E)
+    L = (1.0 if n[1] % 2 else -1.0, 0.7, 1.3)
+    Z, Y, X = np.meshgrid(*[L[a] * np.arange(n[a] + 1) / n[a] for a in (2, 1, 0)], indexing="ij")
+    h = np.array([abs(L[a]) / n[a] for a in range(3)])
+    vert = np.stack([X, Y, Z], -1).reshape(-1, 3) + 0.15 * h * rng.uniform(-1, 1, (X.size, 3))
+    op = H.Operator(n, p, nu, sig, pec_faces=pec, vert=vert).setup(0.37)
+    X = torch.from_numpy(rng.uniform(-1, 1, (5, op.ndofs))).cuda()
+    Y = op.apply(X)
+    y32 = op.apply_f32(X.float())
+    k = op.apply_curl(X[0].contiguous())
+    for r in range(5):
+        assert torch.equal(op.apply(X[r].contiguous()), Y[r]), r
+        assert torch.equal(op.apply_f32(X[r].float().contiguous()), y32[r]), r
+    op.set_factor_mode(0)
+    Yq, kq = op.apply(X), op.apply_curl(X[0].contiguous())
+    assert float((Y - Yq).norm()) <= 4e-14 * float(Yq.norm())
+    assert float((k - kq).norm()) <= 4e-14 * float(kq.norm())
+    assert float((y32.double() - Yq).norm()) <= 4e-7 * float(Yq.norm())
+    op.close()
+
+
+@pytest.mark.parametrize("p", [1, 2, 3])
+def test_hex_table(env, p):
+    """Trilinear instances of one order in one launch of a batch, with several
+    right-hand sides: every column reaches the asked residual of the operator on
+    stored factors (the factor 1.05 covers the difference of the recurred from
+    the true residual and of the two products)."""
+    torch, H = env
+    import numpy as np
+    print(f"case hex table p={p}", flush=True)
+    rng = np.random.default_rng(p)
+    bt, ops, bs, xs = H.Batch(), [], [], []
+    for n in ((3, 5, 4), (9, 2, 6)):
+        Z, Y, X = np.meshgrid(*[np.arange(n[a] + 1) / n[a] for a in (2, 1, 0)], indexing="ij")
+        vert = np.stack([X, Y, Z], -1).reshape(-1, 3) + 0.1 * rng.uniform(-1, 1, (X.size, 3)) / max(n)
+        E = n[0] * n[1] * n[2]
+        op = H.Operator(n, p, rng.uniform(0.5, 2.0, E), rng.uniform(0.5, 2.0, E), vert=vert).setup(1.0)
+        ops.append(op)
+        bs.append(torch.stack([op.rhs_coil(7 * r + p) for r in range(3)]))
+        xs.append(torch.zeros_like(bs[-1]))
+        bt.add(op, bs[-1], xs[-1], rtol=1e-10, maxit=5000)
+    _, st = bt.solve(mode=H.SOLVE_FP64)
+    assert all(s["converged"] for s in st), st
+    for op, b, x in zip(ops, bs, xs):
+        op.set_factor_mode(0)
+        r = b - op.apply(x)
+        assert bool((r.norm(dim=1) <= 1.05e-10 * b.norm(dim=1)).all())
+    bt.close()
+    for op in ops:
+        op.close()
