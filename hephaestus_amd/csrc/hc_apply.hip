@@ -1004,7 +1004,7 @@ apply_op(const Geom & g, const PlaneSegs & segs, const Tables<T> & tb, const T *
   {
     // box mesh: one launch, results independent of rb (one rhs per work item)
     set_box_tile(d, nrhs);
-    return apply_box<T>(d, nullptr, 1, d.ntiles * nrhs, g.p, d.bt.ns, ef.vert != nullptr, st);
+    return apply_box<T>(d, nullptr, 1, d.ntiles * nrhs, g.p, d.bt.ns, ef.vert != nullptr, st, resid_b ? BOX_RESID : BOX_APPLY);
   }
   if (rb > 1 && nrhs > 1)
   {
@@ -1026,8 +1026,11 @@ template <typename T>
 hipError_t
 apply_scaled(const Geom & g, const PlaneSegs & segs, const Tables<T> & tb, const T * qd, const ElemFactors & ef,
              const T * x, T * y, T * part, double mscale, double cscale, const TileCandidate * cand,
-             ApplyDesc * desc_dev, hipStream_t st)
+             ApplyDesc * desc_dev, hipStream_t st, bool add)
 {
+  const bool box = ef.qc && !ef.vert;
+  if (add && !box)
+    return hipErrorInvalidValue;
   ApplyDesc d{};
   d.g = g;
   d.segs = segs;
@@ -1045,7 +1048,9 @@ apply_scaled(const Geom & g, const PlaneSegs & segs, const Tables<T> & tb, const
   if (ef.qc)
   {
     set_box_tile(d, 1);
-    return apply_box<T>(d, nullptr, 1, d.ntiles, g.p, d.bt.ns, ef.vert != nullptr, st);
+    d.resid = add ? y : nullptr;
+    const BoxKind kind = add ? BOX_ADD : (box && cscale == 0.0 && sizeof(T) == 8 ? BOX_MASS : BOX_APPLY);
+    return apply_box<T>(d, nullptr, 1, d.ntiles, g.p, d.bt.ns, ef.vert != nullptr, st, kind);
   }
   // term weights are honoured by the batched kernel (descriptor in device memory)
   hipError_t e = hipMemcpyAsync(desc_dev, &d, sizeof(d), hipMemcpyHostToDevice, st);
@@ -1058,7 +1063,7 @@ apply_scaled(const Geom & g, const PlaneSegs & segs, const Tables<T> & tb, const
 }
 template hipError_t apply_scaled<double>(const Geom &, const PlaneSegs &, const Tables<double> &, const double *,
                                          const ElemFactors &, const double *, double *, double *, double, double,
-                                         const TileCandidate *, ApplyDesc *, hipStream_t);
+                                         const TileCandidate *, ApplyDesc *, hipStream_t, bool);
 
 int
 default_rhs_block(int ntiles, int nrhs)

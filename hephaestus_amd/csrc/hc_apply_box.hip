@@ -58,6 +58,10 @@
 // 40 meshes of 6x5x4 to 44x34x20: 9.1e-16 -> 7.2e-16 in the mean (the stored
 // factors take the Jacobian from sums of coordinates, here from differences).
 //
+// The mass term alone (BOX_MASS: 10 matrix products a layer instead of 39 at
+// order 2) and the product added to y (BOX_ADD) save the A-V block operator the
+// curl of its mass product and its closing pass: 31x37x29 order 2 59 -> 47 us.
+//
 // Measured on boxes at 48^3 order 3 (9.08 M DOFs): 194 us per FP64 apply with the
 // LDS-staged tile kernel and its face assembly, 69 us here (FP32 vectors: 114
 // and 60 us).  Memory traffic is 164 MB (147 MB algorithmic, 30 us at the copy
@@ -224,7 +228,7 @@ plane_geom(const double * v, double a, double b)
 }
 
 // The right-hand sides [r_begin, r_end) of tile `tile` of one instance.
-template <int P, typename T, int NS, bool TABLE, bool RES, bool HEX>
+template <int P, typename T, int NS, bool TABLE, int KIND, bool HEX>
 __device__ __forceinline__ void
 box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
 {
@@ -598,6 +602,26 @@ box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
           yz[k] = mm(b, bGc, mm(a, bBc, 0.0));
         }
       }
+      else if constexpr (KIND == BOX_MASS)
+      {
+        const double kmx = mk0 * (sgN * wf), kmy = mk1 * (sgT * wf), kmz = mk2 * sgN;
+#pragma unroll
+        for (int q = 0; q < P; q++)
+          yz[q] = tb.w[q] * mm(mm(kmz * uz[q], opM, 0.0), opM, 0.0);
+#pragma unroll
+        for (int k = 0; k <= P; k++)
+        {
+          double mx = 0.0, my = 0.0;
+#pragma unroll
+          for (int m = 0; m <= P; m++)
+          {
+            mx = __builtin_fma(tb.M[k][m], ux[m], mx);
+            my = __builtin_fma(tb.M[k][m], uy[m], my);
+          }
+          yx[k] = mm(opM, kmx * mx, 0.0);
+          yy[k] = mm(kmy * my, opM, 0.0);
+        }
+      }
       else
       {
         // In phases (the scheduler keeps to them: the order holds the number of
@@ -738,7 +762,7 @@ box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
         }
       }
       T rbx[P], rby[P], rbz[P];
-      if constexpr (RES)
+      if constexpr (KIND == BOX_RESID || KIND == BOX_ADD)
       {
         const T * bv = (const T *)ad.resid + rof;
 #pragma unroll
@@ -758,6 +782,16 @@ box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
         yy[k] += sY[buf][k][rL];
         yz[k] = ((yz[k] + sZC[buf][k][rL]) + sZR[buf][k][rD]) + sZR[buf][k][rB];
       }
+      if constexpr (KIND == BOX_ADD)
+      {
+#pragma unroll
+        for (int k = 0; k < P; k++)
+        {
+          yx[k] = (double)rbx[k] + yx[k];
+          yy[k] = (double)rby[k] + yy[k];
+          yz[k] = (double)rbz[k] + yz[k];
+        }
+      }
       // PEC DOFs: y = x
       if (stash)
       {
@@ -773,7 +807,7 @@ box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
           yz[k] = essz ? vz : yz[k];
         }
       }
-      if constexpr (RES)
+      if constexpr (KIND == BOX_RESID)
       {
 #pragma unroll
         for (int k = 0; k < P; k++)
@@ -807,9 +841,15 @@ box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
       T * yv = (T *)ad.y + rof;
       const uint32_t isx = ownx ? oxN : OOB, isy = owny ? oyN : OOB;
       const T vx = ldb(xv + bx, isx), vy = ldb(xv + by, isy);
+      if constexpr (KIND == BOX_ADD)
+      {
+        const T * bv = (const T *)ad.resid + rof;
+        carx = (double)ldb(bv + bx, isx) + carx;
+        cary = (double)ldb(bv + by, isy) + cary;
+      }
       carx = (essx || zf) ? (double)vx : carx;
       cary = (essy || zf) ? (double)vy : cary;
-      if constexpr (RES)
+      if constexpr (KIND == BOX_RESID)
       {
         const T * bv = (const T *)ad.resid + rof;
         carx = (double)ldb(bv + bx, isx) - carx;
@@ -825,7 +865,7 @@ box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
 
 // P = 0: the instances of the table may have any order (one launch, and the
 // small instances of one order run beside the large ones of another)
-template <int P, typename T, int NS, bool TABLE, bool RES, bool HEX>
+template <int P, typename T, int NS, bool TABLE, int KIND, bool HEX>
 __global__ void __launch_bounds__(16 * NS, HEX ? 2 : 4)
 k_apply_box(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc)
 {
@@ -844,14 +884,14 @@ k_apply_box(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc)
   if constexpr (P == 0)
   {
     if (ad.g.p == 1)
-      box_body<1, T, NS, TABLE, RES, HEX>(ad, tile, r_begin, r_end, lds);
+      box_body<1, T, NS, TABLE, KIND, HEX>(ad, tile, r_begin, r_end, lds);
     else if (ad.g.p == 2)
-      box_body<2, T, NS, TABLE, RES, HEX>(ad, tile, r_begin, r_end, lds);
+      box_body<2, T, NS, TABLE, KIND, HEX>(ad, tile, r_begin, r_end, lds);
     else
-      box_body<3, T, NS, TABLE, RES, HEX>(ad, tile, r_begin, r_end, lds);
+      box_body<3, T, NS, TABLE, KIND, HEX>(ad, tile, r_begin, r_end, lds);
   }
   else
-    box_body<P, T, NS, TABLE, RES, HEX>(ad, tile, r_begin, r_end, lds);
+    box_body<P, T, NS, TABLE, KIND, HEX>(ad, tile, r_begin, r_end, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -935,7 +975,7 @@ box_fits(const Geom & g)
 
 template <typename T>
 hipError_t
-apply_box(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, int p, int ns, bool hex, hipStream_t st)
+apply_box(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, int p, int ns, bool hex, hipStream_t st, BoxKind kind)
 {
   if (nwork <= 0)
     return hipSuccess;
@@ -945,20 +985,26 @@ apply_box(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, i
     const dim3 blk(16 * NS);
     auto run = [&](auto kern) { hipLaunchKernelGGL(kern, grid, blk, 0, st, d0, descs, ndesc); };
     if constexpr (P == 0)
-      run(k_apply_box<0, T, NS, true, false, false>);
+      run(k_apply_box<0, T, NS, true, BOX_APPLY, false>);
     else
     {
       if constexpr (NS <= 32)
       {
         if (hex)
-          return descs ? run(k_apply_box<P, T, NS, true, false, true>) : run(k_apply_box<P, T, NS, false, false, true>);
+          return descs ? run(k_apply_box<P, T, NS, true, BOX_APPLY, true>) : run(k_apply_box<P, T, NS, false, BOX_APPLY, true>);
       }
       if (descs)
-        run(k_apply_box<P, T, NS, true, false, false>);
-      else if (d0.resid)
-        run(k_apply_box<P, T, NS, false, true, false>);
-      else
-        run(k_apply_box<P, T, NS, false, false, false>);
+        return run(k_apply_box<P, T, NS, true, BOX_APPLY, false>);
+      if constexpr (sizeof(T) == 8)
+      {
+        if (kind == BOX_ADD)
+          return run(k_apply_box<P, T, NS, false, BOX_ADD, false>);
+        if (kind == BOX_MASS)
+          return run(k_apply_box<P, T, NS, false, BOX_MASS, false>);
+      }
+      if (kind == BOX_RESID)
+        return run(k_apply_box<P, T, NS, false, BOX_RESID, false>);
+      run(k_apply_box<P, T, NS, false, BOX_APPLY, false>);
     }
   };
   auto by_ns = [&](auto pc) {
@@ -971,7 +1017,9 @@ apply_box(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, i
   };
   // residuals are formed for multigrid and tables of several orders for batches
   // of box meshes only
-  if ((hex && (ns > 32 || d0.resid || p == 0)) || (p == 0 && !descs))
+  const bool with_y = kind == BOX_RESID || kind == BOX_ADD;
+  if ((hex && (ns > 32 || kind != BOX_APPLY || p == 0)) || (p == 0 && !descs) || (descs && kind != BOX_APPLY) ||
+      (sizeof(T) != 8 && (kind == BOX_ADD || kind == BOX_MASS)) || (!descs && with_y != (d0.resid != nullptr)))
     return hipErrorInvalidValue;
   switch (p)
   {
@@ -993,7 +1041,7 @@ apply_box(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, i
   return hipGetLastError();
 }
 
-template hipError_t apply_box<double>(const ApplyDesc &, const ApplyDesc *, int, int, int, int, bool, hipStream_t);
-template hipError_t apply_box<float>(const ApplyDesc &, const ApplyDesc *, int, int, int, int, bool, hipStream_t);
+template hipError_t apply_box<double>(const ApplyDesc &, const ApplyDesc *, int, int, int, int, bool, hipStream_t, BoxKind);
+template hipError_t apply_box<float>(const ApplyDesc &, const ApplyDesc *, int, int, int, int, bool, hipStream_t, BoxKind);
 
 } // namespace hc

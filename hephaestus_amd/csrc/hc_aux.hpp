@@ -282,7 +282,8 @@ constexpr double FP32_MIN_TERM_RATIO = 6.0e-6;
 // s = a0 + G v with a0 = a zeroed on the PEC DOFs of g (all ND DOFs).
 hipError_t av_gather(const Geom & g, const AuxGeom & a, const double * av, const double * v, double * s,
                      hipStream_t st);
-// ya = ya + k on the free DOFs, ya = a on the PEC DOFs of g.
+// ya = ya + k on the free DOFs, ya = a on the PEC DOFs of g (where the product
+// itself does not add: stored factors, trilinear meshes).
 hipError_t av_finish(const Geom & g, const AuxGeom & a, const double * av, const double * k, double * ya,
                      hipStream_t st);
 // y = G v on every ND DOF.

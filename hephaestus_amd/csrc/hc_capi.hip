@@ -567,7 +567,15 @@ try
   HC_TRY_HIP(hc::apply_scaled<double>(g0, pl.segs, op->tb64, op->qd64, op->ef(false), s, ya, op->ws.part64, 1.0, 0.0, pl.cand,
                                       op->desc_dev, st));
   HC_TRY_HIP(hc::grad_transpose(op->ag, ya, yv, st));
-  // k = dt K a0 on the free DOFs (the quadrature data hold dt nu); ya += k there, ya = a on PEC DOFs
+  // ya += dt K a0 on the free DOFs (the factors hold dt nu), ya = a on PEC DOFs: on
+  // box meshes in the product itself (31x37x29 order 2: 59 -> 47 us with the
+  // mass-only form of the first one), else through k
+  if (op->box && op->ef(false).qc)
+  {
+    HC_TRY_HIP(hc::apply_scaled<double>(pl.g, pl.segs, op->tb64, op->qd64, op->ef(false), a, ya, op->ws.part64, 0.0, 1.0, pl.cand,
+                                        op->desc_dev, st, true));
+    return HC_OK;
+  }
   HC_TRY_HIP(hc::apply_scaled<double>(pl.g, pl.segs, op->tb64, op->qd64, op->ef(false), a, k, op->ws.part64, 0.0, 1.0, pl.cand,
                                       op->desc_dev, st));
   HC_TRY_HIP(hc::av_finish(pl.g, op->ag, a, k, ya, st));

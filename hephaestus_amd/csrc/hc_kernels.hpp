@@ -268,11 +268,22 @@ hipError_t apply_op(const Geom & g,
                     ApplyDesc * desc_dev = nullptr,
                     const T * resid_b = nullptr);
 // The box apply (every instance reads element factors; ApplyDesc::bt set, ns
-// common to the launch; p = 0: a table of instances of any orders), and its decomposition of a mesh for nrhs vectors
-// (ns_only: with that many slots).  The results do not depend on it.
+// common to the launch; p = 0: a table of instances of any orders), and its
+// decomposition of a mesh for nrhs vectors (ns_only: with that many slots).  The
+// results do not depend on it.  Forms of one instance (box meshes):
+//   BOX_RESID  y = b - A x with b = ApplyDesc::resid (on PEC DOFs b - x)
+//   BOX_ADD    y = y + A x with resid = y, PEC DOFs y = x (FP64)
+//   BOX_MASS   the mass term alone, cscale taken as 0 (FP64)
+enum BoxKind
+{
+  BOX_APPLY,
+  BOX_RESID,
+  BOX_ADD,
+  BOX_MASS
+};
 template <typename T>
 hipError_t apply_box(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, int p, int ns, bool hex,
-                     hipStream_t st);
+                     hipStream_t st, BoxKind kind = BOX_APPLY);
 bool box_fits(const Geom & g); // (32-bit offsets within a plane)
 BoxTile box_tile(const Geom & g, int nrhs, int ns_only, bool hex);
 inline void
@@ -290,11 +301,12 @@ set_box_tile(ApplyDesc & d, int nrhs)
 int default_rhs_block(int ntiles, int nrhs);
 // y = (mscale M + cscale K') x (K' = the curl part of the quadrature data,
 // i.e. dt K) with the batched kernel; its descriptor is staged in desc_dev.
-// part: 4 N scratch.
+// part: 4 N scratch.  add (FP64 on box meshes with element factors): the product
+// is added to y on the free DOFs, PEC DOFs take x.
 template <typename T>
 hipError_t apply_scaled(const Geom & g, const PlaneSegs & segs, const Tables<T> & tb, const T * qd,
                         const ElemFactors & ef, const T * x, T * y, T * part, double mscale, double cscale,
-                        const TileCandidate * cand, ApplyDesc * desc_dev, hipStream_t st);
+                        const TileCandidate * cand, ApplyDesc * desc_dev, hipStream_t st, bool add = false);
 
 // Fill the plane-assembly fields of a descriptor (segments, rows per rhs).
 void plane_rows(ApplyDesc & d);

@@ -153,3 +153,27 @@ def test_hex_table(env, p):
     bt.close()
     for op in ops:
         op.close()
+
+
+@pytest.mark.parametrize("p", [1, 2, 3])
+@pytest.mark.parametrize("n,pec", [((1, 1, 1), 0x3F), ((1, 1, 1), 0x00), ((2, 1, 3), 0x15), ((5, 4, 6), 0x2A), ((17, 9, 5), 0x3F),
+                                   ((8, 3, 41), 0x19)])
+def test_box_av_edges(env, p, n, pec):
+    """The mass-only and the adding form of the box apply, through the A-V block
+    operator, against the stored factors of the same operator (general product
+    and a sum afterwards).  Random inputs, no cancellation beyond that of a
+    difference of neighbours: 4e-14 as for a product."""
+    torch, H = env
+    import numpy as np
+    print(f"case box av p={p} n={n} pec={pec:#x}", flush=True)
+    rng = np.random.default_rng(3 * p + sum(n))
+    E = n[0] * n[1] * n[2]
+    op = H.Operator(n, p, rng.uniform(0.5, 2.0, E), 10.0 ** rng.uniform(-2, 2, E), pec_faces=pec, length=(1.0, 0.8, 1.4)).setup(0.3)
+    a = torch.from_numpy(rng.uniform(-1, 1, op.ndofs)).cuda()
+    v = torch.from_numpy(rng.uniform(-1, 1, op.nnodes)).cuda()
+    ya, yv = op.av_apply(a, v)
+    op.set_factor_mode(0)
+    ra, rv = op.av_apply(a, v)
+    assert float((ya - ra).norm()) <= 4e-14 * float(ra.norm())
+    assert float((yv - rv).norm()) <= 4e-14 * float(rv.norm())
+    op.close()
