@@ -1,4 +1,6 @@
-// Tiled sum-factorised apply of dt*nu K + sigma M on ND_p hexes (gfx950).
+// Tiled sum-factorised apply of dt*nu K + sigma M on ND_p hexes (gfx950) from
+// stored quadrature-point factors, and the choice between it and the box apply
+// (hc_apply_box.hip), which operators with element factors take.
 //
 // This is the operator EquationSystem::Mult (src/equation_systems/equation_system.cpp:200-204)
 // on the system formed by FormLinearSystem (equation_system.cpp:132-190): PEC
@@ -1002,7 +1004,7 @@ apply_op(const Geom & g, const PlaneSegs & segs, const Tables<T> & tb, const T *
   hipError_t e;
   if (ef.qc)
   {
-    // box mesh: one launch, results independent of rb (one rhs per work item)
+    // one launch, results independent of rb (one rhs per work item)
     set_box_tile(d, nrhs);
     return apply_box<T>(d, nullptr, 1, d.ntiles * nrhs, g.p, d.bt.ns, ef.vert != nullptr, st, resid_b ? BOX_RESID : BOX_APPLY);
   }
