@@ -167,7 +167,11 @@ make_box_lanes()
   return t;
 }
 // interpolation to the quadrature points (open, closed, derivative of closed),
-// [f][s] and [s][f]; the lane's point (f, s) and its weight
+// [f][s] and [s][f]; the lane's point (f, s) and its weight.  The lanes without
+// a point of their own (order 2) take the last one's with weight zero: their
+// determinant is then that of a quadrature point too, which is not zero where an
+// edge of the element is collapsed (a corner's is, and 0 / 0 would spread from
+// there through the matrix products).
 template <int P>
 constexpr LaneTab<10>
 make_hex_lanes()
@@ -179,6 +183,8 @@ make_hex_lanes()
     {
       const int pf = P == 1 ? f % 2 : f, ps = P == 1 ? s % 2 : s;
       double * v = t.v[f * 4 + s];
+      v[6] = b.qp[pf < P ? pf : P];
+      v[7] = b.qp[ps < P ? ps : P];
       if (pf > P || ps > P)
         continue;
       if (P > 1 || f / 2 == s / 2)
@@ -190,8 +196,6 @@ make_hex_lanes()
         v[4] = b.Bc[ps * (P + 1) + pf];
         v[5] = b.Gc[ps * (P + 1) + pf];
       }
-      v[6] = b.qp[pf];
-      v[7] = b.qp[ps];
       v[8] = b.qw[pf] * b.qw[ps];
     }
   return t;
