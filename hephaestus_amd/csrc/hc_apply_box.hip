@@ -231,6 +231,12 @@ plane_geom(const double * v, double a, double b)
   return g;
 }
 
+// dt nu and sigma of a lane's element in the N and the T layout
+struct Coef
+{
+  double nuN, sgN, nuT, sgT;
+};
+
 // The right-hand sides [r_begin, r_end) of tile `tile` of one instance.
 template <int P, typename T, int NS, bool TABLE, int KIND, bool HEX>
 __device__ __forceinline__ void
@@ -472,13 +478,36 @@ box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
       }
       ux[P] = ztop ? 0.0 : ux[P];
       uy[P] = ztop ? 0.0 : uy[P];
-      const double nuN = (double)nq[0], sgN = (double)nq[1];
-      const double nuT = (P == 1 && !HEX) ? (double)nq[P == 1 ? 2 : 0] : nuN;
-      const double sgT = (P == 1 && !HEX) ? (double)nq[P == 1 ? 3 : 1] : sgN;
+      Coef cf;
+      cf.nuN = (double)nq[0];
+      cf.sgN = (double)nq[1];
+      cf.nuT = (P == 1 && !HEX) ? (double)nq[P == 1 ? 2 : 0] : cf.nuN;
+      cf.sgT = (P == 1 && !HEX) ? (double)nq[P == 1 ? 3 : 1] : cf.sgN;
       if (!HEX && z + 1 < z1)
         load_layer(bx + P * plx, by + P * ply, bz + P * plz, z + 1);
+      // upper vertex plane of the layer, and the difference along z at the lane's point
+      PlaneGeom g1;
+      double jz[3];
+      auto upper_plane = [&]() {
+        g1 = plane_geom(nv, qa, qb);
+#pragma unroll
+        for (int r = 0; r < 3; r++)
+          jz[r] = (nv[r] - nv[12 + r]) + (g1.p[r] - g0.p[r]);
+      };
+      if constexpr (HEX && P == 1)
+        upper_plane();
 
+      // the element products y = A_e u of the layer (first: with the loads of the
+      // next one in the trilinear form; lanes without `use` have no element)
       double yx[P + 1], yy[P + 1], yz[P];
+      auto products = [&](const double (&ux)[P + 1], const double (&uy)[P + 1], const double (&uz_)[P], const Coef & c, bool use,
+                          auto first) {
+      constexpr bool FIRST = decltype(first)::value;
+      const double nuN = c.nuN, sgN = c.sgN, nuT = c.nuT, sgT = c.sgT;
+      double uz[P];
+#pragma unroll
+      for (int k = 0; k < P; k++)
+        uz[k] = uz_[k];
       if constexpr (HEX)
       {
         auto phase = []() { __builtin_amdgcn_sched_barrier(0); };
@@ -503,11 +532,8 @@ box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
           uzy[k] = mm(b, fBc, 0.0);
         }
         phase();
-        const PlaneGeom g1 = plane_geom(nv, qa, qb);
-        double jz[3];
-#pragma unroll
-        for (int r = 0; r < 3; r++)
-          jz[r] = (nv[r] - nv[12 + r]) + (g1.p[r] - g0.p[r]);
+        if constexpr (P > 1)
+          upper_plane();
         const double sm0 = wxy * (sgN * msc), sc0 = wxy * (nuN * csc);
         // sums over the quadrature points along z of the transposed stage:
         // (value, y derivative) of x, (value, x derivative) of y, (value, x, y) of z
@@ -551,7 +577,7 @@ box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
           const double cr[3] = {__builtin_fma(jy[1], jz[2], -(jy[2] * jz[1])), __builtin_fma(jy[2], jz[0], -(jy[0] * jz[2])),
                                 __builtin_fma(jy[0], jz[1], -(jy[1] * jz[0]))};
           const double det = __builtin_fabs(dot(jx, cr));
-          const double rd = qt.qw[q] / (vN ? det : 1.0); // (lanes without a point carry zeros)
+          const double rd = qt.qw[q] / (use ? det : 1.0); // (lanes without a point carry zeros)
           const double sm = sm0 * rd, sc = sc0 * rd;
           const double A00 = __builtin_fma(G11, G22, -(G12 * G12)), A01 = __builtin_fma(G02, G12, -(G01 * G22));
           const double A02 = __builtin_fma(G01, G12, -(G02 * G11)), A11 = __builtin_fma(G00, G22, -(G02 * G02));
@@ -583,12 +609,16 @@ box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
           }
           phase();
         }
-        g0 = g1;
-        // (the last layer loads itself again: a branch here would let the
-        // compiler sink the points above past it and keep the loads alive there)
-        const int64_t zn = z + 1 < z1 ? P : 0;
-        load_layer(bx + zn * plx, by + zn * ply, bz + zn * plz, min(z + 1, z1 - 1));
-        load_corners(min(z + 2, z1), nv);
+        if constexpr (P > 1)
+          g0 = g1;
+        if constexpr (FIRST)
+        {
+          // (the last layer loads itself again: a branch here would let the
+          // compiler sink the points above past it and keep the loads alive there)
+          const int64_t zn = z + 1 < z1 ? P : 0;
+          load_layer(bx + zn * plx, by + zn * ply, bz + zn * plz, min(z + 1, z1 - 1));
+          load_corners(min(z + 2, z1), nv);
+        }
         phase();
         // transposed x, y stages
 #pragma unroll
@@ -727,6 +757,43 @@ box_body(const ApplyDesc & ad, int tile, int r_begin, int r_end, double * lds)
 #pragma unroll
         for (int k = 0; k <= P; k++)
           yy[k] = mm(yy[k], opM, ft[k]);
+      }
+      };
+      products(ux, uy, uz, cf, vN, std::true_type{});
+      if constexpr (P == 1)
+      {
+        // A block holds 2 x 2 elements at order 1, and a zero of the block-diagonal
+        // matrices times a value that is not finite is NaN for the elements beside
+        // the one that has it.  Such a layer is done again element by element, the
+        // others with zeros.  (The test and its registers: 64^3 18.3 -> 18.6 us,
+        // trilinear 37.0 -> 38.0; nothing up to 31x37x29.)
+        const bool finite = __builtin_isfinite(yx[0]) && __builtin_isfinite(yx[1]) && __builtin_isfinite(yy[0]) &&
+                            __builtin_isfinite(yy[1]) && __builtin_isfinite(yz[0]);
+        if (__any(!finite))
+        {
+          double rx[2] = {}, ry[2] = {}, rz = 0.0;
+#pragma unroll 1
+          for (int e = 0; e < 4; e++)
+          {
+            const bool inN = ef + 2 * es == e, inT = HEX ? inN : es + 2 * ef == e;
+            const double vx[2] = {inN ? ux[0] : 0.0, inN ? ux[1] : 0.0}, vy[2] = {inT ? uy[0] : 0.0, inT ? uy[1] : 0.0};
+            const double vz[1] = {inN ? uz[0] : 0.0};
+            const Coef ce{inN ? cf.nuN : 0.0, inN ? cf.sgN : 0.0, inT ? cf.nuT : 0.0, inT ? cf.sgT : 0.0};
+            products(vx, vy, vz, ce, vN && inN, std::false_type{});
+            rx[0] = inN ? yx[0] : rx[0];
+            rx[1] = inN ? yx[1] : rx[1];
+            ry[0] = inN ? yy[0] : ry[0];
+            ry[1] = inN ? yy[1] : ry[1];
+            rz = inN ? yz[0] : rz;
+          }
+          yx[0] = rx[0];
+          yx[1] = rx[1];
+          yy[0] = ry[0];
+          yy[1] = ry[1];
+          yz[0] = rz;
+        }
+        if constexpr (HEX)
+          g0 = g1;
       }
       yx[0] = yx[0] + carx;
       yy[0] = yy[0] + cary;

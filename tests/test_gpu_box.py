@@ -216,3 +216,39 @@ def test_hex_collapsed_edge(env, p, n, pec, axis):
         assert bool(torch.isfinite(y).all()), i
         assert float((y - r).norm()) <= 4e-14 * float(r.norm()), i
     op.close()
+
+
+@pytest.mark.parametrize("mesh", ["box", "hex"])
+@pytest.mark.parametrize("p", [1, 2, 3])
+def test_non_finite_entries_stay_in_their_elements(env, p, mesh):
+    """An entry of x that is not finite, or that overflows in the product, makes
+    outputs of the elements that hold it non-finite and no others: elsewhere the
+    bits are those of the product with a zero in its place."""
+    torch, H = env
+    import numpy as np
+    from brute import elem_gids
+    n = (5, 4, 6)
+    print(f"case non-finite p={p} {mesh}", flush=True)
+    rng = np.random.default_rng(p)
+    E = n[0] * n[1] * n[2]
+    vert = None
+    if mesh == "hex":
+        Z, Y, X = np.meshgrid(*[np.arange(n[a] + 1) / n[a] for a in (2, 1, 0)], indexing="ij")
+        vert = np.stack([X, Y, Z], -1).reshape(-1, 3) + 0.01 * rng.uniform(-1, 1, (X.size, 3))
+    op = H.Operator(n, p, rng.uniform(1e3, 2e3, E), rng.uniform(0.5, 2.0, E), pec_faces=0x13, vert=vert).setup(1.0)
+    gids = np.array([np.asarray(elem_gids(n, p, ex, ey, ez)) for ez in range(n[2]) for ey in range(n[1]) for ex in range(n[0])])
+    x = torch.from_numpy(rng.uniform(-1, 1, op.ndofs)).cuda()
+    per = p * (p + 1) ** 2
+    for (ex, ey, ez), loc in (((2, 1, 2), 0), ((1, 2, 3), per), ((3, 2, 0), 2 * per), ((3, 3, 5), 3 * per - 1)):
+        dof = int(gids[(ez * n[1] + ey) * n[0] + ex][loc])
+        away = torch.ones(op.ndofs, dtype=torch.bool, device="cuda")
+        away[torch.from_numpy(np.unique(gids[(gids == dof).any(1)])).cuda()] = False
+        for v in (float("nan"), float("inf"), 1.7e308):
+            x0, xv = x.clone(), x.clone()
+            x0[dof], xv[dof] = 0.0, v
+            for f in (op.apply, op.apply_curl, lambda t: op.apply_f32(t.float())):
+                y0, y = f(x0), f(xv)
+                assert bool(torch.isfinite(y0).all())
+                assert not bool(torch.isfinite(y).all())
+                assert torch.equal(y[away], y0[away]), (dof, v, int((~torch.isfinite(y[away])).sum()))
+    op.close()
