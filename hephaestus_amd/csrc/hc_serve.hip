@@ -9,9 +9,9 @@
 //     u_{n+1} = u_n + dt k.
 // A scheduler thread admits waiting requests as slots whenever their work
 // vectors fit in the device-memory budget (an arena carved once at creation),
-// advances every admitted slot in rounds of the batched solve engine (one
-// launch per ND order for the operator applies of all slots, one launch per
-// vector kernel), and retires finished slots at round boundaries, so requests
+// advances every admitted slot in rounds of the batched solve engine (a launch
+// or a few for the operator applies of all slots, one launch per vector
+// kernel), and retires finished slots at round boundaries, so requests
 // that arrive while others run join the running batch.  Each slot's
 // arithmetic does not depend on the other slots: a request's result is the
 // same alone and in any mix (same tile variant per order).

@@ -4,8 +4,10 @@
 // the C ABI entry points built on it (hc_pcg_solve, hc_batch_*).
 //
 // Every right-hand side of every instance is one solve slot (hc_pcg.hip); the
-// operator applies of one iteration are one launch per ND order over a device
-// table of instances (hc_apply.hip), each gated by the slots' done flags.
+// operator applies of one iteration are one launch over a device table for all
+// box instances on element factors and one per ND order for the trilinear ones
+// and for those on stored factors (hc_apply_box.hip, hc_apply.hip), each gated
+// by the slots' done flags.
 #include "hc_op.hpp"
 
 #include <chrono>
@@ -243,9 +245,18 @@ Engine::set(const std::vector<EngineInst> & inst, int mode, int rhs_block, bool 
     const bool prec32 = (k == K_PQ32);
     // the FP32 group holds the instances whose slots may run FP32 inner
     // solves (work items of the others would only be gated off)
-    std::vector<std::vector<int>> members(PMAX + 1);
-    bool all_box = true; // of every order: one launch of the box apply
-    int orders = 0;
+    // An instance's products read what they read alone, so that its results do
+    // not depend on the others: a launch takes the instances of one order that
+    // read stored factors, that are box meshes or that are trilinear ones.
+    enum
+    {
+      STORED,
+      BOX,
+      HEX,
+      KINDS
+    };
+    std::vector<int> members[KINDS][PMAX + 1];
+    int box_orders = 0;
     for (int p = 1; p <= PMAX; p++)
     {
       for (int i : by_order[p])
@@ -256,28 +267,29 @@ Engine::set(const std::vector<EngineInst> & inst, int mode, int rhs_block, bool 
         // continued in FP64 (the residual group K_XQ holds every instance)
         if (prec32 ? may32 : (k != K_PQ64 || !may32 || inst_[i].fp64))
         {
-          members[p].push_back(i);
-          all_box = all_box && inst_[i].op->ef(prec32).qc && inst_[i].op->box;
+          const hc_op_s * op = inst_[i].op;
+          members[!op->ef(prec32).qc ? STORED : (op->box ? BOX : HEX)][p].push_back(i);
         }
       }
-      orders += !members[p].empty();
+      box_orders += !members[BOX][p].empty();
     }
-    if (all_box && orders > 1)
+    if (box_orders > 1) // box meshes of every order: one launch
     {
       for (int p = 2; p <= PMAX; p++)
       {
-        members[1].insert(members[1].end(), members[p].begin(), members[p].end());
-        members[p].clear();
+        members[BOX][1].insert(members[BOX][1].end(), members[BOX][p].begin(), members[BOX][p].end());
+        members[BOX][p].clear();
       }
     }
-    for (int p = 1; p <= PMAX; p++)
+    for (int kp = 0; kp < KINDS * PMAX; kp++)
     {
-      const std::vector<int> & ids = members[p];
+      const int kind = kp / PMAX, p = kp % PMAX + 1;
+      const std::vector<int> & ids = members[kind][p];
       if (ids.empty())
         continue;
       const hc_op_s * op0 = inst_[ids[0]].op;
       ApplyGroup G{};
-      G.order = all_box && orders > 1 ? 0 : p;
+      G.order = kind == BOX && box_orders > 1 ? 0 : p;
       G.prec = prec32 ? 32 : 64;
       const TileCandidate * over = prec32 ? (cands32 ? cands32[p] : nullptr) : (cands64 ? cands64[p] : nullptr);
       G.cand = over ? over : (prec32 ? op0->plan32.cand : op0->plan64.cand);
@@ -287,16 +299,12 @@ Engine::set(const std::vector<EngineInst> & inst, int mode, int rhs_block, bool 
       G.ndesc = (int)ids.size();
       G.grouped = 0;
       int w0 = 0, pw0 = 0;
-      // every instance has element factors: one launch of the box apply;
-      // mixed: every instance reads its quadrature-point factors
-      // (decomposition: as if all the work were vectors of one instance)
-      bool all_ef = true;
+      // decomposition of the box apply: as if all the work were vectors of one instance
       int64_t work = 0, big = 0;
       const hc_op_s * opb = op0;
       for (int i : ids)
       {
         const hc_op_s * op = inst_[i].op;
-        all_ef = all_ef && op->ef(prec32).qc && op->box == op0->box;
         work += op->N * inst_[i].nrhs;
         if (op->N > big)
         {
@@ -305,8 +313,8 @@ Engine::set(const std::vector<EngineInst> & inst, int mode, int rhs_block, bool 
         }
       }
       auto vecs = [&](const hc_op_s * op) { return (int)std::min<int64_t>((work + op->N / 2) / op->N, 4096); };
-      G.hex = !op0->box;
-      G.box_ns = all_ef ? box_tile(opb->g, vecs(opb), 0, G.hex).ns : 0;
+      G.hex = kind == HEX;
+      G.box_ns = kind != STORED ? box_tile(opb->g, vecs(opb), 0, G.hex).ns : 0;
       for (int i : ids)
       {
         const EngineInst & e = inst_[i];
@@ -316,12 +324,12 @@ Engine::set(const std::vector<EngineInst> & inst, int mode, int rhs_block, bool 
         geom_for(op, G.cand, d.g, d.segs);
         d.prows = (int)d.segs.start[d.segs.nseg];
         d.ntiles = d.g.nt[0] * d.g.nt[1] * d.g.nt[2];
-        if (all_ef)
+        if (kind != STORED)
           set_box_tile(d, box_tile(d.g, vecs(op), G.box_ns, G.hex));
         d.nrhs = e.nrhs;
         d.rb = G.batched ? (rhs_block > 0 ? std::min(rhs_block, e.nrhs) : default_rhs_block(d.ntiles, e.nrhs)) : 1;
         d.qd = prec32 ? (const void *)op->qd32 : (const void *)op->qd64;
-        if (all_ef)
+        if (kind != STORED)
           d.ef = op->ef(prec32);
         if (k == K_PQ32)
         {

@@ -334,15 +334,18 @@ int hc_mg_level_op(hc_op_t op, int level, hc_op_t * level_op);
 int hc_mg_transfer(hc_op_t op, int level, int dir, const double * x, double * y, void * stream);
 
 /* Batches of solves over several operator instances (differing sizes and
- * orders), advanced together: every iteration applies all instances of one
- * order in one launch and updates all right-hand sides in one launch per
- * vector kernel; converged right-hand sides drop out through device flags.
+ * orders), advanced together: every iteration applies all box instances on
+ * element factors (hc_op_set_factor_mode) in one launch and the others of one
+ * order and kind (trilinear, stored factors) in one, and updates all right-hand
+ * sides in one launch per vector kernel; converged right-hand sides drop out
+ * through device flags.
  * Replaces a loop of ImplicitSolve calls
  * (src/problem_operators/time_domain_equation_system_problem_operator.cpp:30-51)
  * over independent problems; the reference has no batched counterpart.
- * The tile variant of each order is that of the batch's first instance of that
- * order (hc_op_set_tile / hc_op_autotune).  Each instance's results equal
- * those of the same solve run alone with the same tile variant.
+ * The tile variant of stored factors is, for each order, that of the batch's
+ * first instance of that order that reads them (hc_op_set_tile /
+ * hc_op_autotune).  Each instance's results equal those of the same solve run
+ * alone with the same tile variant.
  *
  * hc_batch_add: b, x are device arrays of nrhs*N doubles of op (x = initial
  * guess); returns the entry index (>= 0) or a negative status.
@@ -369,7 +372,7 @@ int hc_batch_destroy(hc_batch_t batch);
  * its requests are in flight).  A scheduler thread admits requests in arrival
  * order as soon as their work vectors fit in the device-memory budget and
  * fewer than max_active are running, advances all admitted requests together
- * (one launch per ND order per operator apply), and retires each as soon as it
+ * (operator applies launched as in a batch), and retires each as soon as it
  * converges; a request's result does not depend on what else is running.
  * With mode HC_SOLVE_FP64 | HC_SOLVE_MG each request is solved by the
  * multigrid PCG of hc_pcg_solve (the gradient-space PCG for an operator whose

@@ -365,3 +365,37 @@ def test_graph_rounds_match_eager(torch_cuda, hc, mode):
         assert sa["iterations"] == sb["iterations"] and torch.equal(ya, yb)
     finally:
         hcurl.set_graphs(False)
+
+
+@pytest.mark.parametrize("mode", ["fp64", "fp32_ir", "fp32_ir_aux"])
+def test_batch_of_both_mesh_kinds(torch_cuda, hc, mode):
+    """Box and trilinear meshes of the same orders, and one box operator on stored
+    factors, in one batch: each instance's products are those it has alone, so its
+    solution and iteration count are bitwise those of a batch of one."""
+    torch = torch_cuda
+    md = {"fp64": hc.SOLVE_FP64, "fp32_ir": hc.SOLVE_FP32_IR, "fp32_ir_aux": hc.SOLVE_FP32_IR | hc.SOLVE_AUX}[mode]
+    print(f"case batch of both mesh kinds {mode}", flush=True)
+    rng = np.random.default_rng(17)
+    specs = [((6, 5, 4), 2, "box", 1), ((5, 4, 6), 2, "hex", 2), ((4, 6, 5), 2, "stored", 1), ((7, 6, 5), 1, "box", 2),
+             ((6, 7, 4), 1, "hex", 1), ((4, 5, 3), 3, "box", 1), ((3, 4, 5), 3, "hex", 2)]
+    bt, ents = hc.Batch(), []
+    for i, (n, p, kind, nr) in enumerate(specs):
+        vert = None
+        if kind == "hex":
+            Z, Y, X = np.meshgrid(*[np.arange(n[a] + 1) / n[a] for a in (2, 1, 0)], indexing="ij")
+            vert = np.stack([X, Y, Z], -1).reshape(-1, 3) + 0.02 * rng.uniform(-1, 1, (X.size, 3))
+        E = n[0] * n[1] * n[2]
+        op = hc.Operator(n, p, rng.uniform(0.5, 2.0, E), 10.0 ** rng.uniform(0, 2, E), vert=vert).setup(1.0)
+        if kind == "stored":
+            op.set_factor_mode(0)
+        b = _rand_rhs(torch, op, [300 + 10 * i + r for r in range(nr)])
+        ents.append((op, b, torch.zeros_like(b)))
+        bt.add(*ents[-1], rtol=1e-9, maxit=20000)
+    rc, stats = bt.solve(md)
+    assert rc == 0 and all(s["converged"] for s in stats)
+    for i, (op, b, x) in enumerate(ents):
+        x1, b1 = torch.zeros_like(b), hc.Batch()
+        b1.add(op, b, x1, rtol=1e-9, maxit=20000)
+        rc1, st1 = b1.solve(md)
+        assert rc1 == 0 and st1[0]["iterations"] == stats[i]["iterations"], specs[i]
+        assert torch.equal(x1, x), f"{specs[i]} differs alone vs in the batch"

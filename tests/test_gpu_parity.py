@@ -335,9 +335,9 @@ def test_element_factors(torch_cuda, hc, oracle, p):
 
 
 def test_element_factors_mixed_batch(torch_cuda, hc, oracle):
-    """A batch holding a box and a trilinear instance of one order runs both
-    from their quadrature-point factors; each solution meets rtol on the
-    oracle's operator and agrees with the same instance solved alone."""
+    """A batch holding a box and a trilinear instance of one order: each solution
+    meets rtol on the oracle's operator and agrees with the same instance solved
+    alone."""
     torch = torch_cuda
     p, n = 2, (7, 6, 5)
     print("case element factors mixed batch", flush=True)
