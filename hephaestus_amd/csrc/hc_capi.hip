@@ -153,10 +153,11 @@ plan_of(hc_op_t op)
 
 // y = A x for nrhs right-hand sides (rhs r at r*N) in the precision of T;
 // with resid_b, y = resid_b - A x (the kernels form the difference as they
-// store).
+// store).  ef: what the product reads (none: the stored factors).
 template <typename T>
 int
-apply_t(hc_op_t op, const T * x, T * y, int nrhs, const int * done, hipStream_t st, const T * resid_b = nullptr)
+apply_t(hc_op_t op, const hc::ElemFactors & ef, const T * x, T * y, int nrhs, const int * done, hipStream_t st,
+        const T * resid_b = nullptr)
 {
   const bool f32 = sizeof(T) == 4;
   int rc = op->ensure_ws(nrhs, f32);
@@ -168,7 +169,7 @@ apply_t(hc_op_t op, const T * x, T * y, int nrhs, const int * done, hipStream_t 
   T * part = (T *)(f32 ? (void *)op->ws.part32 : (void *)op->ws.part64);
   const int ntiles = pl.g.nt[0] * pl.g.nt[1] * pl.g.nt[2];
   const int rb = nrhs == 1 ? 1 : (op->rhs_block > 0 ? std::min(op->rhs_block, nrhs) : hc::default_rhs_block(ntiles, nrhs));
-  HC_TRY_HIP(hc::apply_op<T>(pl.g, pl.segs, tb, qd, op->ef(f32), x, y, part, done, st, pl.cand, nrhs, hc::STATE_STRIDE_INT, rb,
+  HC_TRY_HIP(hc::apply_op<T>(pl.g, pl.segs, tb, qd, ef, x, y, part, done, st, pl.cand, nrhs, hc::STATE_STRIDE_INT, rb,
                              f32 ? op->desc_dev + 1 : op->desc_dev, resid_b));
   return HC_OK;
 }
@@ -483,7 +484,7 @@ try
     return fail(HC_EINVAL, "hc_op_apply: hc_op_setup has not been called");
   if (nrhs < 1)
     return fail(HC_EINVAL, "hc_op_apply: nrhs must be >= 1");
-  return apply_t<double>(op, x, y, nrhs, nullptr, (hipStream_t)stream);
+  return apply_t<double>(op, op->ef(false), x, y, nrhs, nullptr, (hipStream_t)stream);
 }
 catch (...)
 {
@@ -502,7 +503,7 @@ try
     return fail(HC_EINVAL, "hc_op_apply_f32: operator created without HC_PREC_FP32");
   if (nrhs < 1)
     return fail(HC_EINVAL, "hc_op_apply_f32: nrhs must be >= 1");
-  return apply_t<float>(op, x, y, nrhs, nullptr, (hipStream_t)stream);
+  return apply_t<float>(op, op->ef(true), x, y, nrhs, nullptr, (hipStream_t)stream);
 }
 catch (...)
 {
@@ -693,7 +694,7 @@ namespace hc
 int
 op_residual(hc_op_t op, const double * b, const double * x, double * r, hipStream_t st, int nrhs)
 {
-  return apply_t<double>(op, x, r, nrhs, nullptr, st, b);
+  return apply_t<double>(op, op->ef(false), x, r, nrhs, nullptr, st, b);
 }
 } // namespace hc
 
@@ -798,18 +799,10 @@ try
     if (prec == 32)
       HC_TRY_HIP(hc::cast_f32(op->ws.r64, op->ws.r32, op->N, st));
     hc::ApplyPlan & pl = prec == 64 ? op->plan64 : op->plan32;
-    float best = 1e30f;
-    const hc::TileCandidate * bestc = pl.cand;
-    // element factors: the box apply runs whatever the tile variant, which is
-    // kept; its time alone is measured
-    const bool box = op->ef(prec == 32).qc != nullptr;
-    for (int i = 0; i < (box ? 1 : n); i++)
-    {
-      if (!box)
-        set_plan(op, pl, &c[i]);
+    auto time = [&](const hc::ElemFactors & ef, float & ms) -> int {
       auto run = [&]() -> int {
-        return prec == 64 ? apply_t<double>(op, op->ws.r64, op->ws.q64, 1, nullptr, st)
-                          : apply_t<float>(op, op->ws.r32, op->ws.q32, 1, nullptr, st);
+        return prec == 64 ? apply_t<double>(op, ef, op->ws.r64, op->ws.q64, 1, nullptr, st)
+                          : apply_t<float>(op, ef, op->ws.r32, op->ws.q32, 1, nullptr, st);
       };
       for (int w = 0; w < 2; w++)
         if ((rc = run()))
@@ -820,16 +813,29 @@ try
           return rc;
       HC_TRY_HIP(hipEventRecord(e1, st));
       HC_TRY_HIP(hipEventSynchronize(e1));
-      float ms = 0;
       HC_TRY_HIP(hipEventElapsedTime(&ms, e0, e1));
+      return HC_OK;
+    };
+    // the variants differ in products from stored factors, whether the operator
+    // reads them now or after a later hc_op_set_factor_mode
+    float best = 1e30f;
+    const hc::TileCandidate * bestc = pl.cand;
+    for (int i = 0; i < n; i++)
+    {
+      float ms = 0;
+      set_plan(op, pl, &c[i]);
+      if ((rc = time(hc::ElemFactors{}, ms)))
+        return rc;
       if (ms < best)
       {
         best = ms;
-        if (!box)
-          bestc = &c[i];
+        bestc = &c[i];
       }
     }
     set_plan(op, pl, bestc);
+    if (const hc::ElemFactors ef = op->ef(prec == 32); ef.qc && best_us)
+      if ((rc = time(ef, best)))
+        return rc;
     if (best_us)
       best_us[prec == 64 ? 0 : 1] = 1000.0 * best / reps;
   }

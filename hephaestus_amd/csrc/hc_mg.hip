@@ -1012,8 +1012,7 @@ estimate_lambda(MgHier & h, MgLevel & L, hipStream_t st, double & lam)
 }
 
 // Hierarchy builds run one at a time in the process: a build is one-time
-// setup (level operators, their autotuning, rocSOLVER on the coarsest level,
-// power iterations), and the multigrid server and batch workers otherwise
+// setup (level operators, rocSOLVER on the coarsest level, power iterations), and the multigrid server and batch workers otherwise
 // start several of them together on their first requests.  Solves on built
 // hierarchies run concurrently.
 std::mutex g_build_mu;
@@ -1115,8 +1114,8 @@ mg_build(hc_op_t op, hipStream_t st)
     h->lev.push_back(c);
     if ((rc = hc_op_setup(h->lev.back().op, op->last_dt, st)))
       return rc;
-    // the level's own fastest tile variant (its mesh differs from the finest)
-    if ((rc = hc_op_autotune(h->lev.back().op, 3, nullptr, st)))
+    // the level's own fastest tile variant, where it reads stored factors
+    if (!h->lev.back().op->ef(false).qc && (rc = hc_op_autotune(h->lev.back().op, 3, nullptr, st)))
       return rc;
     h->lev.back().N = h->lev.back().op->N;
     nu.swap(nuc);
@@ -1201,9 +1200,8 @@ mg_build(hc_op_t op, hipStream_t st)
       return fail(HC_EHIP, "multigrid: rocblas_set_stream failed");
     // A coarsest level with a tiny sigma (a gradient-dominated null space
     // near h^3 sigma against a curl part near 1 / h) is SPD but can be so
-    // ill-conditioned that the rounding of its probed columns (which depends
-    // on the level's tile variant) leaves a Cholesky pivot negative; then
-    // the probe is repeated with the diagonal raised by a relative 1e-12,
+    // ill-conditioned that the rounding of its probed columns leaves a
+    // Cholesky pivot negative; then the probe is repeated with the diagonal raised by a relative 1e-12,
     // 1e-10, 1e-8 (the coarsest solve is part of a preconditioner).  The
     // first attempt is the plain matrix.
     constexpr double BOOST[4] = {0.0, 1e-12, 1e-10, 1e-8};

@@ -289,10 +289,10 @@ int hc_op_set_tile(hc_op_t op, int prec_bits, int tx, int ty, int tz, int mode);
 int hc_tile_list(int order, int * out, int max);
 int hc_op_get_tile(hc_op_t op, int prec_bits, int * tx, int * ty, int * tz, int * mode);
 /* Autotuner: times every compiled tile variant on this operator (after
- * hc_op_setup), `reps` applies each, and keeps the fastest per precision.
- * Where the apply takes element factors (hc_op_set_factor_mode 1) there is
- * nothing to choose: it is timed and the variant kept.
- * best_us (optional, 2 entries): the winning FP64 / FP32 apply times.
+ * hc_op_setup), `reps` applies from stored factors each (whatever
+ * hc_op_set_factor_mode says), and keeps the fastest per precision.
+ * best_us (optional, 2 entries): the FP64 / FP32 apply times that result (of
+ * the apply from element factors where the operator reads those).
  * No reference counterpart (the reference applies a CSR matrix). */
 int hc_op_autotune(hc_op_t op, int reps, double * best_us, void * stream);
 /* Jacobi diagonal (1 on PEC DOFs) into device array d. */

@@ -164,7 +164,7 @@ def test_three_levels_galerkin_and_level_ops(env):
             direct.fill_uniform(3 + lvl, x)
             lo = op.mg_level(lvl)
             assert lo.ndofs == direct.ndofs
-            direct.set_tile(64, *lo.get_tile(64))  # (levels run their own autotuned tile variant)
+            direct.set_tile(64, *lo.get_tile(64))  # (a level that reads stored factors runs its own variant)
             assert torch.equal(lo.apply(x), direct.apply(x)), (dt, lvl)
             direct.close()
     op.close()
