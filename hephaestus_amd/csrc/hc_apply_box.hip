@@ -1059,7 +1059,7 @@ apply_box(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, i
       run(k_apply_box<0, T, NS, true, BOX_APPLY, false>);
     else
     {
-      if constexpr (NS <= 32)
+      if constexpr (NS <= 32 && (sizeof(T) == 8 || P == 1))
       {
         if (hex)
           return descs ? run(k_apply_box<P, T, NS, true, BOX_APPLY, true>) : run(k_apply_box<P, T, NS, false, BOX_APPLY, true>);
@@ -1072,9 +1072,9 @@ apply_box(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, i
           return run(k_apply_box<P, T, NS, false, BOX_ADD, false>);
         if (kind == BOX_MASS)
           return run(k_apply_box<P, T, NS, false, BOX_MASS, false>);
+        if (kind == BOX_RESID)
+          return run(k_apply_box<P, T, NS, false, BOX_RESID, false>);
       }
-      if (kind == BOX_RESID)
-        return run(k_apply_box<P, T, NS, false, BOX_RESID, false>);
       run(k_apply_box<P, T, NS, false, BOX_APPLY, false>);
     }
   };
@@ -1086,11 +1086,11 @@ apply_box(const ApplyDesc & d0, const ApplyDesc * descs, int ndesc, int nwork, i
     else
       go(pc, std::integral_constant<int, 64>{});
   };
-  // residuals are formed for multigrid and tables of several orders for batches
-  // of box meshes only
+  // residuals are formed for multigrid (FP64) and tables of several orders for
+  // batches of box meshes only; FP32 vectors on trilinear meshes at order 1 only
   const bool with_y = kind == BOX_RESID || kind == BOX_ADD;
   if ((hex && (ns > 32 || kind != BOX_APPLY || p == 0)) || (p == 0 && !descs) || (descs && kind != BOX_APPLY) ||
-      (sizeof(T) != 8 && (kind == BOX_ADD || kind == BOX_MASS)) || (!descs && with_y != (d0.resid != nullptr)))
+      (sizeof(T) != 8 && (kind != BOX_APPLY || (hex && p != 1))) || (!descs && with_y != (d0.resid != nullptr)))
     return hipErrorInvalidValue;
   switch (p)
   {

@@ -271,7 +271,7 @@ hipError_t apply_op(const Geom & g,
 // common to the launch; p = 0: a table of instances of any orders), and its
 // decomposition of a mesh for nrhs vectors (ns_only: with that many slots).  The
 // results do not depend on it.  Forms of one instance (box meshes):
-//   BOX_RESID  y = b - A x with b = ApplyDesc::resid (on PEC DOFs b - x)
+//   BOX_RESID  y = b - A x with b = ApplyDesc::resid (on PEC DOFs b - x; FP64)
 //   BOX_ADD    y = y + A x with resid = y, PEC DOFs y = x (FP64)
 //   BOX_MASS   the mass term alone, cscale taken as 0 (FP64)
 enum BoxKind
