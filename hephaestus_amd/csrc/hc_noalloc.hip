@@ -1,8 +1,9 @@
 // hc_op_apply_noalloc: y = A x (FP64, one right-hand side) with no device
 // allocation, for callers that cannot allocate (code under HIP graph capture,
-// tight serving loops).  It runs the same kernels as hc_op_apply (the
-// operator's FP64 tile variant, then the tile-face assembly) and differs only
-// in where the tile-face partials live: a file-scope device array of fixed
+// tight serving loops).  It runs the same kernels as hc_op_apply: the box apply
+// where the operator reads element factors, which needs no memory of its own;
+// from stored factors the operator's FP64 tile variant, then the tile-face
+// assembly, with the tile-face partials in a file-scope device array of fixed
 // size instead of the handle's workspace, which hc_op_apply grows on demand.
 //
 // Every call on a GPU shares that GPU's array (the last call's partials stay
@@ -97,6 +98,8 @@ try
   if (!op->setup_done)
     return hc::fail(HC_EINVAL, "hc_op_apply_noalloc: hc_op_setup has not been called");
   const hc::ApplyPlan & pl = op->plan64;
+  // refused whichever factors are read: an operator that is accepted stays so
+  // after hc_op_set_factor_mode
   const int64_t S = plane_entries(pl.g, pl.segs);
   if (4 * S > SCRATCH_DOUBLES)
     return hc::fail(HC_EINVAL, "hc_op_apply_noalloc: the tile-face partials of this operator need " +

@@ -368,13 +368,14 @@ class Operator:
         return d
 
     def set_factor_mode(self, mode):
-        """1 (default): element factors on box meshes; 0: quadrature-point factors."""
+        """1 (default): products read two factors per element, on trilinear meshes with the
+        vertices (FP32 vectors there at order 1 only); 0: the stored quadrature-point factors."""
         _check(_lib.hc_op_set_factor_mode(self._h, int(mode)), "hc_op_set_factor_mode")
         return self
 
     @property
     def factor_mode(self):
-        """The factor storage the apply kernels read (1: element factors, 0: quadrature points)."""
+        """1 if products read element factors only (a box mesh in mode 1), else 0."""
         r = _lib.hc_op_factor_mode(self._h)
         if r < 0:
             _check(r, "hc_op_factor_mode")

@@ -202,19 +202,21 @@ int hc_op_factor_mode(hc_op_t op);
 int hc_engine_set_graphs(int enable);
 
 /* y = A x (PEC eliminated).  x, y: device, nrhs vectors (rhs r at r*N).
- * With nrhs > 1 a work item of the kernel applies the operator to a group of
- * right-hand sides, reading each tile's quadrature data once per group. */
+ * With nrhs > 1 from stored factors (hc_op_set_factor_mode) a work item of the
+ * kernel may apply the operator to a group of right-hand sides, reading each
+ * tile's quadrature data once per group (hc_op_set_rhs_block). */
 int hc_op_apply(hc_op_t op, const double * x, double * y, int nrhs, void * stream);
 int hc_op_apply_f32(hc_op_t op, const float * x, float * y, int nrhs, void * stream);
 /* y = A x (FP64, one right-hand side) without any device allocation.  No
  * counterpart in the reference: it is for callers that cannot allocate (code
  * under HIP graph capture, tight serving loops).  Same kernels and result bits
- * as hc_op_apply with nrhs = 1; the tile-face partials live in a static device
- * array of hc_noalloc_scratch_doubles() doubles per GPU (32 MiB), shared by
- * every call on that GPU: calls that overlap on one GPU race.  HC_EINVAL when
- * the operator's partials (4 slots of its tile-plane DOFs) exceed it.  The
- * scratch address is resolved at hc_op_create (or at the first call on a
- * device), so a call inside a capture only launches kernels. */
+ * as hc_op_apply with nrhs = 1; from stored factors the tile-face partials live
+ * in a static device array of hc_noalloc_scratch_doubles() doubles per GPU
+ * (32 MiB), shared by every such call on that GPU: calls that overlap on one GPU
+ * race (from element factors they do not use it).  HC_EINVAL when the partials of
+ * the operator's tile variant (4 slots of its tile-plane DOFs) exceed it, in
+ * either factor mode.  The scratch address is resolved at hc_op_create (or at
+ * the first call on a device), so a call inside a capture only launches kernels. */
 int hc_op_apply_noalloc(hc_op_t op, const double * x, double * y, void * stream);
 int64_t hc_noalloc_scratch_doubles(void);
 /* y = K x with K the curl-curl part alone, (nu curl u, curl w), same PEC

@@ -55,13 +55,14 @@ def _rand_rhs(torch, op, seeds):
     return B
 
 
+@pytest.mark.parametrize("factors", [0, 1])  # (groups of right-hand sides are those of stored factors)
 @pytest.mark.parametrize("p,n,rb", [(1, (9, 6, 5), 3), (2, (10, 7, 6), 2), (3, (6, 5, 7), 4), (2, (5, 5, 5), 0)])
-def test_multi_rhs_apply(torch_cuda, hc, O, p, n, rb):
+def test_multi_rhs_apply(torch_cuda, hc, O, p, n, rb, factors):
     torch = torch_cuda
-    print(f"case multi-rhs apply p={p} n={n} rb={rb}", flush=True)
+    print(f"case multi-rhs apply p={p} n={n} rb={rb} factors={factors}", flush=True)
     m = O.Mesh(*n)
     sig = _two_region(n, 3.0, 0.5)
-    op = hc.Operator(n, p, 1.0, sig).setup(1.0)
+    op = hc.Operator(n, p, 1.0, sig).setup(1.0).set_factor_mode(factors)
     op.set_rhs_block(rb)
     X = _rand_rhs(torch, op, [11, 12, 13, 14, 15])
     Y = op.apply(X)
@@ -83,11 +84,12 @@ def test_multi_rhs_apply(torch_cuda, hc, O, p, n, rb):
         assert _rel(Y32[r], Yh[r]) <= 2e-6
 
 
-@pytest.mark.parametrize("mode", ["fp64", "fp32_ir", "fp64_aux", "fp32_ir_aux", "fp64_mg"])
-def test_multi_rhs_solve(torch_cuda, hc, O, mode):
+@pytest.mark.parametrize("mode,factors", [("fp64", 1), ("fp32_ir", 1), ("fp64_aux", 1), ("fp32_ir_aux", 1), ("fp64_mg", 1),
+                                          ("fp64", 0), ("fp32_ir", 0)])
+def test_multi_rhs_solve(torch_cuda, hc, O, mode, factors):
     torch = torch_cuda
     n, p = (8, 7, 6), 2
-    print(f"case multi-rhs solve {mode} n={n} p={p}", flush=True)
+    print(f"case multi-rhs solve {mode} n={n} p={p} factors={factors}", flush=True)
     md = hc.SOLVE_FP64 if mode.startswith("fp64") else hc.SOLVE_FP32_IR
     if mode.endswith("_aux"):
         md |= hc.SOLVE_AUX
@@ -95,7 +97,7 @@ def test_multi_rhs_solve(torch_cuda, hc, O, mode):
         md |= hc.SOLVE_MG
     m = O.Mesh(*n)
     sig = _two_region(n, 100.0, 0.1)
-    op = hc.Operator(n, p, 1.0, sig).setup(1.0)
+    op = hc.Operator(n, p, 1.0, sig).setup(1.0).set_factor_mode(factors)
     op.set_rhs_block(2)
     B = _rand_rhs(torch, op, [21, 22, 23])
     B = torch.cat([B, torch.zeros_like(B[:1])])  # a zero right-hand side converges at once

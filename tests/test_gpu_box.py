@@ -4,7 +4,8 @@ decomposition.
 Its workgroups march columns of 16, 32 or 64 element slots along z, duplicate
 the elements of tile and chunk faces and choose slots, tile and chunk from the
 mesh and the number of right-hand sides.  Against the quadrature-point factors
-of the same operator (the tile kernels that the oracle tests pin): meshes of one
+of the same operator (the tile kernels, which the tests of tile variants pin to
+the oracle in factor mode 0): meshes of one
 element per direction, edges just below, at and above tile and chunk sizes, the
 block pairs of order 1 split by an odd edge, partial PEC, and sizes that take
 each number of slots.  Both sides carry rounding errors of a few units of

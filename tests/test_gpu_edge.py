@@ -44,9 +44,11 @@ def test_tiny_meshes_every_tile(env, p, n, pec):
     y_ref = O.pa_apply(m, p, qd, ess, x)
     op = H.Operator(n, p, nu, sig, pec_faces=pec).setup(1.0)
     xd = torch.from_numpy(x).cuda()
-    for t in hcurl.tile_list(p):
-        op.set_tile(64, *t)
-        op.set_tile(32, *t)
+    for t in [None, *hcurl.tile_list(p)]:
+        op.set_factor_mode(1 if t is None else 0)  # the tiles are those of stored factors
+        if t is not None:
+            op.set_tile(64, *t)
+            op.set_tile(32, *t)
         assert _rel(op.apply(xd).cpu().numpy(), y_ref) <= 1e-13, t
         assert _rel(op.apply_f32(xd.float()).double().cpu().numpy(), y_ref) <= 2e-6, t
 

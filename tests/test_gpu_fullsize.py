@@ -138,6 +138,8 @@ def test_every_tile_variant_full_size(env):
     y_ref = op.apply(x)
     nref = float(torch.linalg.norm(y_ref))
     x32 = x.float()
+    assert float(torch.linalg.norm(op.apply_f32(x32).double() - y_ref)) <= 1e-5 * nref
+    op.set_factor_mode(0)  # the tiles are those of stored factors, y_ref is from element factors
     for t in H.tile_list(p):
         print(f"  tile {t}", flush=True)
         op.set_tile(64, *t)

@@ -131,8 +131,9 @@ def test_apply_vs_oracle(torch_cuda, hc, oracle, p, n, pec, perturb):
 
 @pytest.mark.parametrize("p", [1, 2, 3])
 def test_every_tile_variant(torch_cuda, hc, oracle, p):
-    """Each compiled tile shape of the apply kernel gives the oracle's result
-    (several tiles per direction, partial tiles, trilinear geometry)."""
+    """Each compiled tile shape of the stored-factor kernels gives the oracle's
+    result (several tiles per direction, partial tiles, trilinear geometry), and
+    so does the product from element factors."""
     torch = torch_cuda
     from hephaestus_amd import hcurl
     n = {1: (11, 9, 6), 2: (9, 7, 5), 3: (9, 5, 7)}[p]
@@ -149,8 +150,11 @@ def test_every_tile_variant(torch_cuda, hc, oracle, p):
     y_ref = oracle.pa_apply(m, p, qd, ess, x)
     op = hc.Operator(n, p, nu, sig, vert=vert).setup(1.0)
     xd = _dev(torch, x)
+    assert _rel(op.apply(xd).cpu().numpy(), y_ref) <= 1e-13
+    assert _rel(op.apply_f32(xd.float()).double().cpu().numpy(), y_ref) <= 2e-6
     tiles = hcurl.tile_list(p)
     assert len(tiles) >= 2
+    op.set_factor_mode(0)
     for (tx, ty, tz, pf) in tiles:
         op.set_tile(64, tx, ty, tz, pf)
         op.set_tile(32, tx, ty, tz, pf)
@@ -162,10 +166,11 @@ def test_every_tile_variant(torch_cuda, hc, oracle, p):
 
 @pytest.mark.parametrize("p", [1, 2, 3])
 def test_many_tiles_multi_rhs(torch_cuda, hc, oracle, p):
-    """Every tile variant on a mesh of several hundred tiles (more workgroups
-    than the XCD renumbering's 8 groups times the CUs), three right-hand sides
-    in one launch over (tile, rhs) work items: oracle parity, and the single
-    rhs apply equals its row of the multi-rhs apply bitwise."""
+    """Every tile variant of the stored-factor kernels on a mesh of several
+    hundred tiles (more workgroups than the XCD renumbering's 8 groups times the
+    CUs), three right-hand sides in one launch over (tile, rhs) work items: oracle
+    parity, and the single rhs apply equals its row of the multi-rhs apply
+    bitwise.  The same from element factors."""
     torch = torch_cuda
     from hephaestus_amd import hcurl
     n = {1: (40, 36, 30), 2: (30, 26, 22), 3: (24, 22, 20)}[p]
@@ -182,19 +187,22 @@ def test_many_tiles_multi_rhs(torch_cuda, hc, oracle, p):
     op = hc.Operator(n, p, nu, sig).setup(1.0)
     op.set_rhs_block(1)
     xd = _dev(torch, X)
-    for (tx, ty, tz, pf) in hcurl.tile_list(p):
-        op.set_tile(64, tx, ty, tz, pf)
+    for t in [None, *hcurl.tile_list(p)]:
+        op.set_factor_mode(1 if t is None else 0)
+        if t is not None:
+            op.set_tile(64, *t)
         y = op.apply(xd)
         for r in range(3):
-            assert _rel(y[r].cpu().numpy(), Y[r]) <= 1e-13, (tx, ty, tz, pf, r)
-        assert torch.equal(op.apply(xd[1]), y[1]), (tx, ty, tz, pf)
+            assert _rel(y[r].cpu().numpy(), Y[r]) <= 1e-13, (t, r)
+        assert torch.equal(op.apply(xd[1]), y[1]), t
 
 
 @pytest.mark.parametrize("p", [1, 2, 3])
 def test_tile_variants_repeatable(torch_cuda, hc, p):
-    """Every tile variant gives bitwise identical results over repeated applies
-    on a mesh of several hundred tiles (a race between the waves of a
-    workgroup shows up as an occasional difference)."""
+    """Every tile variant of the stored-factor kernels, and the product from
+    element factors, gives bitwise identical results over repeated applies on a
+    mesh of several hundred tiles (a race between the waves of a workgroup shows
+    up as an occasional difference)."""
     torch = torch_cuda
     from hephaestus_amd import hcurl
     n = {1: (40, 36, 30), 2: (30, 26, 22), 3: (24, 22, 20)}[p]
@@ -205,9 +213,11 @@ def test_tile_variants_repeatable(torch_cuda, hc, p):
     x = torch.empty(op.ndofs, dtype=torch.float64, device="cuda")
     op.fill_uniform(41, x)
     x32 = x.float()
-    for t in hcurl.tile_list(p):
-        op.set_tile(64, *t)
-        op.set_tile(32, *t)
+    for t in [None, *hcurl.tile_list(p)]:
+        op.set_factor_mode(1 if t is None else 0)
+        if t is not None:
+            op.set_tile(64, *t)
+            op.set_tile(32, *t)
         y0, z0 = op.apply(x), op.apply_f32(x32)
         for _ in range(8):
             assert torch.equal(op.apply(x), y0), t
@@ -286,11 +296,11 @@ def test_errors_are_reported(torch_cuda, hc):
 @pytest.mark.parametrize("p", [1, 2, 3])
 def test_element_factors(torch_cuda, hc, oracle, p):
     """Box meshes apply from two factors per element (dt nu_e, sigma_e) and the
-    axis constants: every tile variant against the oracle (FP64 1e-13, FP32
-    2e-6) and against the quadrature-point factors of the same operator
-    (1e-14), partial PEC, several right-hand sides in one launch bitwise equal
-    to single applies, the curl-only term weights; trilinear meshes keep the
-    quadrature-point factors."""
+    axis constants: against the oracle (FP64 1e-13, FP32 2e-6) and against every
+    tile variant of the quadrature-point factors of the same operator (1e-14),
+    partial PEC, several right-hand sides in one launch bitwise equal to single
+    applies, the curl-only term weights; trilinear meshes report that they read
+    more than element factors."""
     torch = torch_cuda
     from hephaestus_amd import hcurl
     n = {1: (11, 9, 6), 2: (9, 7, 5), 3: (9, 5, 7)}[p]

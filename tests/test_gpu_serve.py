@@ -170,7 +170,8 @@ def test_server_step_vs_oracle(torch_cuda, hc, tiles):
     srv = hc.Server(1 << 28, mode=hc.SOLVE_FP64 | hc.SOLVE_MG if tiles == "multigrid" else hc.SOLVE_FP32_IR,
                     rtol=1e-10, maxit=20000)
     if tiles == "server_tile":
-        # the operator keeps its autotuned variant; the server runs another one
+        # the operator keeps its autotuned variant; the server runs another one (of stored factors)
+        op.set_factor_mode(0)
         op.autotune(reps=2)
         own = op.get_tile(64)
         other = [t for t in hcurl.tile_list(p) if t != own and t[3] < 8][-1]

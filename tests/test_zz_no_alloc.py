@@ -1,8 +1,9 @@
 """hc_op_apply_noalloc (needs an MI355X): the entry point that allocates no
 device memory gives the bits of hc_op_apply on two calls in a row (the second
 on a smaller operator, so the shared static scratch holds the first call's
-partials), for every compiled tile variant of the first operator's order, and
-refuses an operator whose tile-face partials exceed the scratch."""
+partials), from element factors and, from stored ones, for every compiled tile
+variant of the first operator's order, and refuses an operator whose tile-face
+partials exceed the scratch, in either factor mode."""
 import ctypes
 
 import numpy as np
@@ -46,13 +47,14 @@ def test_noalloc_apply_matches_apply(env):
         op.fill_uniform(seed, x)
         print(f"case noalloc n={op.n} p={op.order}", flush=True)
         tiles = H.hcurl.tile_list(op.order)
-        for t in tiles if op is big else [None]:
+        for factors, t in [(1, None), *((0, t) for t in (tiles if op is big else [None]))]:
+            op.set_factor_mode(factors)
             if t is not None:
                 op.set_tile(64, *t)
             y_ref = op.apply(x)
             y = _noalloc(H, torch, op, x)
             torch.cuda.synchronize()
-            assert torch.equal(y, y_ref), (op.n, op.order, t)
+            assert torch.equal(y, y_ref), (op.n, op.order, factors, t)
 
 
 def test_noalloc_refuses_too_large(env):
@@ -65,6 +67,8 @@ def test_noalloc_refuses_too_large(env):
     op.set_tile(64, 8, 2, 1, -1)
     x = torch.zeros(op.ndofs, dtype=torch.float64, device="cuda")
     y = torch.zeros_like(x)
-    rc = lib.hc_op_apply_noalloc(op._h, ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(y.data_ptr()), None)
-    assert rc == H.hcurl.HC_EINVAL
-    assert b"static scratch" in lib.hc_last_error()
+    for factors in (0, 1):
+        op.set_factor_mode(factors)
+        rc = lib.hc_op_apply_noalloc(op._h, ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(y.data_ptr()), None)
+        assert rc == H.hcurl.HC_EINVAL
+        assert b"static scratch" in lib.hc_last_error()
