@@ -49,12 +49,13 @@
 // curl factors (adj(J^T J) sigma w / |det J| and J^T J dt nu w / |det J|) and the
 // transposed stages follow.  Against 12 (p + 1)^3 stored factors per element
 // read by the tile kernel of hc_apply_qp.hip this reads 24 bytes a vertex and 16
-// an element.  About 700 vector instructions and 86 matrix products a layer at
-// order 3 keep 244 registers, so two waves per SIMD and tiles of at most 32
-// elements, of whose work 1.5 x 1.1 is duplicated: bound by the FP64 pipe and
-// its latencies.  Measured, stored factors -> here: 48^3 order 3 223 -> 157 us,
-// 48^3 order 2 118 -> 106 us, 33x26x19 order 2 30 -> 24 us, 64^3 order 1
-// 80 -> 39 us, 16^3 order 1 12 -> 7.7 us.  Error against extended precision over
+// an element.  About 680 FP64 vector instructions and 86 matrix products a layer
+// at order 3 (480 and 62 at order 2) keep 244 registers, so two waves per SIMD
+// and tiles of at most 32 elements, of whose work 1.5 x 1.1 is duplicated.  At
+// 33x26x19 order 2 a SIMD issues vector instructions and products for 12 of 24 us;
+// the rest is latency with two waves.  Measured, stored factors -> here: 48^3
+// order 3 223 -> 157 us, 48^3 order 2 118 -> 106 us, 33x26x19 order 2 30 -> 24 us,
+// 64^3 order 1 80 -> 38 us, 16^3 order 1 12 -> 7.4 us.  Error against extended precision over
 // 40 meshes of 6x5x4 to 44x34x20: 9.1e-16 -> 7.2e-16 in the mean (the stored
 // factors take the Jacobian from sums of coordinates, here from differences).
 //
@@ -64,11 +65,13 @@
 //
 // Measured on boxes at 48^3 order 3 (9.08 M DOFs): 194 us per FP64 apply with the
 // LDS-staged tile kernel and its face assembly, 69 us here (FP32 vectors: 114
-// and 60 us).  Memory traffic is 164 MB (147 MB algorithmic, 30 us at the copy
-// rate); the bound is the FP64 pipe -- one 4 x 4 x 4 product takes 7 ns per SIMD
-// and a vector FMA 2.3 ns, and they do not overlap -- at about 65 % use, the
-// rest being latency with the four waves per SIMD that 128 registers allow.
-// Of the work 1.31 x 1.1 is duplicated elements of tile and chunk faces.
+// and 60 us).  Memory traffic is 160 MB (147 MB algorithmic, 30 us at the copy
+// rate).  By the counters a layer takes 55 products (16 cycles each on a SIMD) and
+// 248 other vector instructions (4 cycles; 150 of them FP64), which do not
+// overlap: 14 + 16 us of the 65.  The rest is latency -- chains of dependent
+// products, 152 scalar instructions and one barrier a layer, four waves per SIMD
+// that 128 registers allow; the waves wait for 42 % of their cycles.  Of the work
+// 1.31 x 1.08 is duplicated elements of tile and chunk faces.
 #include "hc_basis.hpp"
 #include "hc_kernels.hpp"
 
@@ -971,11 +974,19 @@ k_apply_box(ApplyDesc d0, const ApplyDesc * __restrict__ descs, int ndesc)
 
 // Decomposition: for each number of slots the tile with the fewest tiles (ties:
 // the widest rows) and the chunk of layers with the least modelled time.  A
-// layer takes about 0.9 + 1.25 w us at order 3 with w waves per SIMD (measured:
-// 2.2 us alone, 5.9 us with four; the other orders scale alike), so a mesh that
-// leaves CUs idle takes small workgroups and short chunks (12^3 order 3: 7.8 us
-// with 16 slots, 14.6 us with 64), one that fills them the fewest duplicated
-// elements (48^3 order 3: 63 us with 64 slots, 78 us with 16).
+// layer takes about 0.9 + 1.25 w us at order 3 with w waves per SIMD, so a mesh
+// that leaves CUs idle takes small workgroups and short chunks (12^3 order 3:
+// 7.8 us with 16 slots, 14.6 us with 64), one that fills them the fewest
+// duplicated elements (48^3 order 3: 63 us with 64 slots, 78 us with 16).
+// Measured, us a layer with 1, 2, 3, 4 waves (16 slots, one chunk):
+//   box        order 1  0.91 1.26 1.53 1.96   2  1.35 1.96 2.56 3.17   3  2.11 3.04 4.29 5.53
+//   trilinear  order 1  1.74 2.77             2  2.60 4.06             3  4.17 6.22
+// Only the ratio of the two terms decides: 0.72 here, 0.85 to 1.2 measured for
+// boxes (1.6 at order 1), 0.7 to 1.0 for the trilinear form, so that one pair
+// serves all.  Against every pair of 16, 32, 64 slots and chunks of 2 to 48 layers
+// on six meshes (17x23x41 to 48^3, 64x12x12, 9x9x63) the choice is within 2.5 % of
+// the best, beyond that at 64x12x12 (order 2 boxes 4 %, order 3 5 %: chunks of 2)
+// and 48^3 order 2 trilinear (6 %: 32 slots).
 BoxTile
 box_tile(const Geom & g, int nrhs, int ns_only, bool hex)
 {

@@ -246,10 +246,11 @@ hipError_t rhs_coil(const Geom & g, const CoilParams & cp, const double * vert, 
 hipError_t diagonal(const Geom & g, const Tables<double> & tb, const double * qd, double * d, hipStream_t st);
 
 // y = A x (PEC eliminated) for nrhs right-hand sides (vector r at r*N).
-// part: 4*N*nrhs scratch for tile-face partials.  done: optional device flags
-// done[r*done_stride]; the kernels skip rhs r when its flag is set.  rb > 1:
-// the batched kernel with rb right-hand sides per work item; its descriptor
-// is staged in desc_dev (device, one ApplyDesc).
+// done: optional device flags done[r*done_stride]; the kernels skip rhs r when its
+// flag is set.  With ef the box apply; else, from stored factors: part is 4*N*nrhs
+// scratch for tile-face partials, and rb > 1 takes the batched kernel with rb
+// right-hand sides per work item, whose descriptor is staged in desc_dev (device,
+// one ApplyDesc).
 template <typename T>
 hipError_t apply_op(const Geom & g,
                     const PlaneSegs & segs,
@@ -299,9 +300,9 @@ set_box_tile(ApplyDesc & d, int nrhs)
 }
 // Right-hand sides per work item for a batch of nrhs on ntiles tiles.
 int default_rhs_block(int ntiles, int nrhs);
-// y = (mscale M + cscale K') x (K' = the curl part of the quadrature data,
-// i.e. dt K) with the batched kernel; its descriptor is staged in desc_dev.
-// part: 4 N scratch.  add (FP64 on box meshes with element factors): the product
+// y = (mscale M + cscale K') x (K' = the curl part of the factors, i.e. dt K).
+// From stored factors with the batched kernel: its descriptor is staged in
+// desc_dev, part is 4 N scratch.  add (FP64 on box meshes with element factors): the product
 // is added to y on the free DOFs, PEC DOFs take x.
 template <typename T>
 hipError_t apply_scaled(const Geom & g, const PlaneSegs & segs, const Tables<T> & tb, const T * qd,
